@@ -33,130 +33,225 @@ __device__ __forceinline__ void ab_of(const Dims& d, const LinParams& lp, int kx
 }
 
 // -------------------------------------------------------------------------------------
-// Build the collocation matrix of one slot and invert it (initAuxMatrix,
-// source/solver.cpp:260-320): _get_coefficient_v / _omega / _get_coef_u0
-// (source/coefficient.cu:7-86), then LU with partial pivoting (largest |a|^2, first on
-// ties) and column-by-column solves of A X = I -- the oracle's restatement of Eigen's
-// inverse (source/matrix_op.cpp:22-27).  One block per (slot, equation); the LU works on
-// a row-major copy in `work` (nz*nz per block), the inverse lands column-major in minv.
+// Inverses of the collocation matrices (initAuxMatrix, source/solver.cpp:260-320):
+// _get_coefficient_v / _omega / _get_coef_u0 (source/coefficient.cu:7-86), then LU with
+// partial pivoting (largest |a|^2, first on ties) and column-by-column solves of A X = I --
+// the oracle's restatement of Eigen's inverse (source/matrix_op.cpp:22-27).  Three kernels:
+// k_lu (one block per matrix), k_lu_solve (one wave per 64 columns of an inverse, written
+// row-major) and k_transpose_square (in place, to the column-major layout of minv).  Every
+// entry goes through the oracle's operations in the oracle's order (each update of a factor
+// entry in ascending k, each dot product in ascending j, no contraction), so the inverses
+// equal the oracle's bit for bit whatever the blocking.
+//
+// The factorisation is left-looking in panels of kLuPanel columns held in LDS: a panel takes
+// the updates of all earlier columns from the stored factor, staged through LDS in chunks of
+// kLuPanel columns, and is then factored in place.  So the factor is read n/16/2 times from
+// L2 instead of being read and written n/3 times, the pivot search is a wave reduction, and
+// the solves read it by scalar loads with their own column coalesced across lanes.  Bound by
+// FP64 vector issue and LDS reads in k_lu (8 separate multiplies and adds per complex update)
+// and by the one serial chain of n^2/2 subtractions per column, which the order fixes, in
+// k_lu_solve.  One block per matrix with the trailing matrix in global memory, a serial pivot
+// search and one thread per column took 186 ms for the 8450 matrices of 128x129x128 and 5.1 ms
+// for the 2178 of 64x65x64; this takes 49 ms (13 + 35 + 1.4) and 1.8 ms (0.62 + 1.1 + 0.06).
 // -------------------------------------------------------------------------------------
-__global__ void k_build_inverse(double2* __restrict__ minv, double2* __restrict__ work, int slot0, Dims d,
-                                LinParams lp, const double* __restrict__ T0, const double* __restrict__ T2,
-                                const double* __restrict__ T4, const double* __restrict__ U,
-                                const double* __restrict__ ddU, int* __restrict__ status) {
-    const int slot = slot0 + blockIdx.x, eq = blockIdx.y;
-    if (slot >= d.nslot) return;
-    const int n = d.nz, N = d.N, tid = threadIdx.x, nthr = blockDim.x;
-    const long nn = (long)n * n;
-    double2* A = work + ((long)blockIdx.y * gridDim.x + blockIdx.x) * nn;
-    double2* X = minv + ((long)eq * d.nslot + slot) * nn;
-    const int kyh = slot / d.hnx, kx = slot - kyh * d.hnx;
-    const double Re = lp.Re, dt = lp.dt;
-    __shared__ int piv[512];
-    __shared__ int s_pr;
-    __shared__ double s_best;
+constexpr int kLuPanel = 16;
+constexpr int kLuThreads = 256;
 
-    if (kx == 0 && kyh == 0) {
-        for (long e = tid; e < nn; e += nthr) {
-            const int i = (int)(e / n), j = (int)(e - (long)i * n);
-            if (i >= 2) A[e] = make_double2(-T2[(long)n * (i - 1) + j] * dt * 0.5 / Re + T0[(long)n * (i - 1) + j], 0.0);
-            else if (i == 0) A[e] = make_double2(1.0, 0.0);
-            else A[e] = make_double2((j % 2 == 0) ? 1.0 : -1.0, 0.0);
-        }
-    } else {
-        double alpha, beta;
-        ab_of(d, lp, kx, kyh, &alpha, &beta);
-        const double kmn = alpha * alpha + beta * beta;
-        for (long e = tid; e < nn; e += nthr) {
-            const int i = (int)(e / n), j = (int)(e - (long)i * n);
-            double2 a;
-            if (eq == 0) {
-                if (i >= 4) {
-                    const long i2 = (long)n * (i - 2) + j;
-                    a.x = -T4[i2] * dt * 0.5 / Re + (1 + kmn * dt / Re) * T2[i2] - kmn * (1 + kmn * dt * 0.5 / Re) * T0[i2];
-                    a.y = alpha * dt * U[i - 2] * 0.5 * T2[i2] -
-                          (kmn * alpha * dt * 0.5 * U[i - 2] + alpha * dt * 0.5 * ddU[i - 2]) * T0[i2];
-                } else if (i == 0) a = make_double2(1.0, 0.0);
-                else if (i == 1) a = make_double2((j % 2 == 0) ? 1.0 : -1.0, 0.0);
-                else if (i == 2) a = make_double2((double)(j * j), 0.0);
-                else a = make_double2(((j % 2 == 0) ? -1.0 : 1.0) * j * j, 0.0);
-            } else {
-                if (i >= 2) {
-                    const long i1 = (long)n * (i - 1) + j;
-                    a.x = -T2[i1] * dt * 0.5 / Re + (1 + kmn * dt * 0.5 / Re) * T0[i1];
-                    a.y = alpha * dt * 0.5 * U[i - 1] * T0[i1];
-                } else if (i == 0) a = make_double2(1.0, 0.0);
-                else a = make_double2((j % 2 == 0) ? 1.0 : -1.0, 0.0);
-            }
-            A[e] = a;
-        }
-    }
-    (void)N;
+// LDS bytes of k_lu: the panel and a chunk of earlier columns, [kLuPanel][n | 1] each
+__host__ __device__ constexpr size_t lu_lds(int n) { return 2 * sizeof(double2) * kLuPanel * (size_t)(n | 1); }
+
+// entry (i, j) of the collocation matrix of equation eq (mean: the (0,0) pencil's)
+__device__ __forceinline__ double2 collocation_entry(int i, int j, int n, int eq, bool mean, double alpha, double kmn,
+                                                     double Re, double dt, const double* __restrict__ T0,
+                                                     const double* __restrict__ T2, const double* __restrict__ T4,
+                                                     const double* __restrict__ U, const double* __restrict__ ddU) {
+    if (i == 0) return make_double2(1.0, 0.0);
+    if (i == 1) return make_double2((j % 2 == 0) ? 1.0 : -1.0, 0.0);
+    const long i1 = (long)n * (i - 1) + j;
+    if (mean) return make_double2(-T2[i1] * dt * 0.5 / Re + T0[i1], 0.0);
+    if (eq == 1)
+        return make_double2(-T2[i1] * dt * 0.5 / Re + (1 + kmn * dt * 0.5 / Re) * T0[i1],
+                            alpha * dt * 0.5 * U[i - 1] * T0[i1]);
+    if (i == 2) return make_double2((double)(j * j), 0.0);
+    if (i == 3) return make_double2(((j % 2 == 0) ? -1.0 : 1.0) * j * j, 0.0);
+    const long i2 = (long)n * (i - 2) + j;
+    return make_double2(-T4[i2] * dt * 0.5 / Re + (1 + kmn * dt / Re) * T2[i2] - kmn * (1 + kmn * dt * 0.5 / Re) * T0[i2],
+                        alpha * dt * U[i - 2] * 0.5 * T2[i2] -
+                            (kmn * alpha * dt * 0.5 * U[i - 2] + alpha * dt * 0.5 * ddU[i - 2]) * T0[i2]);
+}
+
+// LU factors of the matrices of slots slot0 + blockIdx.x, equation blockIdx.y: row-major, unit
+// lower triangle below the diagonal, rows in pivot order; perm[i] = the row at position i.
+__global__ __launch_bounds__(kLuThreads) void k_lu(double2* __restrict__ work, int* __restrict__ perms, int slot0, Dims d,
+                                                   LinParams lp, const double* __restrict__ T0,
+                                                   const double* __restrict__ T2, const double* __restrict__ T4,
+                                                   const double* __restrict__ U, const double* __restrict__ ddU,
+                                                   int* __restrict__ status) {
+    extern __shared__ __align__(16) double2 lu_smem[];
+    __shared__ int perm[256], s_at[kLuThreads / 64];
+    __shared__ double s_max[kLuThreads / 64];
+    const int slot = slot0 + blockIdx.x, eq = blockIdx.y;
+    const int n = d.nz, ld = n | 1, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+    const long mat = (long)blockIdx.y * gridDim.x + blockIdx.x;
+    double2* A = work + mat * n * n;
+    double2 *P = lu_smem, *Lc = lu_smem + (size_t)kLuPanel * ld;  // [column][row]
+    const int kyh = slot / d.hnx, kx = slot - kyh * d.hnx;
+    const bool mean = kx == 0 && kyh == 0;
+    double alpha, beta;
+    ab_of(d, lp, kx, kyh, &alpha, &beta);
+    const double kmn = alpha * alpha + beta * beta;
+    if (tid < n) perm[tid] = tid;
     __syncthreads();
-    int failed = 0;
-    for (int k = 0; k < n; k++) {
-        if (tid == 0) {
-            int pr = k;
-            double2 a = A[(long)n * k + k];
-            double best = a.x * a.x + a.y * a.y;
-            for (int r = k + 1; r < n; r++) {
-                double2 b = A[(long)n * r + k];
-                double v = b.x * b.x + b.y * b.y;
-                if (v > best) { best = v; pr = r; }
+    const int pc = tid >> 4, pr0 = tid & 15;  // the thread's panel column and first row in the updates
+    for (int J0 = 0; J0 < n; J0 += kLuPanel) {
+        const int wc = min(kLuPanel, n - J0);
+        for (int e = tid; e < kLuPanel * n; e += kLuThreads) {
+            const int i = e / kLuPanel, c = e % kLuPanel;
+            if (c < wc) P[c * ld + i] = collocation_entry(perm[i], J0 + c, n, eq, mean, alpha, kmn, lp.Re, lp.dt, T0, T2, T4, U, ddU);
+        }
+        // the updates of the earlier columns, in chunks: a wave owns four panel columns, so the
+        // steps of a chunk need no barrier
+        for (int J = 0; J < J0; J += kLuPanel) {
+            __syncthreads();
+            for (int e = tid; e < kLuPanel * (n - J); e += kLuThreads) {
+                const int i = J + e / kLuPanel, c = e % kLuPanel;
+                Lc[c * ld + i] = A[(long)i * n + J + c];
             }
-            s_pr = pr;
-            s_best = best;
-            piv[k] = pr;
+            __syncthreads();
+            for (int kk = 0; kk < kLuPanel; kk++) {
+                const int k = J + kk;
+                if (pc < wc) {
+                    const double2 u = P[pc * ld + k];
+                    for (int i = k + 1 + pr0; i < n; i += 16) P[pc * ld + i] = zsub(P[pc * ld + i], zmul(Lc[kk * ld + i], u));
+                }
+                __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+                __builtin_amdgcn_wave_barrier();
+            }
         }
         __syncthreads();
-        const int pr = s_pr;
-        if (s_best == 0.0) { failed = 1; break; }
-        if (pr != k)
-            for (int j = tid; j < n; j += nthr) {
-                double2 t = A[(long)n * k + j];
-                A[(long)n * k + j] = A[(long)n * pr + j];
-                A[(long)n * pr + j] = t;
+        for (int jj = 0; jj < wc; jj++) {
+            const int k = J0 + jj;
+            // pivot: the largest |a|^2 of rows k.., the first on ties; a NaN wins at row k only
+            double best = -1.0;
+            int at = k;
+            for (int r = k + tid; r < n; r += kLuThreads) {
+                const double2 a = P[jj * ld + r];
+                const double v = a.x * a.x + a.y * a.y;
+                if (v > best || (r == k && !(v == v))) best = v == v ? v : __longlong_as_double(0x7ff0000000000000LL), at = r;
             }
-        __syncthreads();
-        const double2 dk = A[(long)n * k + k];
-        const double dd = dk.x * dk.x + dk.y * dk.y;
-        const double2 dinv = make_double2(dk.x / dd, -dk.y / dd);
-        for (int r = k + 1 + tid; r < n; r += nthr) A[(long)n * r + k] = zmul(A[(long)n * r + k], dinv);
-        __syncthreads();
-        const int m = n - k - 1;
-        for (long e = tid; e < (long)m * m; e += nthr) {
-            const int r = k + 1 + (int)(e / m), j = k + 1 + (int)(e - (e / m) * m);
-            A[(long)n * r + j] = zsub(A[(long)n * r + j], zmul(A[(long)n * r + k], A[(long)n * k + j]));
-        }
-        __syncthreads();
-    }
-    if (failed) {
-        if (tid == 0) atomicAdd(status, 1);
-        return;
-    }
-    // X = A^{-1}: thread c solves column c; column c of X is contiguous (column-major).
-    for (int c = tid; c < n; c += nthr) {
-        double2* col = X + (long)c * n;
-        for (int i = 0; i < n; i++) col[i] = make_double2(i == c ? 1.0 : 0.0, 0.0);
-        for (int k = 0; k < n; k++)
-            if (piv[k] != k) {
-                double2 t = col[k];
-                col[k] = col[piv[k]];
-                col[piv[k]] = t;
+            for (int m = 1; m < 64; m <<= 1) {
+                const double ov = __shfl_xor(best, m);
+                const int oa = __shfl_xor(at, m);
+                if (ov > best || (ov == best && oa < at)) best = ov, at = oa;
             }
-        for (int i = 0; i < n; i++) {
-            double2 s = col[i];
-            for (int j = 0; j < i; j++) s = zsub(s, zmul(A[(long)n * i + j], col[j]));
-            col[i] = s;
-        }
-        for (int i = n - 1; i >= 0; i--) {
-            double2 s = col[i];
-            for (int j = i + 1; j < n; j++) s = zsub(s, zmul(A[(long)n * i + j], col[j]));
-            const double2 dk = A[(long)n * i + i];
+            if (lane == 0) s_max[wave] = best, s_at[wave] = at;
+            __syncthreads();
+            best = s_max[0], at = s_at[0];
+            for (int w = 1; w < kLuThreads / 64; w++)
+                if (s_max[w] > best || (s_max[w] == best && s_at[w] < at)) best = s_max[w], at = s_at[w];
+            if (best == 0.0) {  // the same for every thread of the block
+                if (tid == 0) atomicAdd(status, 1);
+                return;
+            }
+            if (at != k) {
+                if (tid < wc) {
+                    const double2 t = P[tid * ld + k];
+                    P[tid * ld + k] = P[tid * ld + at];
+                    P[tid * ld + at] = t;
+                }
+                for (int j = tid; j < J0; j += kLuThreads) {
+                    const double2 t = A[(long)k * n + j];
+                    A[(long)k * n + j] = A[(long)at * n + j];
+                    A[(long)at * n + j] = t;
+                }
+                if (tid == 0) {
+                    const int t = perm[k];
+                    perm[k] = perm[at];
+                    perm[at] = t;
+                }
+            }
+            __syncthreads();
+            const double2 dk = P[jj * ld + k];
             const double dd = dk.x * dk.x + dk.y * dk.y;
-            col[i] = make_double2((s.x * dk.x + s.y * dk.y) / dd, (s.y * dk.x - s.x * dk.y) / dd);
+            const double2 dinv = make_double2(dk.x / dd, -dk.y / dd);
+            for (int r = k + 1 + tid; r < n; r += kLuThreads) P[jj * ld + r] = zmul(P[jj * ld + r], dinv);
+            __syncthreads();
+            if (pc > jj && pc < wc) {
+                const double2 u = P[pc * ld + k];
+                for (int i = k + 1 + pr0; i < n; i += 16) P[pc * ld + i] = zsub(P[pc * ld + i], zmul(P[jj * ld + i], u));
+            }
+            __syncthreads();
         }
+        for (int e = tid; e < kLuPanel * n; e += kLuThreads) {
+            const int i = e / kLuPanel, c = e % kLuPanel;
+            if (c < wc) A[(long)i * n + J0 + c] = P[c * ld + i];
+        }
+        __syncthreads();
     }
+    if (tid < n) perms[mat * n + tid] = perm[tid];
+}
+
+// Columns 64 blockIdx.z + lane of the inverses from the factors of k_lu, one wave each:
+// X[j*n + c] (row-major) in the matrix's place in minv.  Forward by four rows at a time (each
+// row's sum still in ascending j), back row by row.
+__global__ __launch_bounds__(64) void k_lu_solve(double2* __restrict__ minv, const double2* __restrict__ work,
+                                                 const int* __restrict__ perms, int slot0, Dims d) {
+    const int n = d.nz, c = blockIdx.z * 64 + threadIdx.x;
+    const long nn = (long)n * n, mat = (long)blockIdx.y * gridDim.x + blockIdx.x;
+    const double2* A = work + mat * nn;
+    const int* perm = perms + mat * n;
+    if (c >= n) return;
+    double2* X = minv + ((long)blockIdx.y * d.nslot + slot0 + blockIdx.x) * nn + c;
+    for (int i0 = 0; i0 < n; i0 += 4) {
+        double2 s[4];
+        const double2* a[4];
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+            const int i = min(i0 + q, n - 1);
+            s[q] = make_double2(perm[i] == c ? 1.0 : 0.0, 0.0);
+            a[q] = A + (long)i * n;
+        }
+#pragma unroll 4
+        for (int j = 0; j < i0; j++) {
+            const double2 y = X[(long)j * n];
+#pragma unroll
+            for (int q = 0; q < 4; q++) s[q] = zsub(s[q], zmul(a[q][j], y));
+        }
+#pragma unroll
+        for (int q = 0; q < 4; q++)
+            if (i0 + q < n) {
+                X[(long)(i0 + q) * n] = s[q];
+#pragma unroll
+                for (int t = q + 1; t < 4; t++) s[t] = zsub(s[t], zmul(a[t][i0 + q], s[q]));
+            }
+    }
+    double2 last = make_double2(0.0, 0.0);
+    for (int i = n - 1; i >= 0; i--) {
+        const double2* a = A + (long)i * n;
+        double2 s = X[(long)i * n];
+        if (i + 1 < n) s = zsub(s, zmul(a[i + 1], last));
+#pragma unroll 8
+        for (int j = i + 2; j < n; j++) s = zsub(s, zmul(a[j], X[(long)j * n]));
+        const double2 dk = a[i];
+        const double dd = dk.x * dk.x + dk.y * dk.y;
+        last = make_double2((s.x * dk.x + s.y * dk.y) / dd, (s.y * dk.x - s.x * dk.y) / dd);
+        X[(long)i * n] = last;
+    }
+}
+
+// In-place transposes of the matrices blockIdx.x (n x n each): tile pairs (bi, bj), bj <= bi.
+__global__ __launch_bounds__(256) void k_transpose_square(double2* __restrict__ m, int n) {
+    constexpr int T = 16;
+    __shared__ double2 a[T][T + 1], b[T][T + 1];
+    m += (long)blockIdx.x * n * n;
+    int bi = 0, bj = blockIdx.y;
+    while (bj > bi) bj -= ++bi;
+    const int x = threadIdx.x % T, y = threadIdx.x / T, i = bi * T + y, j = bj * T + x, i2 = bj * T + y, j2 = bi * T + x;
+    if (i < n && j < n) a[y][x] = m[(long)i * n + j];
+    if (i2 < n && j2 < n) b[y][x] = m[(long)i2 * n + j2];
+    __syncthreads();
+    if (i < n && j < n) m[(long)i * n + j] = b[x][y];
+    if (i2 < n && j2 < n) m[(long)i2 * n + j2] = a[x][y];
 }
 
 // Chebyshev derivative of one complex coefficient: ddz (source/RPCFKernels.cu:476-520)

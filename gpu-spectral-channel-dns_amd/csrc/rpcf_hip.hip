@@ -1296,14 +1296,23 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     double2* work = nullptr;
     int* status = nullptr;
     if ((rc = dalloc(c, &work, 2 * (size_t)chunk * per))) return rc;
-    if ((rc = dalloc(c, &status, 1))) { (void)hipFree(work); return rc; }
+    // [0] the count of singular matrices, then the row orders of a chunk's factors
+    if ((rc = dalloc(c, &status, 1 + 2 * (size_t)chunk * nz))) { (void)hipFree(work); return rc; }
     if ((rc = zero_sync(c, status, sizeof(int)))) { (void)hipFree(work); (void)hipFree(status); return rc; }
+    allow_lds(k_lu, (int)lu_lds(d.nz));
     for (int s0 = 0; s0 < d.nslot && !rc; s0 += chunk) {
-        dim3 g(std::min(chunk, d.nslot - s0), 2);
-        k_build_inverse<<<g, 256, 0, c->stream>>>(minv, work, s0, d, lp, c->T0, c->T2, c->T4, c->U + slot * c->sU,
-                                                  c->DDU + slot * c->sU, status);
+        dim3 g(std::min(chunk, d.nslot - s0), 2, 1);
+        k_lu<<<g, kLuThreads, lu_lds(d.nz), c->stream>>>(work, status + 1, s0, d, lp, c->T0, c->T2, c->T4,
+                                                         c->U + slot * c->sU, c->DDU + slot * c->sU, status);
+        k_lu_solve<<<dim3(g.x, 2, (d.nz + 63) / 64), 64, 0, c->stream>>>(minv, work, status + 1, s0, d);
         hipError_t e = hipGetLastError();
-        if (e != hipSuccess) rc = fail(c, RPCF_EDEVICE, "k_build_inverse: %s", hipGetErrorString(e));
+        if (e != hipSuccess) rc = fail(c, RPCF_EDEVICE, "k_lu: %s", hipGetErrorString(e));
+    }
+    if (!rc) {
+        const int nt = (d.nz + 15) / 16;
+        k_transpose_square<<<dim3(2 * d.nslot, nt * (nt + 1) / 2), 256, 0, c->stream>>>(minv, d.nz);
+        hipError_t e = hipGetLastError();
+        if (e != hipSuccess) rc = fail(c, RPCF_EDEVICE, "k_transpose_square: %s", hipGetErrorString(e));
     }
     int hstatus = 0;
     if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, RPCF_EDEVICE, "matrix build failed");
