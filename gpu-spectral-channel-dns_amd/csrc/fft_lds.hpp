@@ -197,19 +197,42 @@ template <int R1, int R2, int DIR, typename C> struct DftComposite {
 template <int DIR, typename C> struct Dft<16, DIR, C> : DftComposite<4, 4, DIR, C> {};
 template <int DIR, typename C> struct Dft<12, DIR, C> : DftComposite<4, 3, DIR, C> {};
 
+// i / d for a run-time divisor by its reciprocal: exact for i < 2^22 (the quotient's error,
+// i/d 2^-23, stays below the 0.5/d that i + 0.5 keeps from the next integer).  The integer
+// division it replaces in the runtime plans and ragged tiles is some 30 instructions an index;
+// with it, and the runtime plans' twiddles read from LDS, k_lamb_phys, k_span_inv and k_span_fwd
+// take 33, 24 and 16 us at 40x46x60 (50, 33 and 19 before) and 242, 178 and 82 at 100x151x100
+// (390, 222 and 104).
+struct FastDiv {
+    unsigned d;
+    float inv;
+    __device__ __forceinline__ explicit FastDiv(unsigned div) : d(div), inv(1.0f / (float)div) {}
+};
+__device__ __forceinline__ unsigned operator/(unsigned i, FastDiv f) { return (unsigned)(((float)i + 0.5f) * f.inv); }
+// a divisor that is the constant C, or (C = 0) a run-time one
+template <int C> struct ConstDiv {
+    __device__ __forceinline__ explicit ConstDiv(unsigned) {}
+};
+template <> struct ConstDiv<0> : FastDiv { using FastDiv::FastDiv; };
+template <int C> __device__ __forceinline__ unsigned operator/(unsigned i, ConstDiv<C> f) {
+    if constexpr (C > 0) return i / (unsigned)C;
+    else return i / static_cast<FastDiv>(f);
+}
+
 template <int R, int DIR, typename C>
 __device__ __forceinline__ void fft_stage(C* buf, int ld, int B, int n, int Ns, const C* __restrict__ tw, int tid,
                                           int nthr) {
-    const int nR = n / R;
+    const unsigned nR = n / R, ns = Ns;
     const int tot = B * nR;
     const int tstep = n / (Ns * R);
+    const FastDiv dn(nR), ds(ns);
     constexpr int MAXPT = RPCF_REGC / R;
     C v[MAXPT][R];
 #pragma unroll
     for (int it = 0; it < MAXPT; it++) {
-        int t = tid + it * nthr;
+        const int t = tid + it * nthr;
         if (t < tot) {
-            int b = t / nR, j = t - b * nR, k = j % Ns;
+            const unsigned b = (unsigned)t / dn, j = t - b * nR, k = j - (j / ds) * ns;
             const C* base = buf + b * ld;
 #pragma unroll
             for (int r = 0; r < R; r++) {
@@ -227,13 +250,13 @@ __device__ __forceinline__ void fft_stage(C* buf, int ld, int B, int n, int Ns, 
     __syncthreads();
 #pragma unroll
     for (int it = 0; it < MAXPT; it++) {
-        int t = tid + it * nthr;
+        const int t = tid + it * nthr;
         if (t < tot) {
-            int b = t / nR, j = t - b * nR, k = j % Ns;
+            const unsigned b = (unsigned)t / dn, j = t - b * nR, q = j / ds, k = j - q * ns;
             C* base = buf + b * ld;
-            int d = (j / Ns) * Ns * R + k;
+            const unsigned dst = q * ns * R + k;
 #pragma unroll
-            for (int r = 0; r < R; r++) base[d + r * Ns] = v[it][r];
+            for (int r = 0; r < R; r++) base[dst + r * ns] = v[it][r];
         }
     }
     __syncthreads();
@@ -394,6 +417,16 @@ __device__ __forceinline__ void fft_ct(C* buf, int ld, int B, const C* tw, int t
         fft_stage_ct<R, DIR, N, NS, BT, C, S == 0 ? Q : 0, S == 1 ? Q : 0, TW1, T1OFF>(buf, ld, B, tw, tid, nthr);
         fft_ct<N, DIR, BT, TWO, C, T1OFF, S + 1, NS * R>(buf, ld, B, tw, tid, nthr);
     }
+}
+
+// Twiddles of a plan copied into LDS by the kernels that read them there: a compiled plan's own
+// selection, all n of a runtime plan.
+template <int FN> __device__ __forceinline__ int tw_lds_count(const FftPlan& pl) { return FN > 0 ? ct_tw_lds_len(FN) : pl.n; }
+template <int FN, typename C>
+__device__ __forceinline__ void copy_tw(C* twl, FftPlan& pl, int tid, int nthr) {
+    const C* twg = (const C*)pl.tw;
+    for (int i = tid; i < tw_lds_count<FN>(pl); i += nthr) twl[i] = twg[FN > 0 ? ct_tw_lds_src(FN, i) : i];
+    pl.tw = twl;
 }
 
 // FN > 0: the compile-time plan of length FN (must equal pl.n); FN = 0: the runtime plan.

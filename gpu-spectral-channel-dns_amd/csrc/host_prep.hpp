@@ -178,31 +178,31 @@ inline void s2p_tables(int N, std::vector<_Float16>& out) {
 // derivative (ddz_sm, source/RPCFKernels.cu:476-520), S the values at the nz collocation
 // points; folded by reflection parity into Q0s, Q0a, Q1s, Q1a (rows p <= N/2, p < N/2).
 struct P2sFolded {
-    std::vector<long double> q0s, q0a, q1s, q1a;  // [N/2+1][N+1], [N/2][N], [N/2+1][N], [N/2][N+1]
+    std::vector<long double> q0s, q0a, q1s, q1a;  // [N/2+1][N+1], [(N+1)/2][N], [N/2+1][N], [(N+1)/2][N+1]
 };
 inline P2sFolded p2s_folded(int N) {
     const int nz = N + 1, pz = 2 * N + 1;
     std::vector<long double> P((size_t)nz * pz), DP((size_t)nz * pz, 0.0L), M0((size_t)nz * pz), M1((size_t)nz * pz);
+    std::vector<long double> cosn(4 * (size_t)N);  // cos(pi n/(2N)), n < 4N
+    for (int n = 0; n < 4 * N; n++) cosn[n] = cospi_ratio(n, 2L * N);
     for (int k = 0; k < nz; k++)
         for (int q = 0; q < pz; q++) {
             const long double w = (q == 0 || q == 2 * N) ? 1.0L : 2.0L;
-            P[(size_t)k * pz + q] = w * cospi_ratio((long)k * q, 2L * N) / (2.0L * N) * (k == 0 ? 0.5L : 1.0L);
+            P[(size_t)k * pz + q] = w * cosn[(size_t)k * q % (4 * N)] / (2.0L * N) * (k == 0 ? 0.5L : 1.0L);
         }
     for (int k = 0; k < nz; k++)
         for (int j = k + 1; j < nz; j += 2)
             for (int q = 0; q < pz; q++) DP[(size_t)k * pz + q] += 2.0L * j * P[(size_t)j * pz + q] * (k == 0 ? 0.5L : 1.0L);
-    for (int p = 0; p < nz; p++)
-        for (int q = 0; q < pz; q++) {
-            long double a = 0, b = 0;
-            for (int k = 0; k < nz; k++) {
-                const long double c = cospi_ratio((long)k * p, (long)N);
-                a += c * P[(size_t)k * pz + q];
-                b += c * DP[(size_t)k * pz + q];
+    // rows p <= N/2 only: the others are their mirrors
+    const int rs = N / 2 + 1, ra = (N + 1) / 2;
+    for (int p = 0; p < rs; p++)
+        for (int k = 0; k < nz; k++) {
+            const long double c = cosn[(size_t)2 * k * p % (4 * N)];
+            for (int q = 0; q < pz; q++) {
+                M0[(size_t)p * pz + q] += c * P[(size_t)k * pz + q];
+                M1[(size_t)p * pz + q] += c * DP[(size_t)k * pz + q];
             }
-            M0[(size_t)p * pz + q] = a;
-            M1[(size_t)p * pz + q] = b;
         }
-    const int rs = N / 2 + 1, ra = N / 2;
     P2sFolded f;
     f.q0s.resize((size_t)rs * (N + 1));
     f.q0a.resize((size_t)ra * N);
@@ -264,6 +264,34 @@ inline void p2s_tables_f64(int N, std::vector<double>& out) {
     for (int q = 0; q < N; q++) out.push_back((double)f.q1s[(size_t)(N / 2) * N + q]);
     for (int p = 0; p < rs; p++) out.push_back((double)f.q0s[(size_t)p * (N + 1) + N]);
     for (int p = 0; p < ra; p++) out.push_back((double)f.q1a[(size_t)p * (N + 1) + N]);
+}
+
+// FP64 fragments of the Chebyshev products of lengths without a compiled plan
+// (k_p2s_dmfma_n, k_s2p_dmfma_n): the folded p2s tables Q0s, Q0a, Q1s, Q1a as rt row tiles x
+// kp k-steps each, zero past their sizes; then per s2p row tile the even and odd products,
+// E[q][j] = cos(pi 2j q/(2N)) and O[q][j] = cos(pi (2j+1) q/(2N)), q <= N
+inline void cheb_tables_n(int N, int rt, int kp, int rq, int ke, int ko, std::vector<double>& out) {
+    const P2sFolded f = p2s_folded(N);
+    const int rs = N / 2 + 1, ra = (N + 1) / 2;
+    auto padded = [&](const std::vector<long double>& T, int rows, int cols) {
+        std::vector<long double> t((size_t)16 * rt * 4 * kp, 0.0L);
+        for (int r = 0; r < rows; r++)
+            for (int c = 0; c < cols; c++) t[(size_t)r * 4 * kp + c] = T[(size_t)r * cols + c];
+        dmfma_fragments(t, 16 * rt, 4 * kp, out);
+    };
+    padded(f.q0s, rs, N + 1);
+    padded(f.q0a, ra, N);
+    padded(f.q1s, rs, N);
+    padded(f.q1a, ra, N + 1);
+    for (int t = 0; t < rq; t++)
+        for (int par = 0; par < 2; par++) {
+            const int ks = par ? ko : ke, cols = (N + 2 - par) / 2;
+            std::vector<long double> e((size_t)16 * 4 * ks, 0.0L);
+            for (int r = 0; r < 16 && 16 * t + r <= N; r++)
+                for (int j = 0; j < cols; j++)
+                    e[(size_t)r * 4 * ks + j] = cospi_ratio((long)(2 * j + par) * (16 * t + r), 2L * N);
+            dmfma_fragments(e, 16, 4 * ks, out);
+        }
 }
 
 }  // namespace rpcf_host

@@ -350,3 +350,243 @@ __global__ __launch_bounds__(cheb_dmfma::DShape<FN>::NT, 3) void k_p2s_dmfma(
         if (o == 0) __syncthreads();  // the stage is read before N_eta overwrites it
     }
 }
+
+// -------------------------------------------------------------------------------------
+// The Chebyshev transforms of lengths without a compiled plan (any N = nz - 1), as the same
+// kind of FP64 matrix products with N a run-time number.  The runtime-plan FFT kernels they
+// replace (k_cheb_s2p<1, 0>, k_p2s_nl<0>; RPCF_P2S_MFMA=0 keeps them) run 3 to 5 passes over
+// LDS with index arithmetic by run-time strides: at 40x46x60 (N = 45) 72 and 62 us against
+// 11.5 and 10.9 here, at 100x151x100 (N = 150, where the product's N^2 meets the FFT's N log N)
+// 352 and 281 against 182 and 70.  Bound by the latency of a block's phases on small grids, by
+// the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.3 and
+// 0.4 of 72 TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
+// -------------------------------------------------------------------------------------
+namespace cheb_dmfma {
+
+// Sizes of the products of one N.  Rows of the p2s: sym p <= N/2 (NS), anti p <= (N-1)/2 (NA),
+// each in RT row tiles; samples q <= N in NCH chunks of kNChunk.  Rows of the s2p: q <= N in
+// RQ tiles; even and odd coefficients in KE and KO k-steps.  All tables are zero-padded.
+constexpr int kNChunk = 16;
+struct NShape {
+    int N, NS, NA, RT, NCH, KP, RQ, KE, KO;
+    long s2p_off;  // doubles: the s2p table behind the p2s tables
+    long doubles;
+};
+inline NShape nshape(int N) {
+    NShape s;
+    s.N = N;
+    s.NS = N / 2 + 1;
+    s.NA = (N + 1) / 2;
+    s.RT = ceil_div(s.NS, 16);
+    s.NCH = ceil_div(N + 1, kNChunk);
+    s.KP = s.NCH * (kNChunk / 4);
+    s.RQ = ceil_div(N + 1, 16);
+    s.KE = ceil_div(N / 2 + 1, 4);
+    s.KO = ceil_div((N + 1) / 2, 4);
+    s.s2p_off = 4L * s.RT * s.KP * 64;
+    s.doubles = s.s2p_off + (long)s.RQ * (s.KE + s.KO) * 64;
+    return s;
+}
+// LDS bytes: the operands [set h3, h2, h1][G+, G-][kNChunk][kCols] or the output rows
+// [pencil][nz] of one term; the coefficients [even, odd][4 KE]
+inline size_t p2s_n_lds(const NShape& s) {
+    const size_t ops = sizeof(double) * 3 * 2 * kNChunk * kCols, out = sizeof(double2) * kPencils * (s.N + 1);
+    return ops > out ? ops : out;
+}
+// (rows of kS2pLd doubles: 16 bytes past a full turn of the banks, for the writes along k)
+constexpr int kS2pLd = kCols + 2;
+inline size_t s2p_n_lds(const NShape& s) { return sizeof(double) * 2 * 4 * s.KE * kS2pLd; }
+
+}  // namespace cheb_dmfma
+
+// Padded p2s + derivative + rhsNonlinear + unpadded s2p (as k_p2s_dmfma), one item a block:
+// 2 RT waves, wave w < RT the sym row tile w, the others the anti tiles, each over both column
+// tiles.  The centre sample q = N is a sample like the others (G+ = f_N, G- = 0).
+template <int RT>
+__global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restrict__ Z1, long zstride, long sY,
+                                                          double2* __restrict__ NL, long sNL, Dims d,
+                                                          const double* __restrict__ tab, cheb_dmfma::NShape sh,
+                                                          Members mb) {
+    using namespace cheb_dmfma;
+    constexpr int NT = 128 * RT, UPT = ceil_div(kNChunk * kPencils, NT);
+    RPCF_LDS(double);
+    const int N = sh.N, nz = N + 1, pz = 2 * N + 1;
+    const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, lc = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const bool anti = wave >= RT;
+    const int rt = anti ? wave - RT : wave;
+    const int slot = mb.ids[blockIdx.z], kx = blockIdx.y, ky0 = blockIdx.x * kPencils;
+    const int nb = min(kPencils, d.ny - ky0);
+    const double2* in = Z1 + slot * sY + (long)kx * pz * d.ny + ky0;
+    const double aphi = mb.mp[slot].aphi, beta = mb.mp[slot].beta;
+    double2 sa[UPT][3], sb[UPT][3];
+    auto load = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < UPT; u++) {
+            const int i = tid + u * NT, q = c * kNChunk + i / kPencils, b = i % kPencils;
+            const bool ok = i < kNChunk * kPencils && q <= N && b < nb;
+            const long oa = ok ? (long)q * d.ny + b : 0, ob = ok ? (long)(2 * N - q) * d.ny + b : 0;
+#pragma unroll
+            for (int g = 0; g < 3; g++) {
+                sa[u][g] = in[g * zstride + oa];
+                sb[u][g] = in[g * zstride + ob];
+            }
+        }
+    };
+    auto stage = [&](int c) {
+#pragma unroll
+        for (int u = 0; u < UPT; u++) {
+            const int i = tid + u * NT;
+            if (i >= kNChunk * kPencils) continue;
+            const int qq = i / kPencils, b = i % kPencils, q = c * kNChunk + qq, ky = ky0 + b;
+            const double ia = (double)kx / aphi;
+            const double ib = ky >= d.ny / 2 + 1 ? (double)(ky - d.ny) / beta : (double)ky / beta;
+            const double k2 = ia * ia + ib * ib;
+            const bool mean = kx == 0 && ky == 0, ok = b < nb && q <= N;
+#pragma unroll
+            for (int pm = 0; pm < 2; pm++) {
+                double2 f[3];
+#pragma unroll
+                for (int g = 0; g < 3; g++) {
+                    const double2 a = sa[u][g], m = sb[u][g];
+                    f[g] = pm ? make_double2(a.x - m.x, a.y - m.y) : make_double2(a.x + m.x, a.y + m.y);
+                    if (q == N) f[g] = pm ? make_double2(0.0, 0.0) : a;
+                    if (!ok) f[g] = make_double2(0.0, 0.0);
+                }
+                const double2 x = f[0], y = f[1], z = f[2];
+                const double2 h3 = mean ? y : make_double2(-ia * y.y + ib * x.y, ia * y.x - ib * x.x);
+                const double2 h2 = mean ? make_double2(0.0, 0.0)
+                                        : make_double2(-ia * x.y - ib * y.y, ia * x.x + ib * y.x);
+                const double2 h1 = mean ? x : make_double2(k2 * z.x, k2 * z.y);
+                double* o = lds + (pm * kNChunk + qq) * kCols + b;
+                o[0] = h3.x;
+                o[kPencils] = h3.y;
+                o[2 * kNChunk * kCols] = h2.x;
+                o[2 * kNChunk * kCols + kPencils] = h2.y;
+                o[4 * kNChunk * kCols] = h1.x;
+                o[4 * kNChunk * kCols + kPencils] = h1.y;
+            }
+        }
+    };
+    // tables Q0s, Q0a, Q1s, Q1a, [RT][KP] fragments each: sym waves Q0 = Q0s over G+ (h3, h1),
+    // Q1 = Q1s over G- (h2); anti waves Q0a over G-, Q1a over G+
+    const long tsz = (long)RT * sh.KP * 64;
+    const double* tq0 = tab + (anti ? tsz : 0) + (long)rt * sh.KP * 64 + lane;
+    const double* tq1 = tq0 + 2 * tsz;
+    const int pm0 = anti ? 1 : 0;
+    auto bop = [&](int set, int pm, int sl, int ct) {
+        return lds[((set * 2 + pm) * kNChunk + 4 * sl + kq) * kCols + ct * kPencils + lc];
+    };
+    const v4d zero4 = {0.0, 0.0, 0.0, 0.0};
+    v4d accE[2] = {zero4, zero4}, accV[2] = {zero4, zero4};
+    load(0);
+    for (int c = 0; c < sh.NCH; c++) {
+        stage(c);
+        double f0[kNChunk / 4], f1[kNChunk / 4];
+#pragma unroll
+        for (int sl = 0; sl < kNChunk / 4; sl++) {
+            f0[sl] = tq0[(long)(c * (kNChunk / 4) + sl) * 64];
+            f1[sl] = tq1[(long)(c * (kNChunk / 4) + sl) * 64];
+        }
+        __syncthreads();
+        if (c + 1 < sh.NCH) load(c + 1);
+#pragma unroll
+        for (int sl = 0; sl < kNChunk / 4; sl++)
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++) {
+                accE[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0[sl], bop(0, pm0, sl, ct), accE[ct], 0, 0, 0);
+                accV[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(f0[sl], bop(2, pm0, sl, ct), accV[ct], 0, 0, 0);
+                accV[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[sl], bop(1, 1 - pm0, sl, ct), accV[ct], 0, 0, 0);
+            }
+        __syncthreads();  // the operands are read before the next chunk or the output overwrites them
+    }
+    // sym waves write S to rows p and N - p, then the anti waves add and subtract A
+    const int ph = mb.phase[slot];
+    const long PS = (long)d.P * nz, po = ((long)ky0 * d.hnx + kx) * nz, pstride = (long)d.hnx * nz;
+    double* out = lds;
+#pragma unroll
+    for (int o = 0; o < 2; o++) {
+        const v4d* acc = o ? accE : accV;
+#pragma unroll
+        for (int half = 0; half < 2; half++) {
+            if ((half == 1) == anti) {
+#pragma unroll
+                for (int r = 0; r < 4; r++) {
+                    const int p = 16 * rt + kq + 4 * r;
+                    if (p >= (anti ? sh.NA : sh.NS)) continue;
+#pragma unroll
+                    for (int ct = 0; ct < 2; ct++) {
+                        double* a = out + (lc * nz + p) * 2 + ct;
+                        double* m = out + (lc * nz + N - p) * 2 + ct;
+                        if (anti) *a += acc[ct][r], *m -= acc[ct][r];
+                        else *a = acc[ct][r], *m = acc[ct][r];
+                    }
+                }
+            }
+            __syncthreads();
+        }
+        double2* dst = NL + slot * sNL + (o ? 2 + ph : ph) * PS;
+        const double2* ov = (const double2*)out;
+        for (int bb = wave; bb < nb; bb += 2 * RT)
+            for (int j = lane; j < nz; j += 64) dst[po + bb * pstride + j] = ov[bb * nz + j];
+        if (o == 0) __syncthreads();
+    }
+}
+
+// Padded s2p: F[6][P][nz] -> Y[6][kx][q][ky], one block of four waves per 16 pencils of a field.
+// The pencils' coefficients lie in LDS as B operands; a wave takes row tiles q of the even and
+// odd products (fragments from L2), rows q and 2N - q are their sum and difference, stored from
+// the accumulators: 16 pencils of a row are 256 contiguous bytes.
+__global__ __launch_bounds__(256) void k_s2p_dmfma_n(const double2* __restrict__ F, long fstride, long sF,
+                                                     double2* __restrict__ Y, long ystride, long sY, Dims d,
+                                                     const double* __restrict__ tab, cheb_dmfma::NShape sh,
+                                                     const int* __restrict__ ids) {
+    using namespace cheb_dmfma;
+    RPCF_LDS(double);
+    const int N = sh.N, nz = N + 1, pz = 2 * N + 1, KE = sh.KE, KO = sh.KO;
+    const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, lc = lane & 15;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int f = blockIdx.z % 6, kx = blockIdx.y, ky0 = blockIdx.x * kPencils;
+    const long slot = ids[blockIdx.z / 6];
+    const int nb = min(kPencils, d.ny - ky0);
+    const double2* in = F + slot * sF + f * fstride + ((long)ky0 * d.hnx + kx) * nz;
+    double2* out = Y + slot * sY + f * ystride + (long)kx * pz * d.ny + ky0;
+    const int rows = 4 * KE;  // of each parity, zero past the coefficients
+    for (int b = wave; b < kPencils; b += 4)
+        for (int k = lane; k < 2 * rows; k += 64) {
+            const double2 v = b < nb && k < nz ? in[(long)b * d.hnx * nz + k] : make_double2(0.0, 0.0);
+            double* o = lds + ((k & 1) * rows + (k >> 1)) * kS2pLd + b;
+            o[0] = v.x;
+            o[kPencils] = v.y;
+        }
+    __syncthreads();
+    const v4d zero4 = {0.0, 0.0, 0.0, 0.0};
+    for (int rt = wave; rt < sh.RQ; rt += 4) {
+        const double* te = tab + sh.s2p_off + (long)rt * (KE + KO) * 64 + lane;
+        const double* to = te + (long)KE * 64;
+        v4d e[2] = {zero4, zero4}, o[2] = {zero4, zero4};
+#pragma unroll 4
+        for (int s = 0; s < KE; s++) {
+            const double a = te[(long)s * 64];
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+                e[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, lds[(4 * s + kq) * kS2pLd + ct * kPencils + lc], e[ct], 0, 0, 0);
+        }
+#pragma unroll 4
+        for (int s = 0; s < KO; s++) {
+            const double a = to[(long)s * 64];
+#pragma unroll
+            for (int ct = 0; ct < 2; ct++)
+                o[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, lds[(rows + 4 * s + kq) * kS2pLd + ct * kPencils + lc], o[ct], 0, 0, 0);
+        }
+        if (lc < nb) {
+#pragma unroll
+            for (int r = 0; r < 4; r++) {
+                const int q = 16 * rt + kq + 4 * r;
+                if (q > N) continue;
+                out[(long)q * d.ny + lc] = make_double2(e[0][r] + o[0][r], e[1][r] + o[1][r]);
+                if (q < N) out[(long)(2 * N - q) * d.ny + lc] = make_double2(e[0][r] - o[0][r], e[1][r] - o[1][r]);
+            }
+        }
+    }
+}

@@ -376,88 +376,9 @@ struct LinState {
 // with T4q = T4*dt*0.5/Re and T2q = T2*0.5/Re*dt (the quotients of source/linear.cpp:100,
 // 142).  The reference rebuilds B_rj = f(T0, T2, T4) per element (source/linear.cpp:95-107,
 // 137-153); by linearity sum_j v_j B_rj is a combination of these row products, so one
-// pass over the operator tables serves the NPB pencils of a block (real-matrix times
-// complex-vector products, fused multiply-adds).  Register tile: a thread owns 4 rows x
-// 8 pencils of one product m, so each vector element read from LDS feeds 8 FMAs
-// (tables transposed: Tt[j*nz + p], vectors in LDS as [j][pencil]).
-// -------------------------------------------------------------------------------------
-constexpr int kTvRows = 4, kTvCols = 8;
-
-template <int NPB>
-__global__ __launch_bounds__(384) void k_lin_tv(const double2* __restrict__ sv, const double2* __restrict__ se, long sS,
-                                                double2* __restrict__ W, long sWl, Dims d, const double* __restrict__ T0t,
-                                                const double* __restrict__ T2t, const double* __restrict__ T4q,
-                                                const double* __restrict__ T2q, long sQ, const int* __restrict__ ids) {
-    {
-        const long slot = ids[blockIdx.y];
-        sv += slot * sS;
-        se += slot * sS;
-        W += slot * sWl;
-        T4q += slot * sQ;
-        T2q += slot * sQ;
-    }
-    static_assert(NPB % kTvCols == 0, "pencil tile");
-    extern __shared__ __align__(16) unsigned char tv_lds_raw[];
-    constexpr int LDX = NPB + 1;  // padded row: the transposing stores hit different banks
-    double2* xv = (double2*)tv_lds_raw;  // [nz][LDX]
-    double2* xe = xv + (size_t)d.nz * LDX;
-    const int n = d.nz, p0 = blockIdx.x * NPB;
-    const int np = min(NPB, d.P - p0);
-    for (int i = threadIdx.x; i < NPB * n; i += blockDim.x) {
-        const int q = i / n, j = i - q * n;
-        const bool ok = q < np;
-        xv[j * LDX + q] = ok ? sv[(long)(p0 + q) * n + j] : make_double2(0.0, 0.0);
-        xe[j * LDX + q] = ok ? se[(long)(p0 + q) * n + j] : make_double2(0.0, 0.0);
-    }
-    __syncthreads();
-    constexpr int NH = NPB / kTvCols;
-    const int ngr = (n + kTvRows - 1) / kTvRows;
-    for (int u = threadIdx.x; u < 5 * ngr * NH; u += blockDim.x) {
-        const int m = u / (ngr * NH), rem = u - m * ngr * NH;
-        const int g = rem / NH, h = rem - g * NH;
-        const int pb = g * kTvRows, qb = h * kTvCols;
-        const double* T = m == 0 || m == 3 ? T0t : (m == 1 ? T2t : (m == 2 ? T4q : T2q));
-        const double2* X = (m < 3 ? xv : xe) + qb;
-        double ar[kTvRows][kTvCols], ai[kTvRows][kTvCols];
-#pragma unroll
-        for (int i = 0; i < kTvRows; i++)
-#pragma unroll
-            for (int q = 0; q < kTvCols; q++) ar[i][q] = ai[i][q] = 0.0;
-        // the table column of j+1 is loaded while column j is used
-        double cn[kTvRows];
-#pragma unroll
-        for (int i = 0; i < kTvRows; i++) cn[i] = pb + i < n ? T[pb + i] : 0.0;
-        for (int j = 0; j < n; j++) {
-            double c[kTvRows];
-#pragma unroll
-            for (int i = 0; i < kTvRows; i++) {
-                c[i] = cn[i];
-                cn[i] = (j + 1 < n && pb + i < n) ? T[(long)(j + 1) * n + pb + i] : 0.0;
-            }
-#pragma unroll
-            for (int q = 0; q < kTvCols; q++) {
-                const double2 x = X[j * LDX + q];
-#pragma unroll
-                for (int i = 0; i < kTvRows; i++) {
-                    ar[i][q] = fma(c[i], x.x, ar[i][q]);
-                    ai[i][q] = fma(c[i], x.y, ai[i][q]);
-                }
-            }
-        }
-        double2* out = W + (long)m * d.P * n;
-#pragma unroll
-        for (int q = 0; q < kTvCols; q++)
-            if (qb + q < np)
-#pragma unroll
-                for (int i = 0; i < kTvRows; i++)
-                    if (pb + i < n) out[(long)(p0 + qb + q) * n + pb + i] = make_double2(ar[i][q], ai[i][q]);
-    }
-}
-
-// -------------------------------------------------------------------------------------
-// The same operator products on the matrix cores: W[m] = T_m X with X the nz x 2P real
-// matrix of (Re, Im) columns, by v_mfma_f64_16x16x4_f64 (A: lane l holds A[l%16][l/16],
-// B: lane l holds B[l/16][l%16], D: item r of lane l is D[l/16 + 4r][l%16]).
+// pass over the operator tables serves many pencils.  On the matrix cores: W[m] = T_m X with
+// X the nz x 2P real matrix of (Re, Im) columns, by v_mfma_f64_16x16x4_f64 (A: lane l holds
+// A[l%16][l/16], B: lane l holds B[l/16][l%16], D: item r of lane l is D[l/16 + 4r][l%16]).
 // The Chebyshev tables have the reflection parity T_m[N-i][j] = (-1)^j T_m[i][j] (m = 0, 2,
 // 4 at the symmetric points), so with E_i = sum_{j even} T_m[i][j] x_j and
 // O_i = sum_{j odd} T_m[i][j] x_j for the rows i <= N/2,
@@ -479,6 +400,16 @@ constexpr int kTvBlockPencils = 32;
 // 128x129x128.  Longer Chebyshev lengths (S = 25, 33) hold 4 S B-fragment registers and
 // would spill at three waves, so they run two.
 constexpr int tv_waves(int s) { return s <= 17 ? 3 : 2; }
+// Instantiated k-step counts: those of the compiled Chebyshev lengths; another length takes the
+// next one up (its table is zero-padded): 7.7 us at 40x46x60 (S = 7 for the 6 it needs)
+// and 104 at 100x151x100 (25 for 19) against 33 and 489 for a kernel on the vector units.
+#define RPCF_TV_STEPS(X) X(2) X(3) X(4) X(5) X(7) X(9) X(13) X(17) X(25) X(33)
+inline int tv_steps(int need) {
+#define RPCF_CASE(S) if (need <= S) return S;
+    RPCF_TV_STEPS(RPCF_CASE)
+#undef RPCF_CASE
+    return 0;
+}
 template <int S>  // k-steps per parity: S >= ceil((N/2 + 1)/4)
 __global__ __launch_bounds__(256, tv_waves(S)) void k_lin_tv_mfma(const double2* __restrict__ sv, const double2* __restrict__ se,
                                                      long sS, double2* __restrict__ W, long sWl, Dims d,
@@ -616,8 +547,8 @@ __global__ __launch_bounds__(64 * NW) void k_lin_tv_stream(const double2* __rest
         }
         const int p = g * 8 + (col >> 1);
         double* Wm = Wm0 + (long)p * 2 * n;
-        // a last row tile that holds only the centre row p = N/2 (N/2 a multiple of 16) is a
-        // dot product on the vector units: lane (column, kq) sums its k-steps' row-0 entries
+        // a last row tile that holds only the row p = N/2 (N/2 a multiple of 16; the centre row
+        // where N is even) is a dot product on the vector units: lane (column, kq) sums its k-steps' row-0 entries
         // times its coefficients, then the four kq lanes of the column add up
         const int RTm = 16 * (RT - 1) + 1 == rows ? RT - 1 : RT;
         if (RTm < RT) {
@@ -631,7 +562,10 @@ __global__ __launch_bounds__(64 * NW) void k_lin_tv_stream(const double2* __rest
             o += __shfl_xor(o, 16);
             e += __shfl_xor(e, 32);
             o += __shfl_xor(o, 32);
-            if (kq == 0 && p < d.P) Wm[2 * (N / 2)] = e + o;
+            if (kq == 0 && p < d.P) {
+                Wm[2 * (N / 2)] = e + o;
+                if (N & 1) Wm[2 * (N - N / 2)] = e - o;
+            }
         }
         for (int t = 0; t < RTm; t++) {
             // the row tile's table fragments first, so that no product waits on an LDS read

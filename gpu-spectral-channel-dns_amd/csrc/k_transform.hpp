@@ -30,6 +30,7 @@ constexpr int cheb_nl_tile_max(int fn) { return fn > 0 && fn <= 128 ? 2 * kChebT
 constexpr int s2p_tile_max(int fn) { return fn >= 192 || fn == 0 ? kChebTile : fn >= 96 ? 2 * kChebTile : 4 * kChebTile; }
 constexpr int kSpanTile = 16;
 constexpr int kLambPairs = 2;  // pairs of span rows per block of k_lamb_phys
+constexpr int kC2rRows = 8;    // pairs of span rows per block of k_x_c2r
 // ... and their bounds for a compiled transform length: shorter rows and columns take wider
 // tiles, so that a block keeps about the work and LDS it has at length 192.
 constexpr int span_tile_max(int fn) { return fn >= 192 || fn == 0 ? kSpanTile : 2 * kSpanTile; }
@@ -346,35 +347,33 @@ __global__ __launch_bounds__(256) void k_span_inv(const cplx<R>* __restrict__ Y,
         const int nk = NK ? NK : nk_rt;
         const int my = FN ? FN : d.my, ldl = FN ? FN + 1 : ld, tid = threadIdx.x, nthr = blockDim.x;
         const int ny = d.ny, nxh = d.nxh;
+        const ConstDiv<FN> by_my(my);
+        const ConstDiv<NK> by_nk(nk);
         const C2* in = Y + f * ystride;
         staged<12>(
             nk * my, tid, nthr,
             [&](int i) {
-                const unsigned kxi = (unsigned)i / my, s = i - kxi * my;
+                const unsigned kxi = (unsigned)i / by_my, s = i - kxi * my;
                 const int ky = ky_of_span(d, s);
                 return ky >= 0 ? in[((kx0 + kxi) * planes + q) * ny + ky] : cmake<C2>(0, 0);
             },
             [&](int i, C2 v) {
-                const unsigned kxi = (unsigned)i / my, s = i - kxi * my;
+                const unsigned kxi = (unsigned)i / by_my, s = i - kxi * my;
                 lds[kxi * ldl + s] = v;
             });
-        FftPlan pll = pl;  // compiled lengths: twiddles from an LDS copy behind the tile
-        if constexpr (FN > 0) {
-            C2* twl = lds + TK * ldl;
-            for (int i = tid; i < ct_tw_lds_len(FN); i += nthr) twl[i] = ((const C2*)pl.tw)[ct_tw_lds_src(FN, i)];
-            pll.tw = twl;
-        }
+        FftPlan pll = pl;  // twiddles from an LDS copy behind the tile
+        copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, +1, span_tile_max(FN), 1, true>(lds, ldl, nk, pll, tid, nthr);
         C2* out = W + f * wstride;
         staged<12>(
             my * nk, tid, nthr,
             [&](int i) {
-                const unsigned s = (unsigned)i / nk, kxi = i - s * nk;
+                const unsigned s = (unsigned)i / by_nk, kxi = i - s * nk;
                 return lds[kxi * ldl + s];
             },
             [&](int i, C2 v) {
-                const unsigned s = (unsigned)i / nk, kxi = i - s * nk;
+                const unsigned s = (unsigned)i / by_nk, kxi = i - s * nk;
                 out[(q * my + s) * nxh + kx0 + kxi] = v;
             });
     };
@@ -442,6 +441,11 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
         const int lds_ld = FN ? FN + 1 : ld;
         const int my = d.my, tid = threadIdx.x, nthr = blockDim.x;
         const int ws = (int)wstride, zs = (int)zstride;
+        const ConstDiv<FN> by_mx(mx);
+        const ConstDiv<FN ? (FN / 3 * 2) / 2 : 0> by_nxh(nxh);
+        const ConstDiv<FN ? (FN / 3 * 2) / 2 + 1 : 0> by_hnx(hnx);
+        const ConstDiv<FN ? FN - 2 * ((FN / 3 * 2) / 2) + 1 : 0> by_nzero(mx - 2 * nxh + 1);
+        const ConstDiv<NC> by_nrp(nrp);
         // packed spectra Z = X_A + i X_B of the row pairs (c2r_pack, element by element):
         // each kept coefficient pair (A_k, B_k), k < nxh, is loaded once and gives Z_k and
         // Z_{mx-k}; Z_k = 0 for nxh <= k <= mx - nxh
@@ -452,8 +456,8 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
             for (int u = 0; u < KL; u++) {
                 const int i = base + u * nthr;
                 if (i < 6 * nrp * nxh) {
-                    const int seq = i / nxh, k = i - seq * nxh;
-                    const int f = seq / nrp, ip = seq - f * nrp;
+                    const int seq = (unsigned)i / by_nxh, k = i - seq * nxh;
+                    const int f = (unsigned)seq / by_nrp, ip = seq - f * nrp;
                     const C2* rA = W + (f * ws + (q * my + 2 * (rp0 + ip)) * nxh);
                     va[u] = rA[k];
                     vb[u] = rA[nxh + k];
@@ -463,7 +467,7 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
             for (int u = 0; u < KL; u++) {
                 const int i = base + u * nthr;
                 if (i < 6 * nrp * nxh) {
-                    const int seq = i / nxh, k = i - seq * nxh;
+                    const int seq = (unsigned)i / by_nxh, k = i - seq * nxh;
                     C2 a = va[u], b = vb[u];
                     C2* z = lds + seq * lds_ld;
                     if (k == 0) {
@@ -478,18 +482,13 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
         }
         const int nzero = mx - 2 * nxh + 1;
         for (int i = tid; i < 6 * nrp * nzero; i += nthr) {
-            const int seq = i / nzero, k = i - seq * nzero;
+            const int seq = (unsigned)i / by_nzero, k = i - seq * nzero;
             lds[seq * lds_ld + nxh + k] = cmake<C2>(0, 0);
         }
-        // compiled lengths: the FFT twiddles from an LDS copy behind the sequences, so that
-        // no butterfly waits on a global load
+        // the FFT twiddles from an LDS copy behind the sequences, so that no butterfly waits on
+        // a global load
         FftPlan pll = pl;
-        if constexpr (FN > 0) {
-            C2* twl = lds + 6 * RP * lds_ld;
-            const C2* twg = (const C2*)pl.tw;
-            for (int i = tid; i < ct_tw_lds_len(FN); i += nthr) twl[i] = twg[ct_tw_lds_src(FN, i)];
-            pll.tw = twl;
-        }
+        copy_tw<FN>(lds + 6 * RP * lds_ld, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, +1, 6 * lamb_pairs_max(FN), 1, true>(lds, lds_ld, 6 * nrp, pll, tid, nthr);
         // Ro U(y) is uniform in x and span, so it reaches only the (0,0) pencil of L_z, which
@@ -497,7 +496,7 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
         // swamp the perturbation products); the FP64 form keeps the reference's expression.
         const R mU = sizeof(R) == 8 ? (R)meanU[q] : R(0);
         for (int i = tid; i < nrp * mx; i += nthr) {
-            const int ip = i / mx, x = i - ip * mx;
+            const int ip = (unsigned)i / by_mx, x = i - ip * mx;
             const C2 u = lds[(0 * nrp + ip) * lds_ld + x], v = lds[(1 * nrp + ip) * lds_ld + x];
             const C2 w = lds[(2 * nrp + ip) * lds_ld + x], ox = lds[(3 * nrp + ip) * lds_ld + x];
             const C2 oy = lds[(4 * nrp + ip) * lds_ld + x], oz = lds[(5 * nrp + ip) * lds_ld + x];
@@ -511,8 +510,8 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
         __syncthreads();
         fft_any<FN, -1, 3 * lamb_pairs_max(FN), 1, true>(lds, lds_ld, 3 * nrp, pll, tid, nthr);
         for (int i = tid; i < 3 * nrp * hnx; i += nthr) {
-            const int seq = i / hnx, k = i - seq * hnx;
-            const int g = seq / nrp, ip = seq - g * nrp;
+            const int seq = (unsigned)i / by_hnx, k = i - seq * hnx;
+            const int g = (unsigned)seq / by_nrp, ip = seq - g * nrp;
             C2 xa, xb;
             r2c_unpack(lds + seq * lds_ld, k, mx, (R)fac, &xa, &xb);
             C2* o = Z2 + (g * zs + (q * my + 2 * (rp0 + ip)) * zld);
@@ -524,21 +523,31 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
     else body(IntC<0>{});
 }
 
-// x C2R of one field (no Lamb): W[q][s][nxh] -> phys[q][s][mx] (rpcf_spec_to_phys).
+// x C2R of one field (no Lamb): W[q][s][nxh] -> phys[q][s][mx] (rpcf_spec_to_phys).  LDS: [RP][ld]
+// sequences, then the twiddles.
+template <int FN = 0>
 __global__ __launch_bounds__(256) void k_x_c2r(const double2* __restrict__ W, double* __restrict__ phys, Dims d, FftPlan pl, int RP, int ld) {
     RPCF_LDS(double2);
     const int q = blockIdx.y, rp0 = blockIdx.x * RP;
     const int nrp = min(RP, d.my / 2 - rp0);
-    const int mx = d.mx, my = d.my, nxh = d.nxh, tid = threadIdx.x, nthr = blockDim.x;
-    for (int i = tid; i < nrp * mx; i += nthr) {
-        const int ip = i / mx, k = i - ip * mx;
-        const double2* rA = W + ((long)q * my + 2 * (rp0 + ip)) * nxh;
-        lds[ip * ld + k] = c2r_pack(rA, rA + nxh, k, mx, nxh);
-    }
+    const int mx = FN ? FN : d.mx, my = d.my, nxh = d.nxh, tid = threadIdx.x, nthr = blockDim.x;
+    const ConstDiv<FN> by_mx(mx);
+    staged<8>(
+        nrp * mx, tid, nthr,
+        [&](int i) {
+            const unsigned ip = (unsigned)i / by_mx, k = i - ip * mx;
+            const double2* rA = W + ((long)q * my + 2 * (rp0 + ip)) * nxh;
+            return c2r_pack(rA, rA + nxh, k, mx, nxh);
+        },
+        [&](int i, double2 v) {
+            const unsigned ip = (unsigned)i / by_mx, k = i - ip * mx;
+            lds[ip * ld + k] = v;
+        });
+    copy_tw<FN>(lds + RP * ld, pl, tid, nthr);
     __syncthreads();
-    fft_run<+1>(lds, ld, nrp, pl, tid, nthr);
+    fft_any<FN, +1, kC2rRows, 1, true>(lds, ld, nrp, pl, tid, nthr);
     for (int i = tid; i < nrp * mx; i += nthr) {
-        const int ip = i / mx, x = i - ip * mx;
+        const int ip = (unsigned)i / by_mx, x = i - ip * mx;
         double* rowA = phys + ((long)q * my + 2 * (rp0 + ip)) * mx;
         const double2 z = lds[ip * ld + x];
         rowA[x] = z.x;
@@ -599,34 +608,32 @@ __global__ __launch_bounds__(256) void k_span_fwd(const cplx<R>* __restrict__ Z2
         constexpr int NK = decltype(nkc)::value;
         const int nk = NK ? NK : nk_rt;
         const int my = FN ? FN : d.my, ldl = FN ? FN + 1 : ld, ny = d.ny, tid = threadIdx.x, nthr = blockDim.x;
+        const ConstDiv<NK> by_nk(nk);
+        const FastDiv by_ny(ny);
         const C2* in = Z2 + g * zstride;
         staged<12>(
             my * nk, tid, nthr,
             [&](int i) {
-                const unsigned s = (unsigned)i / nk, kxi = i - s * nk;
+                const unsigned s = (unsigned)i / by_nk, kxi = i - s * nk;
                 return in[(q * my + s) * zld + kx0 + kxi];
             },
             [&](int i, C2 v) {
-                const unsigned s = (unsigned)i / nk, kxi = i - s * nk;
+                const unsigned s = (unsigned)i / by_nk, kxi = i - s * nk;
                 lds[kxi * ldl + s] = v;
             });
-        FftPlan pll = pl;  // compiled lengths: twiddles from an LDS copy behind the tile
-        if constexpr (FN > 0) {
-            C2* twl = lds + TK * ldl;
-            for (int i = tid; i < ct_tw_lds_len(FN); i += nthr) twl[i] = ((const C2*)pl.tw)[ct_tw_lds_src(FN, i)];
-            pll.tw = twl;
-        }
+        FftPlan pll = pl;  // twiddles from an LDS copy behind the tile
+        copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, -1, span_tile_max(FN), 1, true>(lds, ldl, nk, pll, tid, nthr);
         C2* out = Z1 + g * ostride;
         staged<8>(
             nk * ny, tid, nthr,
             [&](int i) {
-                const unsigned kxi = (unsigned)i / ny, ky = i - kxi * ny;
+                const unsigned kxi = (unsigned)i / by_ny, ky = i - kxi * ny;
                 return lds[kxi * ldl + span_of(d, ky)];
             },
             [&](int i, C2 v) {
-                const unsigned kxi = (unsigned)i / ny, ky = i - kxi * ny;
+                const unsigned kxi = (unsigned)i / by_ny, ky = i - kxi * ny;
                 out[((kx0 + kxi) * planes + q) * ny + ky] = v;
             });
     };

@@ -43,7 +43,8 @@ const char* const kKernelNames[KID_COUNT] = {"k_velocity", "k_cheb_s2p", "k_span
                                              "k_span_fwd", "k_p2s_nl",   "k_lin_tv",   "k_lin_solve"};
 
 constexpr int kFftThreads = 256;
-constexpr int kTvPencils = 16;  // pencils per block of the fallback k_lin_tv
+// row tiles of k_p2s_dmfma_n: ceil((N/2 + 1)/16), N <= 255
+#define RPCF_P2S_TILES(X) X(1) X(2) X(3) X(4) X(5) X(6) X(7) X(8)
 
 struct Pending {
     int kid;
@@ -96,7 +97,10 @@ struct rpcf_ctx {
     int mt_s0 = 0, mt_s1 = 0;
     // FP64 form: the padded p2s with the nonlinear combination as FP64 products (k_cheb_dmfma.hpp)
     int use_dmfma = 0;
-    double* DT = nullptr;  // fragments of the folded p2s tables
+    // lengths without a compiled plan: s2p and p2s as FP64 products of run-time size
+    int use_dmfma_n = 0;
+    cheb_dmfma::NShape dn{};
+    double* DT = nullptr;  // fragments of the tables of either
     // per-slot arrays ([capacity][...]) and their slot strides in elements
     double2* F = nullptr;     // [6][P][nz] u, v, w, ox, oy, oz
     double2* SV = nullptr;    // [P][nz] v-hat (u0 in pencil 0)
@@ -115,15 +119,13 @@ struct rpcf_ctx {
     int4* PAIRS = nullptr;    // [2][np] row pairs (i, i', sign, 0) of the v and eta systems
     int npair = 0;            // np = N/2 + 1
     double* TF = nullptr;     // [5][RT][S][64] MFMA A-operand tiles of T0, T2, T4q, T0, T2q
-    double* T4Q = nullptr;    // [nz*nz] T4*dt*0.5/Re, transposed (fallback operator products)
-    double* T2Q = nullptr;    // [nz*nz] T2*0.5/Re*dt, transposed
     double *U = nullptr, *DU = nullptr, *DDU = nullptr;  // [nz] base profile at the collocation points
     double* MEANU = nullptr;                             // [pz] base profile at the padded points
     MemberParams* MP = nullptr;                          // [capacity]
     int* PH = nullptr;                                   // [capacity] history phase
-    long sF = 0, sS = 0, sNL = 0, sY = 0, sW = 0, sZ = 0, sWl = 0, sM = 0, sMH = 0, sME = 0, sTf = 0, sQ = 0, sU = 0, sPz = 0;
+    long sF = 0, sS = 0, sNL = 0, sY = 0, sW = 0, sZ = 0, sWl = 0, sM = 0, sMH = 0, sME = 0, sTf = 0, sU = 0, sPz = 0;
     // shape tables shared by all slots
-    double *T0 = nullptr, *T2 = nullptr, *T4 = nullptr, *T0t = nullptr, *T2t = nullptr, *qw = nullptr, *tw = nullptr;
+    double *T0 = nullptr, *T2 = nullptr, *T4 = nullptr, *T0t = nullptr, *qw = nullptr, *tw = nullptr;
     std::vector<double> T0h, T2h, T4h, qw_host;
     // slot-id lists on the device: ids_zero = {0}; ids = the list of the last grouped launch
     int* ids_dev = nullptr;
@@ -185,11 +187,11 @@ int check_sizes(const rpcf_params* prm, Dims* out) {
 
 // per-slot element counts of every per-slot array (= the slot strides)
 struct SlotSizes {
-    long F, S, NL, Y, W, Z, Wl, M, MH, ME, MF, Tf, Q, U, Pz;
+    long F, S, NL, Y, W, Z, Wl, M, MH, ME, MF, Tf, U, Pz;
     size_t bytes() const {
         return sizeof(double2) * (size_t)(F + 2 * S + NL + Y + W + Z + Wl + M + MH) + sizeof(unsigned) * (size_t)ME +
                sizeof(float2) * (size_t)MF +
-               sizeof(double) * (size_t)(Tf + 2 * Q + 3 * U + Pz) + sizeof(MemberParams) + 2 * sizeof(int);
+               sizeof(double) * (size_t)(Tf + 3 * U + Pz) + sizeof(MemberParams) + 2 * sizeof(int);
     }
 };
 
@@ -201,7 +203,7 @@ struct SlotSizes {
 SlotSizes slot_sizes(const Dims& d, int precision) {
     SlotSizes s;
     const long P = d.P, nz = d.nz, zld = (d.hnx + 7) & ~7;
-    const long RT = (d.N / 2 + 16) / 16, S = (d.N / 2 + 4) / 4;  // rows and columns per parity: N/2 + 1
+    const long RT = (d.N / 2 + 16) / 16, S = tv_steps((d.N / 2 + 4) / 4);  // rows and columns per parity: N/2 + 1
     s.F = 6 * P * nz;
     s.S = P * nz;
     s.NL = 4 * P * nz;
@@ -214,7 +216,6 @@ SlotSizes slot_sizes(const Dims& d, int precision) {
     s.ME = precision <= 1 ? (long)d.nslot * nz * (d.N / 2 + 1) : 0;  // v remainders / eta low parts
     s.MF = precision == 1 ? s.ME : 0;                                  // eta high parts
     s.Tf = 5 * 2 * RT * S * 64;
-    s.Q = nz * nz;
     s.U = nz;
     s.Pz = d.pz;
     return s;
@@ -569,6 +570,45 @@ int enq_velocity(rpcf_ctx* c, const int* ids, int n, bool cap = false) {
         cap);
 }
 
+// twiddles of a plan of length n in the LDS of the kernels that copy them there
+size_t tw_lds(int n) { return compiled_len(n) ? ct_tw_lds_len(n) : n; }
+
+// span transforms of nf fields (6 or 3 a member, or one): the compiled plan of my where there
+// is one; the mixed form has no other
+template <typename R>
+void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* W, long wS, long sW, int planes,
+              const FftPlan& pl, const int* ids) {
+    const Dims d = c->d;
+    const int TK = c->TK_inv, ld = c->ld_my;
+    dim3 g((d.nxh + TK - 1) / TK, planes, nf);
+    const size_t lds = sizeof(cplx<R>) * (TK * ld + tw_lds(d.my));
+    switch (d.my) {
+#define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
+        RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+        default:
+            if constexpr (sizeof(R) == 8)
+                k_span_inv<<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids);
+    }
+}
+
+template <typename R>
+void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld, cplx<R>* Y, long yS, long sY, int planes,
+              const FftPlan& pl, const int* ids, int* phase) {
+    const Dims d = c->d;
+    const int TK = c->TK_fwd, ld = c->ld_my;
+    dim3 g((d.hnx + TK - 1) / TK, planes, nf);
+    const size_t lds = sizeof(cplx<R>) * (TK * ld + tw_lds(d.my));
+    switch (d.my) {
+#define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
+        RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+        default:
+            if constexpr (sizeof(R) == 8)
+                k_span_fwd<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase);
+    }
+}
+
 // Backward transforms, Lamb vector, forward transforms and rhsNonlinear of the listed
 // slots with the intermediates Y, W, Z2 and the x/span FFTs in precision R (FP64, or FP32
 // in the mixed form); the Chebyshev transforms and everything that reaches the state are
@@ -633,38 +673,26 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
                     default:
-                        if constexpr (f64)
-                            k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(c->F, fS, c->sF, Y, yS, c->sY, d,
-                                                                              c->pl_zn, tw4, TB, ld, ids);
+                        if constexpr (f64) {
+                            if (c->use_dmfma_n)
+                                k_s2p_dmfma_n<<<dim3((d.ny + cheb_dmfma::kPencils - 1) / cheb_dmfma::kPencils, d.hnx, 6 * n),
+                                                256, cheb_dmfma::s2p_n_lds(c->dn), c->stream>>>(
+                                    c->F, fS, c->sF, Y, yS, c->sY, d, c->DT, c->dn, ids);
+                            else
+                                k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(c->F, fS, c->sF, Y, yS, c->sY, d,
+                                                                                  c->pl_zn, tw4, TB, ld, ids);
+                        }
                 }
             },
             cap);
         if (rc) return rc;
     }
-    {
-        const int TK = c->TK_inv, ld = c->ld_my;
-        dim3 g((d.nxh + TK - 1) / TK, d.pz, 6 * n);
-        size_t lds = sizeof(C2) * (TK * ld + (compiled_len(d.my) ? ct_tw_lds_len(d.my) : 0));
-        rc = launch(
-            c, KID_SPAN_INV,
-            [&] {
-                switch (d.my) {
-#define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, kFftThreads, lds, c->stream>>>(Y, yS, c->sY, W, wS, c->sW, d, d.pz, ply, TK, ld, ids); break;
-                    RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
-                    default:
-                        if constexpr (f64)
-                            k_span_inv<<<g, kFftThreads, lds, c->stream>>>(Y, yS, c->sY, W, wS, c->sW, d, d.pz, ply,
-                                                                           TK, ld, ids);
-                }
-            },
-            cap);
-        if (rc) return rc;
-    }
+    rc = launch(c, KID_SPAN_INV, [&] { span_inv<R>(c, 6 * n, Y, yS, c->sY, W, wS, c->sW, d.pz, ply, ids); }, cap);
+    if (rc) return rc;
     {
         const int RP = c->RP, ld = c->ld_mx;
         dim3 g((d.my / 2 + RP - 1) / RP, d.pz, n);
-        size_t lds = sizeof(C2) * (6 * RP * ld + (compiled_len(d.mx) ? ct_tw_lds_len(d.mx) : 0));
+        size_t lds = sizeof(C2) * (6 * RP * ld + tw_lds(d.mx));
         rc = launch(
             c, KID_LAMB,
             [&] {
@@ -682,26 +710,8 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
             cap);
         if (rc) return rc;
     }
-    {
-        const int TK = c->TK_fwd, ld = c->ld_my;
-        dim3 g((d.hnx + TK - 1) / TK, d.pz, 3 * n);
-        size_t lds = sizeof(C2) * (TK * ld + (compiled_len(d.my) ? ct_tw_lds_len(d.my) : 0));
-        rc = launch(
-            c, KID_SPAN_FWD,
-            [&] {
-                switch (d.my) {
-#define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, c->sY, d, d.pz, ply, TK, ld, ids, c->PH); break;
-                    RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
-                    default:
-                        if constexpr (f64)
-                            k_span_fwd<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, c->sY, d,
-                                                                           d.pz, ply, TK, ld, ids, c->PH);
-                }
-            },
-            cap);
-        if (rc) return rc;
-    }
+    rc = launch(c, KID_SPAN_FWD, [&] { span_fwd<R>(c, 3 * n, Z2, zS, sZ, zld, Y, yS, c->sY, d.pz, ply, ids, c->PH); }, cap);
+    if (rc) return rc;
     // the AB2 history swap ran inside k_span_fwd: the new N lands in the old "previous" buffers
     if constexpr (!f64) {
         if (c->use_mfma) {
@@ -741,6 +751,25 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                 Y, yS, c->sY, c->NL, c->sNL, d, c->DT, mb, nitems, nyb);                                          \
         break;
                         RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+                    }
+                },
+                cap);
+        }
+    }
+    if constexpr (f64) {
+        if (c->use_dmfma_n) {
+            dim3 g((d.ny + cheb_dmfma::kPencils - 1) / cheb_dmfma::kPencils, d.hnx, n);
+            return launch(
+                c, KID_P2S_NL,
+                [&] {
+                    switch (c->dn.RT) {
+#define RPCF_CASE(RT)                                                                                         \
+    case RT:                                                                                                  \
+        k_p2s_dmfma_n<RT><<<g, 128 * RT, cheb_dmfma::p2s_n_lds(c->dn), c->stream>>>(Y, yS, c->sY, c->NL, c->sNL, d, \
+                                                                                   c->DT, c->dn, mb);         \
+        break;
+                        RPCF_P2S_TILES(RPCF_CASE)
 #undef RPCF_CASE
                     }
                 },
@@ -807,24 +836,18 @@ int enq_lin_tv(rpcf_ctx* c, const int* ids, int n, bool cap, hipStream_t s) {
             // a multiple of 8: the five operator blocks of one pencil range (linear ids x + gs y)
             // land on the same XCD (id mod 8), so v-hat and eta-hat come from its L2 after the first read
             if (gs >= 16) gs &= ~7;
-            switch (2 * d.N) {
-#define RPCF_CASE(L)                                                                                             \
-    case L:                                                                                                      \
+            switch (c->tv_s) {
+#define RPCF_CASE(S)                                                                                             \
+    case S:                                                                                                      \
         if (tv_stream)                                                                                           \
-            k_lin_tv_stream<(L / 4 + 4) / 4, 8><<<dim3(gs, 5 * n), 512, lds_stream, s>>>(                         \
-                c->SV, c->SE, c->sS, c->WL, c->sWl, d, c->TF, c->sTf, c->tv_rt, ids);                            \
+            k_lin_tv_stream<S, 8><<<dim3(gs, 5 * n), 512, lds_stream, s>>>(c->SV, c->SE, c->sS, c->WL, c->sWl,    \
+                                                                          d, c->TF, c->sTf, c->tv_rt, ids);      \
         else                                                                                                     \
-            k_lin_tv_mfma<(L / 4 + 4) / 4><<<g, 256, lds, s>>>(c->SV, c->SE, c->sS, c->WL, c->sWl, d,            \
-                                                               c->TF, c->sTf, c->tv_rt, ids);                   \
+            k_lin_tv_mfma<S><<<g, 256, lds, s>>>(c->SV, c->SE, c->sS, c->WL, c->sWl, d, c->TF, c->sTf,           \
+                                                 c->tv_rt, ids);                                                 \
         break;
-                RPCF_FFT_LENGTHS(RPCF_CASE)
+                RPCF_TV_STEPS(RPCF_CASE)
 #undef RPCF_CASE
-                default: {
-                    dim3 gv((d.P + kTvPencils - 1) / kTvPencils, n);
-                    const size_t lv = sizeof(double2) * 2 * (size_t)d.nz * (kTvPencils + 1);
-                    k_lin_tv<kTvPencils><<<gv, 384, lv, s>>>(c->SV, c->SE, c->sS, c->WL, c->sWl, d, c->T0t,
-                                                             c->T2t, c->T4Q, c->T2Q, c->sQ, ids);
-                }
             }
     };
     if (s == c->stream) return launch(c, KID_LIN_TV, body, cap);
@@ -911,7 +934,7 @@ int autotune_tiles(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     // k_velocity_tile and k_p2s_nl2 run for compiled Chebyshev lengths only
-    const bool tunable[6] = {!c->use_mfma, true, true, true, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
+    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, true, true, true, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
     if (mode == "half") {
         for (int i = 0; i < 6; i++)
             if (tunable[i] && *tile_ref(c, i) >= 2) *tile_ref(c, i) /= 2;
@@ -991,9 +1014,9 @@ void free_ctx(rpcf_ctx* c) {
     if (!c) return;
     if (c->stream) (void)hipStreamSynchronize(c->stream);
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
-    void* ptrs[] = {c->F,   c->SV, c->SE, c->NL,  c->Y,     c->W,  c->Z2, c->WL, c->MINV, c->TF,  c->T4Q,
-                    c->T2Q, c->U,  c->DU, c->DDU, c->MEANU, c->MP, c->PH, c->T0, c->T2,   c->T4,  c->T0t,
-                    c->T2t, c->qw, c->tw, c->ids_dev, c->ids_zero, c->twf, c->MINVH, c->MINVE, c->MINVF, c->PAIRS, c->MT, c->DT};
+    void* ptrs[] = {c->F,   c->SV, c->SE, c->NL,  c->Y,     c->W,  c->Z2, c->WL, c->MINV, c->TF,
+                    c->U,  c->DU, c->DDU, c->MEANU, c->MP, c->PH, c->T0, c->T2,   c->T4,  c->T0t,
+                    c->qw, c->tw, c->ids_dev, c->ids_zero, c->twf, c->MINVH, c->MINVE, c->MINVF, c->PAIRS, c->MT, c->DT};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -1034,7 +1057,7 @@ const MfmaTables& mfma_tables(int N) {
     return g_mt.emplace(N, std::move(t)).first->second;
 }
 
-// Host fragments of the FP64 p2s products of one length 2N, built once per process.
+// Host fragments of the FP64 Chebyshev products of one length 2N, built once per process.
 std::map<int, std::vector<double>> g_dt;
 
 const std::vector<double>& dmfma_tables(int N) {
@@ -1042,7 +1065,12 @@ const std::vector<double>& dmfma_tables(int N) {
     auto it = g_dt.find(N);
     if (it != g_dt.end()) return it->second;
     std::vector<double> t;
-    rpcf_host::p2s_tables_f64(N, t);
+    if (compiled_len(2 * N)) {
+        rpcf_host::p2s_tables_f64(N, t);
+    } else {
+        const cheb_dmfma::NShape s = cheb_dmfma::nshape(N);
+        rpcf_host::cheb_tables_n(N, s.RT, s.KP, s.RQ, s.KE, s.KO, t);
+    }
     return g_dt.emplace(N, std::move(t)).first->second;
 }
 
@@ -1067,17 +1095,16 @@ int init_ctx(rpcf_ctx* c) {
 
     const SlotSizes ss = slot_sizes(d, c->shape.precision);
     c->sF = ss.F; c->sS = ss.S; c->sNL = ss.NL; c->sY = ss.Y; c->sW = ss.W; c->sZ = ss.Z;
-    c->sWl = ss.Wl; c->sM = ss.M; c->sMH = ss.MH; c->sME = ss.ME; c->sTf = ss.Tf; c->sQ = ss.Q; c->sU = ss.U; c->sPz = ss.Pz;
+    c->sWl = ss.Wl; c->sM = ss.M; c->sMH = ss.MH; c->sME = ss.ME; c->sTf = ss.Tf; c->sU = ss.U; c->sPz = ss.Pz;
     c->zld = (d.hnx + 7) & ~7;
     c->tv_rt = (d.N / 2 + 16) / 16;
-    c->tv_s = (d.N / 2 + 4) / 4;
+    c->tv_s = tv_steps((d.N / 2 + 4) / 4);
     if ((rc = dalloc(c, &c->F, C * ss.F)) || (rc = dalloc(c, &c->SV, C * ss.S)) || (rc = dalloc(c, &c->SE, C * ss.S)) ||
         (rc = dalloc(c, &c->NL, C * ss.NL)) || (rc = dalloc(c, &c->Y, C * ss.Y)) || (rc = dalloc(c, &c->W, C * ss.W)) ||
         (rc = dalloc(c, &c->Z2, C * ss.Z)) || (rc = dalloc(c, &c->WL, C * ss.Wl)) ||
         (rc = dalloc(c, &c->MINV, C * ss.M)) || (rc = dalloc(c, &c->MINVH, C * ss.MH)) ||
         (ss.ME && (rc = dalloc(c, &c->MINVE, C * ss.ME))) || (ss.MF && (rc = dalloc(c, &c->MINVF, C * ss.MF))) ||
         (rc = dalloc(c, &c->TF, C * ss.Tf)) ||
-        (rc = dalloc(c, &c->T4Q, C * ss.Q)) || (rc = dalloc(c, &c->T2Q, C * ss.Q)) ||
         (rc = dalloc(c, &c->U, C * ss.U)) || (rc = dalloc(c, &c->DU, C * ss.U)) || (rc = dalloc(c, &c->DDU, C * ss.U)) ||
         (rc = dalloc(c, &c->MEANU, C * ss.Pz)) || (rc = dalloc(c, &c->MP, (size_t)C)) ||
         (rc = dalloc(c, &c->PH, (size_t)C)) || (rc = dalloc(c, &c->ids_dev, (size_t)C)) ||
@@ -1085,7 +1112,7 @@ int init_ctx(rpcf_ctx* c) {
         return rc;
     const size_t nz = d.nz;
     if ((rc = dalloc(c, &c->T0, nz * nz)) || (rc = dalloc(c, &c->T2, nz * nz)) || (rc = dalloc(c, &c->T4, nz * nz)) ||
-        (rc = dalloc(c, &c->T0t, nz * nz)) || (rc = dalloc(c, &c->T2t, nz * nz)) || (rc = dalloc(c, &c->qw, nz)))
+        (rc = dalloc(c, &c->T0t, nz * nz)) || (rc = dalloc(c, &c->qw, nz)))
         return rc;
     if ((rc = dalloc(c, &c->tw, 2 * ((size_t)ct_tw_len(d.mx) + ct_tw_len(d.my) + ct_tw_len(4 * d.N) +
                                        ct_tw_len(2 * d.N)))))
@@ -1125,14 +1152,10 @@ int init_ctx(rpcf_ctx* c) {
     RCCHK(copy_sync(c, c->T2, c->T2h.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
     RCCHK(copy_sync(c, c->T4, c->T4h.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
     {
-        std::vector<double> t0(nz * nz), t2(nz * nz);
+        std::vector<double> t0(nz * nz);
         for (size_t i = 0; i < nz; i++)
-            for (size_t j = 0; j < nz; j++) {
-                t0[j * nz + i] = c->T0h[i * nz + j];
-                t2[j * nz + i] = c->T2h[i * nz + j];
-            }
+            for (size_t j = 0; j < nz; j++) t0[j * nz + i] = c->T0h[i * nz + j];
         RCCHK(copy_sync(c, c->T0t, t0.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
-        RCCHK(copy_sync(c, c->T2t, t2.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
     }
     RCCHK(copy_sync(c, c->qw, c->qw_host.data(), sizeof(double) * nz, hipMemcpyHostToDevice));
 
@@ -1173,18 +1196,20 @@ int init_ctx(rpcf_ctx* c) {
         }
     }
     // FP64 form: the padded p2s + nonlinear combination as FP64 matrix-core products for the
-    // compiled lengths up to 2N = 384; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
-    if (!c->mixed && 2 * d.N <= 384) {
-        bool compiled = false;
-#define RPCF_CASE(L) compiled |= 2 * d.N == L;
-        RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
+    // compiled lengths up to 2N = 384, and both padded Chebyshev transforms for the lengths
+    // without a compiled plan; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
+    if (!c->mixed && (2 * d.N <= 384 || !compiled_len(2 * d.N))) {
         const char* e = getenv("RPCF_P2S_MFMA");
-        if (compiled && !(e && e[0] == '0')) {
+        if (!(e && e[0] == '0')) {
             const std::vector<double>& t = dmfma_tables(d.N);
             if ((rc = dalloc(c, &c->DT, t.size()))) return rc;
             RCCHK(copy_sync(c, c->DT, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
-            c->use_dmfma = 1;
+            if (compiled_len(2 * d.N)) {
+                c->use_dmfma = 1;
+            } else {
+                c->use_dmfma_n = 1;
+                c->dn = cheb_dmfma::nshape(d.N);
+            }
         }
     }
 
@@ -1232,11 +1257,11 @@ int init_ctx(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     c->TK_inv = pick_tile(tk_max, d.my, c->cap_y, lim3, [&](int t) {
-        return sizeof(double2) * ((size_t)t * c->ld_my + (compiled_len(d.my) ? ct_tw_lds_len(d.my) : 0));
+        return sizeof(double2) * ((size_t)t * c->ld_my + tw_lds(d.my));
     });
     c->TK_fwd = c->TK_inv;
     c->RP = pick_tile(rp_max, 6 * d.mx, c->cap_x, lim3, [&](int t) {
-        return sizeof(double2) * (6 * (size_t)t * c->ld_mx + (compiled_len(d.mx) ? ct_tw_lds_len(d.mx) : 0));
+        return sizeof(double2) * (6 * (size_t)t * c->ld_mx + tw_lds(d.mx));
     });
     if (!c->TB_s2p || !c->TB_nl || !c->TK_inv || !c->RP)
         return fail(c, RPCF_EINVAL, "grid too large for the LDS tiles (limit %d bytes)", lim);
@@ -1253,8 +1278,6 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_span_fwd<L>, lim);    \
     allow_lds(k_lamb_phys<L>, lim);   \
     allow_lds(k_p2s_nl<L>, lim);      \
-    allow_lds(k_lin_tv_mfma<(L / 4 + 4) / 4>, lim);      \
-    allow_lds(k_lin_tv_stream<(L / 4 + 4) / 4, 8>, lim); \
     allow_lds(k_cheb_s2p<1, L, float>, lim);              \
     allow_lds(k_span_inv<L, float>, lim);                 \
     allow_lds(k_span_fwd<L, float>, lim);                 \
@@ -1265,6 +1288,7 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_cheb_s2p_h<(L >= 64 ? L : 64), float>, lim); \
     allow_lds(k_p2s_nl2<L, float>, lim);                  \
     allow_lds(k_velocity_tile<L>, lim);                   \
+    allow_lds(k_x_c2r<L>, lim);                           \
     allow_lds(k_velocity_tile<L, float2>, lim);           \
     allow_lds(k_p2s_mfma<(L <= 384 ? L : 384)>, lim);    \
     allow_lds(k_s2p_mfma<(L <= 384 ? L : 384)>, lim);    \
@@ -1272,9 +1296,17 @@ int init_ctx(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     allow_lds(k_cheb_p2s, lim);
-    allow_lds(k_x_c2r, lim);
+    allow_lds(k_x_c2r<0>, lim);
     allow_lds(k_x_r2c, lim);
-    allow_lds(k_lin_tv<kTvPencils>, lim);
+#define RPCF_CASE(S)                 \
+    allow_lds(k_lin_tv_mfma<S>, lim); \
+    allow_lds(k_lin_tv_stream<S, 8>, lim);
+    RPCF_TV_STEPS(RPCF_CASE)
+#undef RPCF_CASE
+    allow_lds(k_s2p_dmfma_n, lim);
+#define RPCF_CASE(RT) allow_lds(k_p2s_dmfma_n<RT>, lim);
+    RPCF_P2S_TILES(RPCF_CASE)
+#undef RPCF_CASE
     (void)hipGetLastError();
     RCCHK(autotune_tiles(c));
     if (getenv("RPCF_VERBOSE"))
@@ -1334,7 +1366,7 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     RCCHK(copy_sync(c, c->MEANU + slot * c->sPz, mU.data(), sizeof(double) * d.pz, hipMemcpyHostToDevice));
     {
         // the quotients T2*0.5/Re*dt and T4*dt*0.5/Re of source/linear.cpp:100, 142 in the
-        // reference's order (transposed), and the five operators of the right-hand sides as
+        // reference's order, and the five operators of the right-hand sides as
         // MFMA A-operand tiles (T0, T2, T4q for v; T0, T2q for eta)
         const double Re = prm->Re, dt = prm->dt;
         std::vector<double> t0(nz * nz), t2(nz * nz), q4(nz * nz), q2(nz * nz);
@@ -1345,8 +1377,6 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
                 q2[j * nz + i] = c->T2h[i * nz + j] * 0.5 / Re * dt;
                 q4[j * nz + i] = c->T4h[i * nz + j] * dt * 0.5 / Re;
             }
-        RCCHK(copy_sync(c, c->T4Q + slot * c->sQ, q4.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
-        RCCHK(copy_sync(c, c->T2Q + slot * c->sQ, q2.data(), sizeof(double) * nz * nz, hipMemcpyHostToDevice));
         const int RT = c->tv_rt, S = c->tv_s;
         const std::vector<double>* ops[5] = {&t0, &t2, &q4, &t0, &q2};  // op[j*nz + i] = T[i][j]
         std::vector<double> tf((size_t)c->sTf, 0.0);
@@ -1695,26 +1725,54 @@ __global__ __launch_bounds__(256) void k_gather_pencils(const double2* __restric
     }
 }
 
-// The backward transform of one field on the context's stream: Chebyshev s2p (pencils f,
+// The backward transform of one field on the context's stream, by the kernels of a step where
+// they have a plan of the length (41 us against 70 with runtime plans for a padded 64x65x64 field,
+// launches and the wait included): Chebyshev s2p (pencils f,
 // nz contiguous) -> planes y -> span C2C -> planes w -> x C2R -> ph; y and w are the
 // caller's intermediates of hnx*planes*ny and planes*my*nxh complex values.
 int enq_spec_to_phys(rpcf_ctx* c, const double2* f, double2* y, double2* w, double* ph, int padded) {
     const Dims d = c->d;
     const int planes = padded ? d.pz : d.nz;
     const FftPlan& plz = c->pl_zn;
-    const int L = 2 * d.N, ld = L + 1;
-    const int TB = pick_tile(16, L, c->cap_zn, c->lds_limit, [&](int t) { return sizeof(double2) * (size_t)t * ld; });
-    const int RP1 = pick_tile(8, d.mx, c->cap_x, c->lds_limit, [&](int t) { return sizeof(double2) * (size_t)t * c->ld_mx; });
     const double2* tw4 = (const double2*)c->pl_zp.tw;
+    // the kernels of a step on one field (blockIdx.z = 0)
+    const int TB = c->TB_s2p, ld = c->ld_zn;
     dim3 g((d.ny + TB - 1) / TB, d.hnx, 1);
     const size_t lds = sizeof(double2) * TB * ld;
-    if (padded) k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
-    else k_cheb_s2p<0><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
-    dim3 g2((d.nxh + c->TK_inv - 1) / c->TK_inv, planes, 1);
-    k_span_inv<0><<<g2, kFftThreads, sizeof(double2) * c->TK_inv * c->ld_my, c->stream>>>(
-        y, 0, 0, w, 0, 0, d, planes, c->pl_y, c->TK_inv, c->ld_my, c->ids_zero);
+    switch (2 * d.N) {
+#define RPCF_CASE(L)                                                                                                \
+    case L:                                                                                                         \
+        if (!padded)                                                                                                \
+            k_cheb_s2p<0, L><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero); \
+        else if constexpr (L >= 64)                                                                                 \
+            k_cheb_s2p_h<(L >= 64 ? L : 64)><<<g, kFftThreads, sizeof(double2) * s2p_h_lds(L, TB), c->stream>>>(     \
+                f, 0, 0, y, 0, 0, d, tw4, TB, c->ids_zero);                                                         \
+        else                                                                                                        \
+            k_cheb_s2p<1, L><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero); \
+        break;
+        RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+        default:
+            if (padded && c->use_dmfma_n)
+                k_s2p_dmfma_n<<<dim3((d.ny + cheb_dmfma::kPencils - 1) / cheb_dmfma::kPencils, d.hnx, 1), 256,
+                                cheb_dmfma::s2p_n_lds(c->dn), c->stream>>>(f, 0, 0, y, 0, 0, d, c->DT, c->dn, c->ids_zero);
+            else if (padded)
+                k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
+            else
+                k_cheb_s2p<0><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
+    }
+    span_inv<double>(c, 1, y, 0, 0, w, 0, 0, planes, c->pl_y, c->ids_zero);
+    const int RP1 = pick_tile(kC2rRows, d.mx, c->cap_x, c->lds_limit / 3, [&](int t) {
+        return sizeof(double2) * ((size_t)t * c->ld_mx + tw_lds(d.mx));
+    });
     dim3 g3((d.my / 2 + RP1 - 1) / RP1, planes);
-    k_x_c2r<<<g3, kFftThreads, sizeof(double2) * RP1 * c->ld_mx, c->stream>>>(w, ph, d, c->pl_x, RP1, c->ld_mx);
+    const size_t lds3 = sizeof(double2) * (RP1 * c->ld_mx + tw_lds(d.mx));
+    switch (d.mx) {
+#define RPCF_CASE(L) case L: k_x_c2r<L><<<g3, kFftThreads, lds3, c->stream>>>(w, ph, d, c->pl_x, RP1, c->ld_mx); break;
+        RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+        default: k_x_c2r<<<g3, kFftThreads, lds3, c->stream>>>(w, ph, d, c->pl_x, RP1, c->ld_mx);
+    }
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? RPCF_OK : fail(c, RPCF_EDEVICE, "spec_to_phys launch: %s", hipGetErrorString(e));
 }
@@ -1757,9 +1815,7 @@ int rpcf_phys_to_spec(rpcf_ctx* c, const double* phys, double* spec, long stride
         dim3 g3((d.my / 2 + RP1 - 1) / RP1, planes);
         k_x_r2c<<<g3, kFftThreads, sizeof(double2) * RP1 * c->ld_mx, c->stream>>>(ph, z, d.hnx, c->fac, d, c->pl_x, RP1,
                                                                                   c->ld_mx);
-        dim3 g2((d.hnx + c->TK_fwd - 1) / c->TK_fwd, planes, 1);
-        k_span_fwd<0><<<g2, kFftThreads, sizeof(double2) * c->TK_fwd * c->ld_my, c->stream>>>(
-            z, 0, 0, d.hnx, y, 0, 0, d, planes, c->pl_y, c->TK_fwd, c->ld_my, c->ids_zero);
+        span_fwd<double>(c, 1, z, 0, 0, d.hnx, y, 0, 0, planes, c->pl_y, c->ids_zero, nullptr);
         dim3 g((d.ny + TB - 1) / TB, d.hnx);
         k_cheb_p2s<<<g, kFftThreads, sizeof(double2) * TB * ld, c->stream>>>(y, f, d, planes, plz, TB, ld);
         hipError_t e = hipGetLastError();
@@ -2051,8 +2107,6 @@ int rpcf_member_adopt(rpcf_ctx* c, int slot, rpcf_ctx* src, int src_slot) {
     cp(c->MINVE, src->MINVE, c->sME);
     cp(c->MINVF, src->MINVF, c->MINVF ? c->sME : 0);
     cp(c->TF, src->TF, c->sTf);
-    cp(c->T4Q, src->T4Q, c->sQ);
-    cp(c->T2Q, src->T2Q, c->sQ);
     cp(c->U, src->U, c->sU);
     cp(c->DU, src->DU, c->sU);
     cp(c->DDU, src->DDU, c->sU);

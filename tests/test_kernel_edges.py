@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 import rpcf
+from helpers import rel
 
 pytestmark = pytest.mark.gpu
 
@@ -43,3 +44,29 @@ def test_state_crosses_the_boundary_unchanged(grid, pad):
         assert sim.dll.rpcf_get_state(sim.h, ptr[0], ptr[1], nz + pad) == 0
         assert np.array_equal(out[0, :, :nz], a) and np.array_equal(out[1, :, :nz], b)
         assert (out[:, :, nz:] == 7.0 + 1j).all()
+
+
+# lengths without a compiled plan: N odd and even, row tiles of the Chebyshev products whole,
+# one row over and partial (N/2 + 1 = 8 .. 126 rows), the largest N; ragged pencil tiles; x and
+# span lengths with radices 2 to 8, 3 and 5.  The library's bars: 1e-12 after one step, 1e-13
+# for a transform of one field.
+@pytest.mark.parametrize("N,mx,my", [(15, 30, 20), (25, 36, 54), (27, 20, 30), (30, 54, 24), (36, 50, 36), (45, 24, 90),
+                                     (50, 40, 60), (75, 72, 18), (81, 48, 20), (125, 12, 30), (160, 18, 24),
+                                     (225, 12, 12), (243, 10, 12), (250, 12, 10)])
+def test_lengths_without_compiled_plans(N, mx, my):
+    channel = N % 2 == 0
+    prm = rpcf.make_params(mx, my, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=900.0, Ro=0.1, dt=0.002,
+                           u_profile=(1.0, 0.0, -1.0) if channel else (0.0, 1.0, 0.0), flow_control=int(channel))
+    g, o = pair(prm)
+    v, e = rpcf.seed_state(g.dll, prm, 5, 0.1, 3, 8, 0.5)
+    for s in (g, o):
+        s.set_state(v, e)
+        s.nonlinear()
+    assert rel(g.get_nonlinear()[1], o.get_nonlinear()[1]) < 1e-12
+    for s in (g, o):
+        s.step(1)
+    for a, b in zip(g.get_state(), o.get_state()):
+        assert rel(a, b) < 1e-12
+    for padded in (True, False):
+        assert rel(g.spec_to_phys(v, padded), o.spec_to_phys(v, padded)) < 1e-13
+    g.close(), o.close()
