@@ -356,10 +356,10 @@ __global__ __launch_bounds__(cheb_dmfma::DShape<FN>::NT, 3) void k_p2s_dmfma(
 // kind of FP64 matrix products with N a run-time number.  The runtime-plan FFT kernels they
 // replace (k_cheb_s2p<1, 0>, k_p2s_nl<0>; RPCF_P2S_MFMA=0 keeps them) run 3 to 5 passes over
 // LDS with index arithmetic by run-time strides: at 40x46x60 (N = 45) 72 and 62 us against
-// 11.5 and 10.9 here, at 100x151x100 (N = 150, where the product's N^2 meets the FFT's N log N)
-// 352 and 281 against 182 and 70.  Bound by the latency of a block's phases on small grids, by
-// the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.3 and
-// 0.4 of 72 TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
+// 10.5 and 10.3 here, at 100x151x100 (N = 150, where the product's N^2 meets the FFT's N log N)
+// 352 and 281 against 145 and 70.  Bound by the latency of a block's phases on small grids, by
+// the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.2 and
+// 0.3 of 72 TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
 // -------------------------------------------------------------------------------------
 namespace cheb_dmfma {
 
@@ -381,8 +381,8 @@ inline NShape nshape(int N) {
     s.NCH = ceil_div(N + 1, kNChunk);
     s.KP = s.NCH * (kNChunk / 4);
     s.RQ = ceil_div(N + 1, 16);
-    s.KE = ceil_div(N / 2 + 1, 4);
-    s.KO = ceil_div((N + 1) / 2, 4);
+    s.KE = 2 * ceil_div(N / 2 + 1, 8);  // pairs of k-steps
+    s.KO = 2 * ceil_div((N + 1) / 2, 8);
     s.s2p_off = 4L * s.RT * s.KP * 64;
     s.doubles = s.s2p_off + (long)s.RQ * (s.KE + s.KO) * 64;
     return s;
@@ -537,6 +537,7 @@ __global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restr
 // The pencils' coefficients lie in LDS as B operands; a wave takes row tiles q of the even and
 // odd products (fragments from L2), rows q and 2N - q are their sum and difference, stored from
 // the accumulators: 16 pencils of a row are 256 contiguous bytes.
+template <int = 0>
 __global__ __launch_bounds__(256) void k_s2p_dmfma_n(const double2* __restrict__ F, long fstride, long sF,
                                                      double2* __restrict__ Y, long ystride, long sY, Dims d,
                                                      const double* __restrict__ tab, cheb_dmfma::NShape sh,
@@ -565,20 +566,23 @@ __global__ __launch_bounds__(256) void k_s2p_dmfma_n(const double2* __restrict__
         const double* te = tab + sh.s2p_off + (long)rt * (KE + KO) * 64 + lane;
         const double* to = te + (long)KE * 64;
         v4d e[2] = {zero4, zero4}, o[2] = {zero4, zero4};
-#pragma unroll 4
-        for (int s = 0; s < KE; s++) {
-            const double a = te[(long)s * 64];
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++)
-                e[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, lds[(4 * s + kq) * kS2pLd + ct * kPencils + lc], e[ct], 0, 0, 0);
-        }
-#pragma unroll 4
-        for (int s = 0; s < KO; s++) {
-            const double a = to[(long)s * 64];
-#pragma unroll
-            for (int ct = 0; ct < 2; ct++)
-                o[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(a, lds[(rows + 4 * s + kq) * kS2pLd + ct * kPencils + lc], o[ct], 0, 0, 0);
-        }
+        // two k-steps at a time, the next two fragments in flight
+        auto product = [&](const double* t, int par, int ks, v4d* acc) {
+            double a0 = t[0], a1 = t[64];
+            for (int s = 0; s < ks; s += 2) {
+                const long nx = 64L * min(s + 2, ks - 2);
+                const double n0 = t[nx], n1 = t[nx + 64];
+                const double* b = lds + (par * rows + 4 * s + kq) * kS2pLd + lc;
+                const double b00 = b[0], b01 = b[kPencils], b10 = b[4 * kS2pLd], b11 = b[4 * kS2pLd + kPencils];
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b00, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b01, acc[1], 0, 0, 0);
+                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b10, acc[0], 0, 0, 0);
+                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b11, acc[1], 0, 0, 0);
+                a0 = n0, a1 = n1;
+            }
+        };
+        product(te, 0, KE, e);
+        product(to, 1, KO, o);
         if (lc < nb) {
 #pragma unroll
             for (int r = 0; r < 4; r++) {

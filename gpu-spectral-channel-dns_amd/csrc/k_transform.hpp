@@ -556,6 +556,7 @@ __global__ __launch_bounds__(256) void k_x_c2r(const double2* __restrict__ W, do
 }
 
 // x R2C of one field: phys[q][s][mx] -> Z2[q][s][hnx] with 1/(mx my) (rpcf_phys_to_spec).
+template <int = 0>
 __global__ __launch_bounds__(256) void k_x_r2c(const double* __restrict__ phys, double2* __restrict__ Z2, int zld, double fac, Dims d,
                         FftPlan pl, int RP, int ld) {
     RPCF_LDS(double2);
@@ -657,6 +658,7 @@ __device__ __forceinline__ void load_p2s(double2* lds, int ld, const double2* Z1
 
 // Chebyshev physical -> spectral of one field (rpcf_phys_to_spec): cheby_p2s
 // (source/transform.cu:538-658, post-processing 513-536).  Z1[kx][q][ky] -> F[p][k<nz].
+template <int = 0>
 __global__ __launch_bounds__(256) void k_cheb_p2s(const double2* __restrict__ Z1, double2* __restrict__ F, Dims d, int planes, FftPlan pl,
                            int TB, int ld) {
     RPCF_LDS(double2);

@@ -25,10 +25,12 @@
 #include "../../include/rpcf_group.h"
 #include "../../include/rpcf_static.h"
 #include "host_prep.hpp"
+#include "instances.hpp"
 #include "k_linear.hpp"
-#include "k_transform.hpp"
-#include "k_cheb_mfma.hpp"
-#include "k_cheb_dmfma.hpp"
+
+#define RPCF_CASE(L) RPCF_INSTANCES(extern, L)
+RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
 
 // Static device scratch of the entry points that allocate nothing (include/rpcf_static.h):
 // each GPU holds its own copy, RPCF_STATIC_SCRATCH_BYTES, until the process ends.
@@ -1295,15 +1297,15 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384)>, lim);
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-    allow_lds(k_cheb_p2s, lim);
+    allow_lds(k_cheb_p2s<0>, lim);
     allow_lds(k_x_c2r<0>, lim);
-    allow_lds(k_x_r2c, lim);
+    allow_lds(k_x_r2c<0>, lim);
 #define RPCF_CASE(S)                 \
     allow_lds(k_lin_tv_mfma<S>, lim); \
     allow_lds(k_lin_tv_stream<S, 8>, lim);
     RPCF_TV_STEPS(RPCF_CASE)
 #undef RPCF_CASE
-    allow_lds(k_s2p_dmfma_n, lim);
+    allow_lds(k_s2p_dmfma_n<0>, lim);
 #define RPCF_CASE(RT) allow_lds(k_p2s_dmfma_n<RT>, lim);
     RPCF_P2S_TILES(RPCF_CASE)
 #undef RPCF_CASE
