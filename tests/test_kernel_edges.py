@@ -70,3 +70,33 @@ def test_lengths_without_compiled_plans(N, mx, my):
     for padded in (True, False):
         assert rel(g.spec_to_phys(v, padded), o.spec_to_phys(v, padded)) < 1e-13
     g.close(), o.close()
+
+
+# solves of an odd base profile by conjugate parity blocks, at N odd and even, the smallest pair
+# counts, row pairs that fill whole and partial batches of every column group, the largest N: the
+# full inverses' results after one step.  2e-13 is the bound of the even profiles' blocks with
+# remainders (2^-9 of the 1e-11 the blocks alone leave).  Without stored remainders the same values are formed from the full inverses.
+@pytest.mark.parametrize("N", [4, 5, 6, 12, 27, 48, 64, 75, 96, 125, 128, 160, 250])
+@pytest.mark.parametrize("precision", [0, 2])
+def test_odd_profile_solves(N, precision, monkeypatch):
+    def step(p, full):
+        monkeypatch.setenv("RPCF_FULL_INVERSE", str(int(full)))
+        prm = rpcf.make_params(24, 24, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=1300.0, Ro=0.1, dt=0.002,
+                               u_profile=(0.0, 1.0, 0.0), precision=p)
+        with rpcf.Simulation(rpcf.HIP_LIB, prm) as s:
+            if N < 12:  # no room for a seed that satisfies the wall conditions
+                rng = np.random.default_rng(N)
+                shape = s.s["P"], s.s["nz"]
+                s.set_state(*(rng.standard_normal(shape) + 1j * rng.standard_normal(shape) for _ in range(2)))
+            else:
+                s.set_state(*rpcf.seed_state(s.dll, prm, 0, 0.1, 4, min(24, N - 5), 5.0 / 6.0, True))
+            s.bootstrap()
+            return s.get_state()
+
+    a, f = step(precision, False), step(precision, True)
+    e = max(rel(x, y) for x, y in zip(a, f))
+    print("N=%d precision %d: blocks vs full inverses %.2e" % (N, precision, e))
+    assert e < 2e-13
+    if precision == 2:
+        b = step(0, False)
+        assert all(np.array_equal(x, y) for x, y in zip(a, b))
