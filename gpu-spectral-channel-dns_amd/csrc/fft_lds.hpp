@@ -143,7 +143,7 @@ template <int DIR, typename C> struct Dft<8, DIR, C> {
     }
 };
 
-// cos(2 pi m / N), sin(2 pi m / N) for the composite radices (N = 12, 16)
+// cos(2 pi m / N), sin(2 pi m / N) for the composite radices (N = 12, 16, 24)
 template <int N> struct TwTab;
 template <> struct TwTab<16> {
     static constexpr double c[16] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173,
@@ -154,6 +154,20 @@ template <> struct TwTab<16> {
                                      1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173,
                                      0.0, -0.38268343236508977173, -0.70710678118654752440, -0.92387953251128675613,
                                      -1.0, -0.92387953251128675613, -0.70710678118654752440, -0.38268343236508977173};
+};
+template <> struct TwTab<24> {
+    static constexpr double c[24] = {1.0, 0.96592582628906828675, 0.86602540378443864676, 0.70710678118654752440,
+                                     0.5, 0.25881904510252076235, 0.0, -0.25881904510252076235,
+                                     -0.5, -0.70710678118654752440, -0.86602540378443864676, -0.96592582628906828675,
+                                     -1.0, -0.96592582628906828675, -0.86602540378443864676, -0.70710678118654752440,
+                                     -0.5, -0.25881904510252076235, 0.0, 0.25881904510252076235,
+                                     0.5, 0.70710678118654752440, 0.86602540378443864676, 0.96592582628906828675};
+    static constexpr double s[24] = {0.0, 0.25881904510252076235, 0.5, 0.70710678118654752440,
+                                     0.86602540378443864676, 0.96592582628906828675, 1.0, 0.96592582628906828675,
+                                     0.86602540378443864676, 0.70710678118654752440, 0.5, 0.25881904510252076235,
+                                     0.0, -0.25881904510252076235, -0.5, -0.70710678118654752440,
+                                     -0.86602540378443864676, -0.96592582628906828675, -1.0, -0.96592582628906828675,
+                                     -0.86602540378443864676, -0.70710678118654752440, -0.5, -0.25881904510252076235};
 };
 template <> struct TwTab<12> {
     static constexpr double c[12] = {1.0, 0.86602540378443864676, 0.5, 0.0, -0.5, -0.86602540378443864676,
@@ -196,6 +210,7 @@ template <int R1, int R2, int DIR, typename C> struct DftComposite {
 };
 template <int DIR, typename C> struct Dft<16, DIR, C> : DftComposite<4, 4, DIR, C> {};
 template <int DIR, typename C> struct Dft<12, DIR, C> : DftComposite<4, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<24, DIR, C> : DftComposite<8, 3, DIR, C> {};
 
 // i / d for a run-time divisor by its reciprocal: exact for i < 2^22 (the quotient's error,
 // i/d 2^-23, stays below the 0.5/d that i + 0.5 keeps from the next integer).  The integer
@@ -416,6 +431,64 @@ __device__ __forceinline__ void fft_ct(C* buf, int ld, int B, const C* tw, int t
         constexpr bool TW1 = TWO && S == 1 && ct2_nst(N) >= 2;  // stage 1 from the [r-1][k] table
         fft_stage_ct<R, DIR, N, NS, BT, C, S == 0 ? Q : 0, S == 1 ? Q : 0, TW1, T1OFF>(buf, ld, B, tw, tid, nthr);
         fft_ct<N, DIR, BT, TWO, C, T1OFF, S + 1, NS * R>(buf, ld, B, tw, tid, nthr);
+    }
+}
+
+// A two-pass transform from and to global memory: TK sequences (columns) by one block, whose
+// threads hold at most one butterfly of either pass (tp_threads).  The first pass reads its
+// inputs straight into registers (load(b, j, o): element j + o of column b, o a constant once
+// unrolled), the second hands its outputs to store(b, j, o, x), so the columns cross LDS once --
+// written by the first pass, read by the second after the one barrier -- instead of six or more
+// times (fill, a read and a write per stage, read-back).  COLS_FIRST: neighbouring threads of the
+// first pass take neighbouring columns and those of the second neighbouring elements (input
+// contiguous over columns, output over elements), else the other way round.  tw: the plan's n
+// twiddles, read from cache.  The radix-24 first pass of 384 replaces three stages (16, 12, 2).
+constexpr int tp_rad(int n, int s) {
+    const int a = n == 24 || n == 32 || n == 96 ? 8 : n == 384 ? 24 : 16;
+    return s == 0 ? a : n / a;
+}
+constexpr bool tp_has(int n) { return n >= 24 && n <= 384; }  // of the compiled lengths; 512 needs three passes
+constexpr int tp_threads(int n, int tk) {
+    const int a = tk * tp_rad(n, 1), b = tk * tp_rad(n, 0);
+    return ((a > b ? a : b) + 63) / 64 * 64;
+}
+template <int N, int DIR, int TK, bool COLS_FIRST, typename C, typename Load, typename Store>
+__device__ __forceinline__ void fft_two_pass(C* lds, const C* __restrict__ tw, int tid, Load load, Store store) {
+    constexpr unsigned RA = tp_rad(N, 0), RB = tp_rad(N, 1), ld = N + 1;
+    // the LDS swizzle between the passes (24 = 3 mod 8 spreads the butterflies over all eight)
+    constexpr int Q = RA == 24 ? 8 : RA;
+    static_assert(RA * RB == N, "two passes");
+    {
+        const unsigned t = tid;
+        if (t < TK * RB) {
+            const unsigned b = COLS_FIRST ? t % TK : t / RB, j = COLS_FIRST ? t / TK : t % RB;
+            C v[RA];
+#pragma unroll
+            for (unsigned r = 0; r < RA; r++) v[r] = load(b, j, r * RB);
+            Dft<RA, DIR, C>::run(v);
+            C* col = lds + b * ld;
+#pragma unroll
+            for (unsigned r = 0; r < RA; r++) col[swz<Q>(j * RA + r)] = v[r];
+        }
+    }
+    __syncthreads();
+    const unsigned t = tid;
+    if (t < TK * RA) {
+        const unsigned b = COLS_FIRST ? t / RA : t % TK, k = COLS_FIRST ? t % RA : t / TK;
+        const C* col = lds + b * ld;
+        C v[RB];
+#pragma unroll
+        for (unsigned r = 0; r < RB; r++) {
+            v[r] = col[swz<Q>(k + r * RA)];
+            if (r > 0) {
+                C w = tw[r * k];
+                if (DIR > 0) w.y = -w.y;
+                v[r] = cmul(v[r], w);
+            }
+        }
+        Dft<RB, DIR, C>::run(v);
+#pragma unroll
+        for (unsigned r = 0; r < RB; r++) store(b, k, r * RA, v[r]);
     }
 }
 

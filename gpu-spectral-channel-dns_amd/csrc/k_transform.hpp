@@ -34,6 +34,18 @@ constexpr int kC2rRows = 8;    // pairs of span rows per block of k_x_c2r
 // ... and their bounds for a compiled transform length: shorter rows and columns take wider
 // tiles, so that a block keeps about the work and LDS it has at length 192.
 constexpr int span_tile_max(int fn) { return fn >= 192 || fn == 0 ? kSpanTile : 2 * kSpanTile; }
+// The span transforms of the compiled lengths in FP64 go through fft_two_pass, with whole
+// 128-byte lines (8 columns) or two of W and Z2 rows per block, three to six blocks per CU.  At
+// length 384 tiles of 7 columns (what three blocks' LDS took) and three stages in LDS gave
+// k_span_inv 579 us and k_span_fwd 188 at 256x97x256; this gives 311 (the time a copy of their
+// 1.52 GB takes) and 143; at 64x65x64 20.3 and 14.1 -> 15.3 and 11.4, at 32x33x32 9.0 and 9.1 ->
+// 7.6 and 6.7, at 128x129x128, where both were at the copy rate, 99.6 and 56 -> 96.6 and 55.  The
+// mixed form keeps its FP32 kernels: another order of FP32 roundings is as far off as FP32 itself.
+template <typename R> constexpr bool span_two_pass(int fn) { return sizeof(R) == 8 && tp_has(fn); }
+constexpr int span2_tile(int fn) { return fn >= 256 ? 8 : 16; }
+template <typename R> constexpr int span_threads(int fn) {
+    return span_two_pass<R>(fn) ? tp_threads(fn, span2_tile(fn)) : kFftBlock;
+}
 constexpr int lamb_pairs_max(int fn) { return fn >= 192 || fn == 0 ? kLambPairs : fn >= 96 ? 2 * kLambPairs : 4 * kLambPairs; }
 
 template <int V> struct IntC { static constexpr int value = V; };
@@ -330,7 +342,7 @@ __global__ __launch_bounds__(256) void k_cheb_s2p_h(const double2* __restrict__ 
 // plane.  Y[f][kx][q][ky] -> W[f][q][s][kx] for kx < nxh (the x-Nyquist column is zero).
 // -------------------------------------------------------------------------------------
 template <int FN = 0, typename R = double>  // R: precision of Y, W and the FFT
-__global__ __launch_bounds__(256) void k_span_inv(const cplx<R>* __restrict__ Y, long ystride, long sY, cplx<R>* __restrict__ W,
+__global__ __launch_bounds__(span_threads<R>(FN)) void k_span_inv(const cplx<R>* __restrict__ Y, long ystride, long sY, cplx<R>* __restrict__ W,
                                                   long wstride, long sW, Dims d, int planes, FftPlan pl, int TK, int ld,
                                                   const int* __restrict__ ids) {
     using C2 = cplx<R>;
@@ -340,6 +352,23 @@ __global__ __launch_bounds__(256) void k_span_inv(const cplx<R>* __restrict__ Y,
     Y += slot * sY;
     W += slot * sW;
     const int nk_rt = min(TK, d.nxh - kx0);
+    if constexpr (span_two_pass<R>(FN)) {
+        constexpr unsigned NY = FN / 3 * 2, B = tp_rad(FN, 1);
+        const C2* in = Y + f * ystride + q * NY + (long)kx0 * planes * NY;
+        C2* out = W + f * wstride + (long)q * FN * d.nxh + kx0;
+        fft_two_pass<FN, +1, span2_tile(FN), false>(
+            lds, (const C2*)pl.tw, threadIdx.x,
+            [&](unsigned b, unsigned j, unsigned o) {
+                // element s = j + o, j < B: pencil s or s - (my - ny), or none (ky_of_span)
+                if (o >= NY / 2 && o + B - 1 <= FN - NY / 2) return cmake<C2>(0, 0);
+                const int ky = o + B - 1 < NY / 2 ? j + o : o > FN - NY / 2 ? j + o - (FN - NY) : ky_of_span(d, j + o);
+                return ky >= 0 && (int)b < nk_rt ? in[b * planes * NY + ky] : cmake<C2>(0, 0);
+            },
+            [&](unsigned b, unsigned j, unsigned o, C2 v) {
+                if ((int)b < nk_rt) out[(j + o) * d.nxh + b] = v;
+            });
+        return;
+    }
     // a full tile of a compiled length: constant tile width, length and LDS stride (my + 1);
     // offsets inside a slot's field fit 32 bits
     auto body = [&](auto nkc) {
@@ -588,7 +617,7 @@ __global__ __launch_bounds__(256) void k_x_r2c(const double* __restrict__ phys, 
 // member * 3 + component.
 // -------------------------------------------------------------------------------------
 template <int FN = 0, typename R = double>  // R: precision of Z2, Z1 and the FFT
-__global__ __launch_bounds__(256) void k_span_fwd(const cplx<R>* __restrict__ Z2, long zstride, long sZ, int zld,
+__global__ __launch_bounds__(span_threads<R>(FN)) void k_span_fwd(const cplx<R>* __restrict__ Z2, long zstride, long sZ, int zld,
                                                   cplx<R>* __restrict__ Z1, long ostride, long sY, Dims d, int planes,
                                                   FftPlan pl, int TK, int ld, const int* __restrict__ ids,
                                                   int* __restrict__ phase = nullptr) {
@@ -603,6 +632,24 @@ __global__ __launch_bounds__(256) void k_span_fwd(const cplx<R>* __restrict__ Z2
     Z2 += slot * sZ;
     Z1 += slot * sY;
     const int nk_rt = min(TK, d.hnx - kx0);
+    if constexpr (span_two_pass<R>(FN)) {
+        constexpr unsigned NY = FN / 3 * 2, A = tp_rad(FN, 0);
+        const C2* in = Z2 + g * zstride + (long)q * FN * zld + kx0;
+        C2* out = Z1 + g * ostride + q * NY + (long)kx0 * planes * NY;
+        fft_two_pass<FN, -1, span2_tile(FN), true>(
+            lds, (const C2*)pl.tw, threadIdx.x,
+            [&](unsigned b, unsigned j, unsigned o) {
+                return (int)b < nk_rt ? in[(j + o) * zld + b] : cmake<C2>(0, 0);
+            },
+            [&](unsigned b, unsigned j, unsigned o, C2 v) {
+                // element s = j + o, j < A: pencil s <= ny/2 or s - (my - ny) > ny/2 (span_of)
+                if (o > NY / 2 && o + A - 1 <= FN - NY + NY / 2) return;
+                const unsigned s = j + o;
+                if ((int)b < nk_rt && (s <= NY / 2 || s > FN - NY + NY / 2))
+                    out[b * planes * NY + (s <= NY / 2 ? s : s - (FN - NY))] = v;
+            });
+        return;
+    }
     // a full tile of a compiled length: constant tile width, length and LDS stride (my + 1);
     // offsets inside a slot's field fit 32 bits
     auto body = [&](auto nkc) {

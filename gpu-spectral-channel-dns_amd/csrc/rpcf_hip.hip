@@ -581,11 +581,12 @@ template <typename R>
 void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* W, long wS, long sW, int planes,
               const FftPlan& pl, const int* ids) {
     const Dims d = c->d;
-    const int TK = c->TK_inv, ld = c->ld_my;
+    const bool two = compiled_len(d.my) && span_two_pass<R>(d.my);  // a tile of its own
+    const int TK = two ? span2_tile(d.my) : c->TK_inv, ld = c->ld_my;
     dim3 g((d.nxh + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (TK * ld + tw_lds(d.my));
+    const size_t lds = sizeof(cplx<R>) * (TK * ld + (two ? 0 : tw_lds(d.my)));
     switch (d.my) {
-#define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
+#define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
         default:
@@ -598,11 +599,12 @@ template <typename R>
 void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld, cplx<R>* Y, long yS, long sY, int planes,
               const FftPlan& pl, const int* ids, int* phase) {
     const Dims d = c->d;
-    const int TK = c->TK_fwd, ld = c->ld_my;
+    const bool two = compiled_len(d.my) && span_two_pass<R>(d.my);
+    const int TK = two ? span2_tile(d.my) : c->TK_fwd, ld = c->ld_my;
     dim3 g((d.hnx + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (TK * ld + tw_lds(d.my));
+    const size_t lds = sizeof(cplx<R>) * (TK * ld + (two ? 0 : tw_lds(d.my)));
     switch (d.my) {
-#define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
+#define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
         default:
@@ -936,7 +938,8 @@ int autotune_tiles(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     // k_velocity_tile and k_p2s_nl2 run for compiled Chebyshev lengths only
-    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, true, true, true, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
+    const bool span = c->mixed || !(compiled_len(d.my) && span_two_pass<double>(d.my));
+    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, span, span, true, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
     if (mode == "half") {
         for (int i = 0; i < 6; i++)
             if (tunable[i] && *tile_ref(c, i) >= 2) *tile_ref(c, i) /= 2;

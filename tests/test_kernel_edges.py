@@ -72,6 +72,21 @@ def test_lengths_without_compiled_plans(N, mx, my):
     g.close(), o.close()
 
 
+# span transforms of every compiled length: tiles of 8 and 16 columns whole, partial and of one
+# column (nx/2 = 3 .. 18 columns in, nx/2 + 1 out), every butterfly's zeroed and dropped rows
+@pytest.mark.parametrize("my", [24, 32, 48, 64, 96, 128, 192, 256, 384, 512])
+@pytest.mark.parametrize("mx", [10, 24, 50, 54])
+def test_span_transforms(my, mx):
+    g, o = pair(rpcf.make_params(mx, my, 40, n_pi_x=2.0, n_pi_y=1.0))
+    rng = np.random.default_rng(my + mx)
+    a = rng.standard_normal((g.s["P"], g.s["nz"])) + 1j * rng.standard_normal((g.s["P"], g.s["nz"]))
+    p, q = g.spec_to_phys(a), o.spec_to_phys(a)
+    assert rel(p, q) < 1e-13
+    f = rng.standard_normal(q.shape)
+    assert rel(g.phys_to_spec(f), o.phys_to_spec(f)) < 1e-13
+    g.close(), o.close()
+
+
 # solves of an odd base profile by conjugate parity blocks, at N odd and even, the smallest pair
 # counts, row pairs that fill whole and partial batches of every column group, the largest N: the
 # full inverses' results after one step.  2e-13 is the bound of the even profiles' blocks with
