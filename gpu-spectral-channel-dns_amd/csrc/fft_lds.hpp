@@ -143,8 +143,36 @@ template <int DIR, typename C> struct Dft<8, DIR, C> {
     }
 };
 
-// cos(2 pi m / N), sin(2 pi m / N) for the composite radices (N = 12, 16, 24)
-template <int N> struct TwTab;
+// cos(2 pi m / N), sin(2 pi m / N) for the composite radices: by their Taylor series within an
+// eighth of the circle, in long double, rounded once
+constexpr long double ct_sin_series(long double x) {
+    long double t = x, s = x;
+    for (int k = 1; k < 14; k++) t *= -x * x / ((2 * k) * (2 * k + 1)), s += t;
+    return s;
+}
+constexpr long double ct_cos_series(long double x) {
+    long double t = 1, s = 1;
+    for (int k = 1; k < 14; k++) t *= -x * x / ((2 * k - 1) * (2 * k)), s += t;
+    return s;
+}
+constexpr double ct_cos2pi(int m, int n) {  // 0 <= m < n
+    if (2 * m > n) m = n - m;
+    if (4 * m > n) return -ct_cos2pi(n - 2 * m, 2 * n);  // cos(pi - x), x = pi - 2 pi m / n
+    constexpr long double pi = 3.141592653589793238462643383279502884L;
+    return (double)(8 * m <= n ? ct_cos_series(2 * pi * m / n) : ct_sin_series(pi * (n - 4 * m) / (2 * n)));
+}
+constexpr double ct_sin2pi(int m, int n) {  // cos(2 pi (m/n - 1/4))
+    return ct_cos2pi((4 * m + 3 * n) % (4 * n), 4 * n);
+}
+template <int N> struct TwTab {
+    struct Row { double v[N]; constexpr double operator[](int m) const { return v[m]; } };
+    static constexpr Row make(bool sine) {
+        Row r{};
+        for (int m = 0; m < N; m++) r.v[m] = sine ? ct_sin2pi(m, N) : ct_cos2pi(m, N);
+        return r;
+    }
+    static constexpr Row c = make(false), s = make(true);
+};
 template <> struct TwTab<16> {
     static constexpr double c[16] = {1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173,
                                      0.0, -0.38268343236508977173, -0.70710678118654752440, -0.92387953251128675613,
@@ -154,20 +182,6 @@ template <> struct TwTab<16> {
                                      1.0, 0.92387953251128675613, 0.70710678118654752440, 0.38268343236508977173,
                                      0.0, -0.38268343236508977173, -0.70710678118654752440, -0.92387953251128675613,
                                      -1.0, -0.92387953251128675613, -0.70710678118654752440, -0.38268343236508977173};
-};
-template <> struct TwTab<24> {
-    static constexpr double c[24] = {1.0, 0.96592582628906828675, 0.86602540378443864676, 0.70710678118654752440,
-                                     0.5, 0.25881904510252076235, 0.0, -0.25881904510252076235,
-                                     -0.5, -0.70710678118654752440, -0.86602540378443864676, -0.96592582628906828675,
-                                     -1.0, -0.96592582628906828675, -0.86602540378443864676, -0.70710678118654752440,
-                                     -0.5, -0.25881904510252076235, 0.0, 0.25881904510252076235,
-                                     0.5, 0.70710678118654752440, 0.86602540378443864676, 0.96592582628906828675};
-    static constexpr double s[24] = {0.0, 0.25881904510252076235, 0.5, 0.70710678118654752440,
-                                     0.86602540378443864676, 0.96592582628906828675, 1.0, 0.96592582628906828675,
-                                     0.86602540378443864676, 0.70710678118654752440, 0.5, 0.25881904510252076235,
-                                     0.0, -0.25881904510252076235, -0.5, -0.70710678118654752440,
-                                     -0.86602540378443864676, -0.96592582628906828675, -1.0, -0.96592582628906828675,
-                                     -0.86602540378443864676, -0.70710678118654752440, -0.5, -0.25881904510252076235};
 };
 template <> struct TwTab<12> {
     static constexpr double c[12] = {1.0, 0.86602540378443864676, 0.5, 0.0, -0.5, -0.86602540378443864676,
@@ -210,14 +224,21 @@ template <int R1, int R2, int DIR, typename C> struct DftComposite {
 };
 template <int DIR, typename C> struct Dft<16, DIR, C> : DftComposite<4, 4, DIR, C> {};
 template <int DIR, typename C> struct Dft<12, DIR, C> : DftComposite<4, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<6, DIR, C> : DftComposite<3, 2, DIR, C> {};
+template <int DIR, typename C> struct Dft<9, DIR, C> : DftComposite<3, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<10, DIR, C> : DftComposite<5, 2, DIR, C> {};
+template <int DIR, typename C> struct Dft<15, DIR, C> : DftComposite<5, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<18, DIR, C> : DftComposite<6, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<20, DIR, C> : DftComposite<5, 4, DIR, C> {};
 template <int DIR, typename C> struct Dft<24, DIR, C> : DftComposite<8, 3, DIR, C> {};
+template <int DIR, typename C> struct Dft<25, DIR, C> : DftComposite<5, 5, DIR, C> {};
 
 // i / d for a run-time divisor by its reciprocal: exact for i < 2^22 (the quotient's error,
 // i/d 2^-23, stays below the 0.5/d that i + 0.5 keeps from the next integer).  The integer
 // division it replaces in the runtime plans and ragged tiles is some 30 instructions an index;
-// with it, and the runtime plans' twiddles read from LDS, k_lamb_phys, k_span_inv and k_span_fwd
-// take 33, 24 and 16 us at 40x46x60 (50, 33 and 19 before) and 242, 178 and 82 at 100x151x100
-// (390, 222 and 104).
+// with it, and the runtime plans' twiddles read from LDS, lengths that then had no compiled plan
+// took 33, 24 and 16 us in k_lamb_phys, k_span_inv and k_span_fwd at 40x46x60 (50, 33 and 19 with
+// divisions) and 242, 178 and 82 at 100x151x100 (390, 222 and 104).
 struct FastDiv {
     unsigned d;
     float inv;
@@ -434,62 +455,110 @@ __device__ __forceinline__ void fft_ct(C* buf, int ld, int B, const C* tw, int t
     }
 }
 
-// A two-pass transform from and to global memory: TK sequences (columns) by one block, whose
-// threads hold at most one butterfly of either pass (tp_threads).  The first pass reads its
-// inputs straight into registers (load(b, j, o): element j + o of column b, o a constant once
-// unrolled), the second hands its outputs to store(b, j, o, x), so the columns cross LDS once --
-// written by the first pass, read by the second after the one barrier -- instead of six or more
-// times (fill, a read and a write per stage, read-back).  COLS_FIRST: neighbouring threads of the
-// first pass take neighbouring columns and those of the second neighbouring elements (input
-// contiguous over columns, output over elements), else the other way round.  tw: the plan's n
-// twiddles, read from cache.  The radix-24 first pass of 384 replaces three stages (16, 12, 2).
+// ---- two-pass transforms (FP64) ---------------------------------------------------------
+// Lengths n = RA RB with radices of 2 to 25: butterflies of RA points, one exchange through
+// LDS, butterflies of RB points.  RA is the smallest radix >= sqrt(n).
+constexpr bool tp_radix(int r) {
+    for (int q : {2, 3, 4, 5, 6, 8, 9, 10, 12, 15, 16, 18, 20, 24, 25})
+        if (q == r) return true;
+    return false;
+}
 constexpr int tp_rad(int n, int s) {
-    const int a = n == 24 || n == 32 || n == 96 ? 8 : n == 384 ? 24 : 16;
-    return s == 0 ? a : n / a;
+    for (int a = 2; a <= 25; a++)
+        if (a * a >= n && n % a == 0 && tp_radix(a) && tp_radix(n / a)) return s == 0 ? a : n / a;
+    return 0;
 }
-constexpr bool tp_has(int n) { return n >= 24 && n <= 384; }  // of the compiled lengths; 512 needs three passes
-constexpr int tp_threads(int n, int tk) {
-    const int a = tk * tp_rad(n, 1), b = tk * tp_rad(n, 0);
-    return ((a > b ? a : b) + 63) / 64 * 64;
-}
-template <int N, int DIR, int TK, bool COLS_FIRST, typename C, typename Load, typename Store>
-__device__ __forceinline__ void fft_two_pass(C* lds, const C* __restrict__ tw, int tid, Load load, Store store) {
-    constexpr unsigned RA = tp_rad(N, 0), RB = tp_rad(N, 1), ld = N + 1;
-    // the LDS swizzle between the passes (24 = 3 mod 8 spreads the butterflies over all eight)
-    constexpr int Q = RA == 24 ? 8 : RA;
-    static_assert(RA * RB == N, "two passes");
-    {
-        const unsigned t = tid;
-        if (t < TK * RB) {
-            const unsigned b = COLS_FIRST ? t % TK : t / RB, j = COLS_FIRST ? t / TK : t % RB;
-            C v[RA];
+constexpr bool tp_has(int n) { return n >= 24 && n % 2 == 0 && tp_rad(n, 0) > 0; }
+// a column between the passes: RB groups of RA entries, one entry of padding behind a group where
+// RA is even, so that the strides of either pass are odd (no bank conflicts) and every butterfly's
+// addresses are constants away from its first
+constexpr int tp_pitch(int n) { return tp_rad(n, 0) | 1; }
+constexpr int tp_ld(int n) { return (tp_rad(n, 1) * tp_pitch(n)) | 1; }
+constexpr int tp_threads(int n, int seqs) { return (seqs * tp_rad(n, 0) + 63) / 64 * 64; }
+
+// pass B: input r of butterfly k times w^(k r), tw[m] = exp(-2 pi i m/N)
+template <int N, int DIR, typename C>
+__device__ __forceinline__ void tp_pass_b(const C* col, unsigned k, const C* __restrict__ tw, C* v) {
+    constexpr unsigned RB = tp_rad(N, 1), P = tp_pitch(N);
 #pragma unroll
-            for (unsigned r = 0; r < RA; r++) v[r] = load(b, j, r * RB);
-            Dft<RA, DIR, C>::run(v);
-            C* col = lds + b * ld;
-#pragma unroll
-            for (unsigned r = 0; r < RA; r++) col[swz<Q>(j * RA + r)] = v[r];
+    for (unsigned r = 0; r < RB; r++) {
+        v[r] = col[k + r * P];
+        if (r > 0) {
+            C w = tw[r * k];
+            if (DIR > 0) w.y = -w.y;
+            v[r] = cmul(v[r], w);
         }
     }
-    __syncthreads();
+    Dft<RB, DIR, C>::run(v);
+}
+
+// From and to global memory: TK sequences (columns) by one block, whose tp_threads(N, TK) threads
+// hold at most one butterfly of either pass.  The first pass reads its inputs straight into
+// registers (load(b, j, o): element j + o of column b, o a constant once unrolled), the second
+// hands its outputs to store(b, j, o, x), so the columns cross LDS once -- written by the first
+// pass, read by the second after the one barrier -- instead of six or more times (fill, a read and
+// a write per stage, read-back).  COLS_FIRST: neighbouring threads of the first pass take
+// neighbouring columns and those of the second neighbouring elements (input contiguous over
+// columns, output over elements), else the other way round.  tw: the plan's n twiddles, read from
+// cache.
+template <int N, int DIR, int TK, bool COLS_FIRST, typename C, typename Load, typename Store>
+__device__ __forceinline__ void fft_two_pass(C* lds, const C* __restrict__ tw, int tid, Load load, Store store) {
+    constexpr unsigned RA = tp_rad(N, 0), RB = tp_rad(N, 1), ld = tp_ld(N);
     const unsigned t = tid;
+    if (t < TK * RB) {
+        const unsigned b = COLS_FIRST ? t % TK : t / RB, j = COLS_FIRST ? t / TK : t % RB;
+        C v[RA];
+#pragma unroll
+        for (unsigned r = 0; r < RA; r++) v[r] = load(b, j, r * RB);
+        Dft<RA, DIR, C>::run(v);
+        C* col = lds + b * ld + j * tp_pitch(N);
+#pragma unroll
+        for (unsigned r = 0; r < RA; r++) col[r] = v[r];
+    }
+    __syncthreads();
     if (t < TK * RA) {
         const unsigned b = COLS_FIRST ? t / RA : t % TK, k = COLS_FIRST ? t % RA : t / TK;
-        const C* col = lds + b * ld;
         C v[RB];
-#pragma unroll
-        for (unsigned r = 0; r < RB; r++) {
-            v[r] = col[swz<Q>(k + r * RA)];
-            if (r > 0) {
-                C w = tw[r * k];
-                if (DIR > 0) w.y = -w.y;
-                v[r] = cmul(v[r], w);
-            }
-        }
-        Dft<RB, DIR, C>::run(v);
+        tp_pass_b<N, DIR>(lds + b * ld, k, tw, v);
 #pragma unroll
         for (unsigned r = 0; r < RB; r++) store(b, k, r * RA, v[r]);
     }
+}
+
+// S sequences of ld entries in LDS (natural order): pass A reads element j + o by load(seq, j, o),
+// the result goes back in natural order by store(seq, k, o, x).  dst: where the exchange happens;
+// with dst == src the passes are separated by barriers, else (disjoint) only the exchange is.
+// The block has at least tp_threads(N, S) threads, and all of them call it.
+template <int N, int DIR, typename C, typename Load, typename Store>
+__device__ __forceinline__ void tp_in_lds(C* dst, bool in_place, int S, const C* __restrict__ tw, int tid, Load load,
+                                          Store store) {
+    constexpr unsigned RA = tp_rad(N, 0), RB = tp_rad(N, 1), ld = tp_ld(N);
+    const unsigned t = tid;
+    {
+        const unsigned b = t / RB, j = t % RB;
+        C v[RA];
+        if (t < S * RB) {
+#pragma unroll
+            for (unsigned r = 0; r < RA; r++) v[r] = load(b, j, r * RB);
+            Dft<RA, DIR, C>::run(v);
+        }
+        if (in_place) __syncthreads();
+        if (t < S * RB) {
+            C* col = dst + b * ld + j * tp_pitch(N);
+#pragma unroll
+            for (unsigned r = 0; r < RA; r++) col[r] = v[r];
+        }
+    }
+    __syncthreads();
+    const unsigned b = t / RA, k = t % RA;
+    C v[RB];
+    if (t < S * RA) tp_pass_b<N, DIR>(dst + b * ld, k, tw, v);
+    if (in_place) __syncthreads();
+    if (t < S * RA) {
+#pragma unroll
+        for (unsigned r = 0; r < RB; r++) store(b, k, r * RA, v[r]);
+    }
+    __syncthreads();
 }
 
 // Twiddles of a plan copied into LDS by the kernels that read them there: a compiled plan's own
@@ -515,3 +584,8 @@ __device__ __forceinline__ void fft_any(C* buf, int ld, int B, const FftPlan& pl
 
 // lengths with compiled plans (every grid of the benchmark, ensemble and serving sets)
 #define RPCF_FFT_LENGTHS(X) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
+// the further lengths whose x and span transforms are compiled, in FP64 (two passes): with the
+// ones above (but 512) every even 2^a 3^b 5^c of 24 .. 384
+#define RPCF_XY_LENGTHS(X) \
+    X(30) X(36) X(40) X(50) X(54) X(60) X(72) X(80) X(90) X(100) X(108) X(120) X(144) X(150) X(160) X(162) X(180) \
+    X(200) X(216) X(240) X(250) X(270) X(288) X(300) X(320) X(324) X(360)

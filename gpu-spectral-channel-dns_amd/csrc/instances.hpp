@@ -6,7 +6,7 @@
 #include "k_cheb_mfma.hpp"
 #include "k_transform.hpp"
 
-// x and span transforms, precision R
+// x and span transforms, precision R (all that an RPCF_XY_LENGTHS length has, in FP64)
 #define RPCF_INSTANCES_XY(EXT, L, R)                                                                                  \
     EXT template __global__ void k_span_inv<L, R>(const cplx<R>*, long, long, cplx<R>*, long, long, Dims, int, FftPlan, \
                                                   int, int, const int*);                                               \

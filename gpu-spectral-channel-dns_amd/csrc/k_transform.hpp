@@ -34,17 +34,31 @@ constexpr int kC2rRows = 8;    // pairs of span rows per block of k_x_c2r
 // ... and their bounds for a compiled transform length: shorter rows and columns take wider
 // tiles, so that a block keeps about the work and LDS it has at length 192.
 constexpr int span_tile_max(int fn) { return fn >= 192 || fn == 0 ? kSpanTile : 2 * kSpanTile; }
-// The span transforms of the compiled lengths in FP64 go through fft_two_pass, with whole
-// 128-byte lines (8 columns) or two of W and Z2 rows per block, three to six blocks per CU.  At
-// length 384 tiles of 7 columns (what three blocks' LDS took) and three stages in LDS gave
-// k_span_inv 579 us and k_span_fwd 188 at 256x97x256; this gives 311 (the time a copy of their
-// 1.52 GB takes) and 143; at 64x65x64 20.3 and 14.1 -> 15.3 and 11.4, at 32x33x32 9.0 and 9.1 ->
-// 7.6 and 6.7, at 128x129x128, where both were at the copy rate, 99.6 and 56 -> 96.6 and 55.  The
-// mixed form keeps its FP32 kernels: another order of FP32 roundings is as far off as FP32 itself.
-template <typename R> constexpr bool span_two_pass(int fn) { return sizeof(R) == 8 && tp_has(fn); }
-constexpr int span2_tile(int fn) { return fn >= 256 ? 8 : 16; }
+// The x and span transforms of the even lengths 24 .. 384 in FP64 take two passes (fft_two_pass,
+// lamb_two_pass).  Span: whole 128-byte lines (8 columns) or two of W and Z2 rows per block, three
+// to six blocks per CU.  At length 384 tiles of 7 columns (what three blocks' LDS took) and three
+// stages in LDS gave k_span_inv 579 us and k_span_fwd 188 at 256x97x256; this gives 309 (the time
+// a copy of its 1.52 GB takes) and 146; at 64x65x64 20.3 and 14.1 -> 14.5 and 10.8, at 32x33x32
+// 9.0 and 9.1 -> 7.1 and 6.5, at 128x129x128, where both were at the copy rate, 99.6 and 56 ->
+// 97 and 54.  At 40x46x60, whose lengths 60 and 90 had run-time plans of four and five stages,
+// 25.8 and 18.0 -> 10.1 and 8.4.  The mixed form keeps its FP32 kernels: another order of FP32
+// roundings is as far off as FP32 itself.
+template <typename R> constexpr bool two_pass(int fn) { return sizeof(R) == 8 && tp_has(fn) && fn <= 384; }
+constexpr int span2_tile(int fn) { return 16 * tp_ld(fn) * 16 <= 54000 ? 16 : 8; }
 template <typename R> constexpr int span_threads(int fn) {
-    return span_two_pass<R>(fn) ? tp_threads(fn, span2_tile(fn)) : kFftBlock;
+    return two_pass<R>(fn) ? tp_threads(fn, span2_tile(fn)) : kFftBlock;
+}
+// row pairs per block of the two-pass k_lamb_phys: at most 20 KB of sequences, eight blocks per CU
+// (one pair where it takes more).  A block's phases are short and its barriers many, so more and
+// smaller blocks hide each other's loads: 40 KB give 136 us at 128x129x128 and 23.4 at 64x65x64,
+// 20 KB 129 and 21.9, 12 KB 129 and 23.7.
+constexpr int lamb2_pairs(int fn) {
+    int p = 8;
+    while (p > 1 && 6 * p * tp_ld(fn) * 16 > 20480) p /= 2;
+    return p;
+}
+template <typename R> constexpr int lamb_threads(int fn) {
+    return two_pass<R>(fn) ? tp_threads(fn, 6 * lamb2_pairs(fn)) : kFftBlock;
 }
 constexpr int lamb_pairs_max(int fn) { return fn >= 192 || fn == 0 ? kLambPairs : fn >= 96 ? 2 * kLambPairs : 4 * kLambPairs; }
 
@@ -352,7 +366,7 @@ __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_inv(const cplx<R>*
     Y += slot * sY;
     W += slot * sW;
     const int nk_rt = min(TK, d.nxh - kx0);
-    if constexpr (span_two_pass<R>(FN)) {
+    if constexpr (two_pass<R>(FN)) {
         constexpr unsigned NY = FN / 3 * 2, B = tp_rad(FN, 1);
         const C2* in = Y + f * ystride + q * NY + (long)kx0 * planes * NY;
         C2* out = W + f * wstride + (long)q * FN * d.nxh + kx0;
@@ -437,6 +451,93 @@ __device__ __forceinline__ void r2c_unpack(const C* z, int k, int mx, decltype(C
     *xb = cmake<C>((zk.y + zm.y) * h * fac, -(zk.x - zm.x) * h * fac);
 }
 
+// k_lamb_phys for the two-pass lengths (FP64).  Bound by the latency of its phases (load, two
+// passes in LDS, products, two passes, store): 419 us at 256x97x256 where the bytes take 285 at the
+// copy rate, 129 (97) at 128x129x128, 21.9 at 64x65x64, 13.9 at 40x46x60, 8.4 at 32x33x32; the
+// staged kernel below took 547, 138, 26.0, 35.1 (run-time plan) and 10.1.  Loading the first pass's
+// inputs straight into registers, as the span transforms do, costs each coefficient twice and
+// serialises on its conditions: 648 us at 256x97x256.
+// nrp <= lamb2_pairs(mx) row pairs from W, Z2 (the first row
+// of the first field).  Sequences [6][RP][tp_ld] in LDS, component g's forward transform exchanged
+// through the room of field 3 + g.
+template <int FN>
+__device__ __forceinline__ void lamb_two_pass(double2* lds, const double2* W, long ws, double2* Z2, long zs, int zld,
+                                              double Ro, double mU, double fac, const double2* __restrict__ tw, int nrp) {
+    constexpr int RP = lamb2_pairs(FN), nthr = lamb_threads<double>(FN), ld = tp_ld(FN);
+    constexpr int nxh = FN / 3, hnx = nxh + 1;
+    const int tid = threadIdx.x;
+    // each kept coefficient pair (A_k, B_k), k < nxh, gives Z_k and Z_{mx-k} of Z = X_A + i X_B
+    constexpr int KL = (6 * RP * nxh + nthr - 1) / nthr > 4 ? 4 : (6 * RP * nxh + nthr - 1) / nthr;
+    for (int base = tid; base < 6 * RP * nxh; base += KL * nthr) {
+        double2 va[KL], vb[KL];
+#pragma unroll
+        for (int u = 0; u < KL; u++) {
+            const int i = base + u * nthr, seq = (unsigned)i / nxh, k = i - seq * nxh;
+            const int f = (unsigned)seq / RP, ip = seq - f * RP;
+            if (i < 6 * RP * nxh && ip < nrp) {
+                const double2* rA = W + f * ws + 2 * ip * nxh;
+                va[u] = rA[k];
+                vb[u] = rA[nxh + k];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < KL; u++) {
+            const int i = base + u * nthr, seq = (unsigned)i / nxh, k = i - seq * nxh;
+            const int f = (unsigned)seq / RP, ip = seq - f * RP;
+            if (i < 6 * RP * nxh && ip < nrp) {
+                double2 a = va[u], b = vb[u];
+                double2* z = lds + seq * ld;
+                if (k == 0) {
+                    a.y = 0;
+                    b.y = 0;
+                } else {
+                    z[FN - k] = make_double2(a.x + b.y, -a.y + b.x);
+                }
+                z[k] = make_double2(a.x - b.y, a.y + b.x);
+            }
+        }
+    }
+    __syncthreads();
+    constexpr unsigned RA = tp_rad(FN, 0), RB = tp_rad(FN, 1);
+    tp_in_lds<FN, +1>(
+        lds, true, 6 * RP, tw, tid,
+        [&](unsigned b, unsigned j, unsigned o) {
+            // Z_k = 0 for nxh <= k <= mx - nxh
+            if (o >= nxh && o + RB - 1 <= FN - nxh) return make_double2(0.0, 0.0);
+            const double2 z = lds[b * ld + j + o];
+            return o + RB - 1 < nxh || o > FN - nxh || j + o < nxh || j + o > FN - nxh ? z : make_double2(0.0, 0.0);
+        },
+        [&](unsigned b, unsigned k, unsigned o, double2 v) { lds[b * ld + k + o] = v; });
+    for (int i = tid; i < RP * FN; i += nthr) {
+        const int ip = (unsigned)i / FN, x = i - ip * FN;
+        double2* p = lds + ip * ld + x;
+        constexpr int fs = RP * ld;
+        const double2 u = p[0], v = p[fs], w = p[2 * fs], ox = p[3 * fs], oy = p[4 * fs], oz = p[5 * fs];
+        p[0] = make_double2(oz.x * v.x - oy.x * w.x - Ro * w.x, oz.y * v.y - oy.y * w.y - Ro * w.y);
+        p[fs] = make_double2(ox.x * w.x - oz.x * u.x, ox.y * w.y - oz.y * u.y);
+        p[2 * fs] = make_double2(oy.x * u.x - ox.x * v.x + Ro * (u.x + mU), oy.y * u.y - ox.y * v.y + Ro * (u.y + mU));
+    }
+    __syncthreads();
+    double2* ex = lds + 3 * RP * ld;
+    tp_in_lds<FN, -1>(
+        ex, false, 3 * RP, tw, tid, [&](unsigned b, unsigned j, unsigned o) { return lds[b * ld + j + o]; },
+        [&](unsigned b, unsigned k, unsigned o, double2 v) {
+            // the rows' spectra take k <= nxh and mx - k
+            if (o > nxh && o + RA - 1 < FN - nxh) return;
+            lds[b * ld + k + o] = v;
+        });
+    for (int i = tid; i < 3 * RP * hnx; i += nthr) {
+        const int seq = (unsigned)i / hnx, k = i - seq * hnx;
+        const int g = (unsigned)seq / RP, ip = seq - g * RP;
+        if (ip >= nrp) continue;
+        double2 xa, xb;
+        r2c_unpack(lds + seq * ld, k, FN, fac, &xa, &xb);
+        double2* o = Z2 + g * zs + 2 * ip * zld;
+        o[k] = xa;
+        o[zld + k] = xb;
+    }
+}
+
 // -------------------------------------------------------------------------------------
 // Fused physical-space stage: x C2R of the six fields, Lamb vector + Coriolis term
 // (computeLambDevice, source/nonlinear.cu:409-428, base flow at padded point q as in
@@ -447,7 +548,7 @@ __device__ __forceinline__ void r2c_unpack(const C* z, int k, int mx, decltype(C
 // then (compiled lengths) the FN twiddles.
 // -------------------------------------------------------------------------------------
 template <int FN = 0, typename R = double>  // R: precision of W, Z2, the FFTs and the products
-__global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W, long wstride, long sW,
+__global__ __launch_bounds__(lamb_threads<R>(FN)) void k_lamb_phys(const cplx<R>* __restrict__ W, long wstride, long sW,
                                                    cplx<R>* __restrict__ Z2, long zstride, long sZ, int zld,
                                                    const double* __restrict__ meanU, long sPz, double fac, Dims d,
                                                    FftPlan pl, int RP, int ld, Members mb) {
@@ -460,6 +561,12 @@ __global__ __launch_bounds__(256) void k_lamb_phys(const cplx<R>* __restrict__ W
     Z2 += slot * sZ;
     meanU += slot * sPz;
     const int nrp_rt = min(RP, d.my / 2 - rp0);
+    if constexpr (two_pass<R>(FN)) {
+        lamb_two_pass<FN>(lds, W + ((long)q * d.my + 2 * rp0) * (FN / 3), wstride,
+                          Z2 + ((long)q * d.my + 2 * rp0) * zld, zstride, zld, Ro, meanU[q], fac,
+                          (const double2*)pl.tw, nrp_rt);
+        return;
+    }
     // The compiled lengths fix mx, nxh = (mx/3*2)/2, hnx = nxh + 1 and the LDS stride
     // mx + 1; a full tile fixes nrp = lamb_pairs_max(mx) -- the index arithmetic then reduces to
     // constant multiplies and shifts.  Offsets inside a slot fit 32 bits.
@@ -632,7 +739,7 @@ __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_fwd(const cplx<R>*
     Z2 += slot * sZ;
     Z1 += slot * sY;
     const int nk_rt = min(TK, d.hnx - kx0);
-    if constexpr (span_two_pass<R>(FN)) {
+    if constexpr (two_pass<R>(FN)) {
         constexpr unsigned NY = FN / 3 * 2, A = tp_rad(FN, 0);
         const C2* in = Z2 + g * zstride + (long)q * FN * zld + kx0;
         C2* out = Z1 + g * ostride + q * NY + (long)kx0 * planes * NY;

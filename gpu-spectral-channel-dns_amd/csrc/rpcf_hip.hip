@@ -31,6 +31,9 @@
 #define RPCF_CASE(L) RPCF_INSTANCES(extern, L)
 RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
+#define RPCF_CASE(L) RPCF_INSTANCES_XY(extern, L, double)
+RPCF_XY_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
 
 // Static device scratch of the entry points that allocate nothing (include/rpcf_static.h):
 // each GPU holds its own copy, RPCF_STATIC_SCRATCH_BYTES, until the process ends.
@@ -581,17 +584,20 @@ template <typename R>
 void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* W, long wS, long sW, int planes,
               const FftPlan& pl, const int* ids) {
     const Dims d = c->d;
-    const bool two = compiled_len(d.my) && span_two_pass<R>(d.my);  // a tile of its own
+    const bool two = two_pass<R>(d.my);  // a tile of its own
     const int TK = two ? span2_tile(d.my) : c->TK_inv, ld = c->ld_my;
     dim3 g((d.nxh + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (TK * ld + (two ? 0 : tw_lds(d.my)));
+    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + tw_lds(d.my));
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
         default:
             if constexpr (sizeof(R) == 8)
-                k_span_inv<<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids);
+                switch (d.my) {
+                    RPCF_XY_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+                    default: k_span_inv<<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids);
+                }
     }
 }
 
@@ -599,17 +605,20 @@ template <typename R>
 void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld, cplx<R>* Y, long yS, long sY, int planes,
               const FftPlan& pl, const int* ids, int* phase) {
     const Dims d = c->d;
-    const bool two = compiled_len(d.my) && span_two_pass<R>(d.my);
+    const bool two = two_pass<R>(d.my);
     const int TK = two ? span2_tile(d.my) : c->TK_fwd, ld = c->ld_my;
     dim3 g((d.hnx + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (TK * ld + (two ? 0 : tw_lds(d.my)));
+    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + tw_lds(d.my));
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
         default:
             if constexpr (sizeof(R) == 8)
-                k_span_fwd<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase);
+                switch (d.my) {
+                    RPCF_XY_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+                    default: k_span_fwd<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase);
+                }
     }
 }
 
@@ -694,21 +703,26 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
     rc = launch(c, KID_SPAN_INV, [&] { span_inv<R>(c, 6 * n, Y, yS, c->sY, W, wS, c->sW, d.pz, ply, ids); }, cap);
     if (rc) return rc;
     {
-        const int RP = c->RP, ld = c->ld_mx;
+        const bool two = two_pass<R>(d.mx);
+        const int RP = two ? lamb2_pairs(d.mx) : c->RP, ld = c->ld_mx;
         dim3 g((d.my / 2 + RP - 1) / RP, d.pz, n);
-        size_t lds = sizeof(C2) * (6 * RP * ld + tw_lds(d.mx));
+        const size_t lds = sizeof(C2) * (two ? 6 * RP * tp_ld(d.mx) : 6 * RP * ld + tw_lds(d.mx));
         rc = launch(
             c, KID_LAMB,
             [&] {
                 switch (d.mx) {
-#define RPCF_CASE(L) case L: k_lamb_phys<L, R><<<g, kFftThreads, lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld, c->MEANU, c->sPz, c->fac, d, plx, RP, ld, mb); break;
+#define RPCF_CASE(L) case L: k_lamb_phys<L, R><<<g, lamb_threads<R>(L), lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld, c->MEANU, c->sPz, c->fac, d, plx, RP, ld, mb); break;
                     RPCF_FFT_LENGTHS(RPCF_CASE)
-#undef RPCF_CASE
                     default:
                         if constexpr (f64)
-                            k_lamb_phys<<<g, kFftThreads, lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld,
-                                                                            c->MEANU, c->sPz, c->fac, d, plx, RP, ld,
-                                                                            mb);
+                            switch (d.mx) {
+                                RPCF_XY_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+                                default:
+                                    k_lamb_phys<<<g, kFftThreads, lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld,
+                                                                                    c->MEANU, c->sPz, c->fac, d, plx,
+                                                                                    RP, ld, mb);
+                            }
                 }
             },
             cap);
@@ -938,8 +952,8 @@ int autotune_tiles(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     // k_velocity_tile and k_p2s_nl2 run for compiled Chebyshev lengths only
-    const bool span = c->mixed || !(compiled_len(d.my) && span_two_pass<double>(d.my));
-    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, span, span, true, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
+    const bool span = c->mixed || !two_pass<double>(d.my), lamb = c->mixed || !two_pass<double>(d.mx);
+    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, span, span, lamb, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
     if (mode == "half") {
         for (int i = 0; i < 6; i++)
             if (tunable[i] && *tile_ref(c, i) >= 2) *tile_ref(c, i) /= 2;
@@ -1299,6 +1313,12 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_s2p_mfma<(L <= 384 ? L : 384)>, lim);    \
     allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384)>, lim);
     RPCF_FFT_LENGTHS(RPCF_CASE)
+#undef RPCF_CASE
+#define RPCF_CASE(L)               \
+    allow_lds(k_span_inv<L>, lim); \
+    allow_lds(k_span_fwd<L>, lim); \
+    allow_lds(k_lamb_phys<L>, lim);
+    RPCF_XY_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     allow_lds(k_cheb_p2s<0>, lim);
     allow_lds(k_x_c2r<0>, lim);

@@ -72,18 +72,42 @@ def test_lengths_without_compiled_plans(N, mx, my):
     g.close(), o.close()
 
 
-# span transforms of every compiled length: tiles of 8 and 16 columns whole, partial and of one
-# column (nx/2 = 3 .. 18 columns in, nx/2 + 1 out), every butterfly's zeroed and dropped rows
-@pytest.mark.parametrize("my", [24, 32, 48, 64, 96, 128, 192, 256, 384, 512])
-@pytest.mark.parametrize("mx", [10, 24, 50, 54])
-def test_span_transforms(my, mx):
-    g, o = pair(rpcf.make_params(mx, my, 40, n_pi_x=2.0, n_pi_y=1.0))
-    rng = np.random.default_rng(my + mx)
+XY_LENGTHS = [24, 30, 32, 36, 40, 48, 50, 54, 60, 64, 72, 80, 90, 96, 100, 108, 120, 128, 144, 150, 160, 162, 180, 192,
+              200, 216, 240, 250, 256, 270, 288, 300, 320, 324, 360, 384, 400, 512]
+
+
+# span transforms of every compiled length and one longer than them: tiles of 8 and 16 columns
+# whole, partial and of one column (nx/2 = 3 .. 18 columns in, nx/2 + 1 out), every butterfly's
+# zeroed and dropped rows
+@pytest.mark.parametrize("my", XY_LENGTHS)
+def test_span_transforms(my):
+    g, o = pair(rpcf.make_params((10, 24, 50, 54)[XY_LENGTHS.index(my) % 4], my, 40, n_pi_x=2.0, n_pi_y=1.0))
+    rng = np.random.default_rng(my)
     a = rng.standard_normal((g.s["P"], g.s["nz"])) + 1j * rng.standard_normal((g.s["P"], g.s["nz"]))
     p, q = g.spec_to_phys(a), o.spec_to_phys(a)
     assert rel(p, q) < 1e-13
     f = rng.standard_normal(q.shape)
     assert rel(g.phys_to_spec(f), o.phys_to_spec(f)) < 1e-13
+    g.close(), o.close()
+
+
+# the x transforms and products of every compiled length: whole and partial tiles of row pairs
+# (5, 12 and 27 pairs).  The library's bar for N after one evaluation.  (512 is refused for mx.)
+@pytest.mark.parametrize("mx", XY_LENGTHS[:-1])
+def test_lamb_vector(mx):
+    prm = rpcf.make_params(mx, (10, 24, 54)[XY_LENGTHS.index(mx) % 3], 40, n_pi_x=2.0, n_pi_y=1.0, Re=900.0, Ro=0.1,
+                           dt=0.002)
+    g, o = pair(prm)
+    rng = np.random.default_rng(mx)
+    shape = g.s["P"], g.s["nz"]
+    f = [(rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / (1.0 + np.arange(g.s["nz"])) ** 2
+         for _ in range(6)]
+    for s in (g, o):
+        for i in range(6):
+            s.set_field(i, f[i])
+        s.nonlinear()
+    for a, b in zip(g.get_nonlinear(), o.get_nonlinear()):
+        assert rel(a, b) < 1e-12
     g.close(), o.close()
 
 
