@@ -266,11 +266,9 @@ inline void p2s_tables_f64(int N, std::vector<double>& out) {
     for (int p = 0; p < ra; p++) out.push_back((double)f.q1a[(size_t)p * (N + 1) + N]);
 }
 
-// FP64 fragments of the Chebyshev products of lengths without a compiled plan
-// (k_p2s_dmfma_n, k_s2p_dmfma_n): the folded p2s tables Q0s, Q0a, Q1s, Q1a as rt row tiles x
-// kp k-steps each, zero past their sizes; then per s2p row tile the even and odd products,
-// E[q][j] = cos(pi 2j q/(2N)) and O[q][j] = cos(pi (2j+1) q/(2N)), q <= N
-inline void cheb_tables_n(int N, int rt, int kp, int rq, int ke, int ko, std::vector<double>& out) {
+// FP64 fragments of the p2s products of lengths without a compiled plan (k_p2s_dmfma_n): the
+// folded tables Q0s, Q0a, Q1s, Q1a as rt row tiles x kp k-steps each, zero past their sizes
+inline void p2s_tables_n(int N, int rt, int kp, std::vector<double>& out) {
     const P2sFolded f = p2s_folded(N);
     const int rs = N / 2 + 1, ra = (N + 1) / 2;
     auto padded = [&](const std::vector<long double>& T, int rows, int cols) {
@@ -283,15 +281,28 @@ inline void cheb_tables_n(int N, int rt, int kp, int rq, int ke, int ko, std::ve
     padded(f.q0a, ra, N);
     padded(f.q1s, rs, N);
     padded(f.q1a, ra, N + 1);
-    for (int t = 0; t < rq; t++)
-        for (int par = 0; par < 2; par++) {
-            const int ks = par ? ko : ke, cols = (N + 2 - par) / 2;
-            std::vector<long double> e((size_t)16 * 4 * ks, 0.0L);
-            for (int r = 0; r < 16 && 16 * t + r <= N; r++)
-                for (int j = 0; j < cols; j++)
-                    e[(size_t)r * 4 * ks + j] = cospi_ratio((long)(2 * j + par) * (16 * t + r), 2L * N);
-            dmfma_fragments(e, 16, 4 * ks, out);
+}
+
+// FP64 fragments of the padded s2p product (k_s2p_dmfma): per row tile t of rh, rows
+// q = 1 + 16 t + i, C[q][k] = cos(pi k q/(2N)) over the coefficients k = 4j (k0 k-steps),
+// k = 4j + 2 (k2) and k = 2j + 1 (k1), then rows N - q over k = 2j + 1; zero past their sizes
+inline void s2p_tables_f64(int N, int rh, int k0, int k2, int k1, std::vector<double>& out) {
+    auto part = [&](int t, int ks, int first, int step, bool mirror) {
+        std::vector<long double> e((size_t)16 * 4 * ks, 0.0L);
+        for (int r = 0; r < 16; r++) {
+            const int q = 1 + 16 * t + r;
+            if (2 * q >= N) break;
+            for (int j = 0; first + step * j <= N && j < 4 * ks; j++)
+                e[(size_t)r * 4 * ks + j] = cospi_ratio((long)(first + step * j) * (mirror ? N - q : q), 2L * N);
         }
+        dmfma_fragments(e, 16, 4 * ks, out);
+    };
+    for (int t = 0; t < rh; t++) {
+        part(t, k0, 0, 4, false);
+        part(t, k2, 2, 4, false);
+        part(t, k1, 1, 2, false);
+        part(t, k1, 1, 2, true);
+    }
 }
 
 }  // namespace rpcf_host

@@ -352,25 +352,21 @@ __global__ __launch_bounds__(cheb_dmfma::DShape<FN>::NT, 3) void k_p2s_dmfma(
 }
 
 // -------------------------------------------------------------------------------------
-// The Chebyshev transforms of lengths without a compiled plan (any N = nz - 1), as the same
-// kind of FP64 matrix products with N a run-time number.  The runtime-plan FFT kernels they
-// replace (k_cheb_s2p<1, 0>, k_p2s_nl<0>; RPCF_P2S_MFMA=0 keeps them) run 3 to 5 passes over
-// LDS with index arithmetic by run-time strides: at 40x46x60 (N = 45) 72 and 62 us against
-// 10.5 and 10.3 here, at 100x151x100 (N = 150, where the product's N^2 meets the FFT's N log N)
-// 352 and 281 against 145 and 70.  Bound by the latency of a block's phases on small grids, by
-// the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.2 and
-// 0.3 of 72 TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
+// The padded p2s of lengths without a compiled plan (any N = nz - 1), as the same kind of FP64
+// matrix products with N a run-time number.  The runtime-plan FFT kernel it replaces (k_p2s_nl<0>;
+// RPCF_P2S_MFMA=0 keeps it) runs 3 to 5 passes over LDS with index arithmetic by run-time strides:
+// 62 us at 40x46x60 (N = 45) against 10.3 here, 281 at 100x151x100 (N = 150, where the product's N^2
+// meets the FFT's N log N) against 70.  Bound by the latency of a block's phases on small grids, by
+// the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.3 of 72
+// TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
 // -------------------------------------------------------------------------------------
 namespace cheb_dmfma {
 
 // Sizes of the products of one N.  Rows of the p2s: sym p <= N/2 (NS), anti p <= (N-1)/2 (NA),
-// each in RT row tiles; samples q <= N in NCH chunks of kNChunk.  Rows of the s2p: q <= N in
-// RQ tiles; even and odd coefficients in KE and KO k-steps.  All tables are zero-padded.
+// each in RT row tiles; samples q <= N in NCH chunks of kNChunk.  All tables are zero-padded.
 constexpr int kNChunk = 16;
 struct NShape {
-    int N, NS, NA, RT, NCH, KP, RQ, KE, KO;
-    long s2p_off;  // doubles: the s2p table behind the p2s tables
-    long doubles;
+    int N, NS, NA, RT, NCH, KP;
 };
 inline NShape nshape(int N) {
     NShape s;
@@ -380,22 +376,38 @@ inline NShape nshape(int N) {
     s.RT = ceil_div(s.NS, 16);
     s.NCH = ceil_div(N + 1, kNChunk);
     s.KP = s.NCH * (kNChunk / 4);
-    s.RQ = ceil_div(N + 1, 16);
-    s.KE = 2 * ceil_div(N / 2 + 1, 8);  // pairs of k-steps
-    s.KO = 2 * ceil_div((N + 1) / 2, 8);
-    s.s2p_off = 4L * s.RT * s.KP * 64;
-    s.doubles = s.s2p_off + (long)s.RQ * (s.KE + s.KO) * 64;
     return s;
 }
 // LDS bytes: the operands [set h3, h2, h1][G+, G-][kNChunk][kCols] or the output rows
-// [pencil][nz] of one term; the coefficients [even, odd][4 KE]
+// [pencil][nz] of one term
 inline size_t p2s_n_lds(const NShape& s) {
     const size_t ops = sizeof(double) * 3 * 2 * kNChunk * kCols, out = sizeof(double2) * kPencils * (s.N + 1);
     return ops > out ? ops : out;
 }
-// (rows of kS2pLd doubles: 16 bytes past a full turn of the banks, for the writes along k)
-constexpr int kS2pLd = kCols + 2;
-inline size_t s2p_n_lds(const NShape& s) { return sizeof(double) * 2 * 4 * s.KE * kS2pLd; }
+
+// Sizes of the s2p product of one N: RH tiles of the rows 0 < q < N/2; coefficients k = 4j, 4j + 2
+// and odd in K0, K2 and K1 k-steps (even counts); CW groups of 16 pencils per block.
+struct SShape {
+    int N, RH, K0, K2, K1;
+};
+inline SShape sshape(int N) {
+    SShape s;
+    s.N = N;
+    s.RH = N > 2 ? ceil_div((N - 1) / 2, 16) : 1;
+    s.K0 = 2 * ceil_div(N / 4 + 1, 8);
+    s.K2 = 2 * ceil_div((N + 2) / 4, 8);
+    s.K1 = 2 * ceil_div((N + 1) / 2, 8);
+    return s;
+}
+// A block: CW groups of 8 CT pencils, one wave per row tile and group; where that makes fewer than
+// three waves, two more (which take the sums of the special rows meanwhile).
+__host__ __device__ inline int s2p_extra(int waves) { return waves < 3 ? 2 : 0; }
+inline int s2p_threads(const SShape& s, int cw) { return 64 * (s.RH * cw + s2p_extra(s.RH * cw)); }
+// LDS rows of the coefficients: 16 bytes past a multiple of 128, for the writes along k
+__host__ __device__ constexpr int s2p_ld(int cw, int ct) { return cw * ct * 16 + 2; }
+inline size_t s2p_lds(const SShape& s, int cw, int ct) {
+    return sizeof(double) * 4 * (s.K0 + s.K2 + s.K1) * s2p_ld(cw, ct);
+}
 
 }  // namespace cheb_dmfma
 
@@ -533,64 +545,165 @@ __global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restr
     }
 }
 
-// Padded s2p: F[6][P][nz] -> Y[6][kx][q][ky], one block of four waves per 16 pencils of a field.
-// The pencils' coefficients lie in LDS as B operands; a wave takes row tiles q of the even and
-// odd products (fragments from L2), rows q and 2N - q are their sum and difference, stored from
-// the accumulators: 16 pencils of a row are 256 contiguous bytes.
-template <int = 0>
-__global__ __launch_bounds__(256) void k_s2p_dmfma_n(const double2* __restrict__ F, long fstride, long sF,
-                                                     double2* __restrict__ Y, long ystride, long sY, Dims d,
-                                                     const double* __restrict__ tab, cheb_dmfma::NShape sh,
-                                                     const int* __restrict__ ids) {
+// Padded s2p of the FP64 form: F[6][P][nz] -> Y[6][kx][q][ky], f_q = sum_k a_k cos(pi k q/(2N)),
+// as dense products on the matrix cores.  The cosines fold twice: with E0, E2 and O the sums over
+// k = 4j, k = 4j + 2 and odd k at row q, and O' that over odd k at row N - q,
+//   f_q = E0 + E2 + O, f_{N-q} = E0 - E2 + O', f_{N+q} = E0 - E2 - O', f_{2N-q} = E0 + E2 - O
+// so the rows 0 < q < N/2 give all the others, for 3/4 N^2 products a column; the rows 0, N, 2N and
+// N/2, 3N/2 (N even) are sums on the vector units.  A block takes CW groups of pencils of a field,
+// their coefficients in LDS as B operands, with one wave per row tile and group; the fragments
+// stream from L2, two k-step pairs ahead, and the rows leave from the accumulators.  A group is 16
+// pencils (CT = 2: a tile of their real parts and one of their imaginary parts, 256 contiguous
+// bytes of a row), or on small grids 8 (CT = 1: real and imaginary parts share a tile), whose
+// waves run half as many products each.  Bound by the latency of a block's phases on small grids,
+// by memory, the fragments' reads from L2 and the matrix cores' rate (N^2) on large ones: 233 us at
+// 256x97x256 (the bytes take 188 at the copy rate), 90 at 128x129x128 (63), 40 at 128x65x128, 16.3
+// at 64x65x64, 7.6 at 32x33x32; the half-length FFTs of k_cheb_s2p_h take 274, 97, 56, 22.9 and
+// 10.3.  With the first fold only (N^2 products) it took 360 at 256x101x256 and 107 at 128x126x128,
+// now 273 and 85.  96 registers keep five waves a SIMD: with four, 265 at 256x97x256.
+template <int CT>
+__global__ __launch_bounds__(512, 5) void k_s2p_dmfma(const double2* __restrict__ F, long fstride, long sF,
+                                                   double2* __restrict__ Y, long ystride, long sY, Dims d,
+                                                   const double* __restrict__ tab, cheb_dmfma::SShape sh, int CW,
+                                                   const int* __restrict__ ids) {
     using namespace cheb_dmfma;
     RPCF_LDS(double);
-    const int N = sh.N, nz = N + 1, pz = 2 * N + 1, KE = sh.KE, KO = sh.KO;
+    constexpr int G = 8 * CT;  // pencils per group; columns [group][re, im][pencil]
+    const int N = sh.N, nz = N + 1, pz = 2 * N + 1, ld = s2p_ld(CW, CT), nthr = blockDim.x;
     const int tid = threadIdx.x, lane = tid & 63, kq = lane >> 4, lc = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int f = blockIdx.z % 6, kx = blockIdx.y, ky0 = blockIdx.x * kPencils;
+    const int rt = wave % sh.RH, cg = wave / sh.RH;
+    const int f = blockIdx.z % 6, kx = blockIdx.y, ky0 = blockIdx.x * G * CW;
     const long slot = ids[blockIdx.z / 6];
-    const int nb = min(kPencils, d.ny - ky0);
+    const int nb = min(G * CW, d.ny - ky0);
     const double2* in = F + slot * sF + f * fstride + ((long)ky0 * d.hnx + kx) * nz;
     double2* out = Y + slot * sY + f * ystride + (long)kx * pz * d.ny + ky0;
-    const int rows = 4 * KE;  // of each parity, zero past the coefficients
-    for (int b = wave; b < kPencils; b += 4)
-        for (int k = lane; k < 2 * rows; k += 64) {
-            const double2 v = b < nb && k < nz ? in[(long)b * d.hnx * nz + k] : make_double2(0.0, 0.0);
-            double* o = lds + ((k & 1) * rows + (k >> 1)) * kS2pLd + b;
-            o[0] = v.x;
-            o[kPencils] = v.y;
+    const int rows0 = 4 * sh.K0, rows2 = 4 * sh.K2, rows = rows0 + rows2 + 4 * sh.K1;
+    // coefficient k of pencil b to its set's row; zeros in the rows past the coefficients
+    {
+        const FastDiv by_nz(nz);
+        const int pstride = d.hnx * nz;
+        staged<8>(
+            G * CW * nz, tid, nthr,
+            [&](int i) {
+                const unsigned b = (unsigned)i / by_nz, k = i - b * nz;
+                return (int)b < nb ? in[b * pstride + k] : make_double2(0.0, 0.0);
+            },
+            [&](int i, double2 v) {
+                const unsigned b = (unsigned)i / by_nz, k = i - b * nz;
+                const unsigned r = k & 1 ? rows0 + rows2 + (k >> 1) : k & 2 ? rows0 + (k >> 2) : k >> 2;
+                double* o = lds + r * ld + (b / G) * (2 * G) + b % G;
+                o[0] = v.x;
+                o[G] = v.y;
+            });
+        for (int i = tid; i < (rows - nz) * 2 * G * CW; i += nthr) {
+            int r = i / (2 * G * CW);
+            const int c = i - r * 2 * G * CW;
+            const int n0 = N / 4 + 1, n2 = (N + 2) / 4;
+            if (r < rows0 - n0) r += n0;
+            else if ((r -= rows0 - n0) < rows2 - n2) r += rows0 + n2;
+            else r += -(rows2 - n2) + rows0 + rows2 + (N + 1) / 2;
+            lds[r * ld + c] = 0.0;
         }
+    }
     __syncthreads();
+    const int P0 = sh.K0 / 2, P2 = P0 + sh.K2 / 2, P1 = P2 + sh.K1 / 2;  // ends of the sets in k-step pairs
     const v4d zero4 = {0.0, 0.0, 0.0, 0.0};
-    for (int rt = wave; rt < sh.RQ; rt += 4) {
-        const double* te = tab + sh.s2p_off + (long)rt * (KE + KO) * 64 + lane;
-        const double* to = te + (long)KE * 64;
-        v4d e[2] = {zero4, zero4}, o[2] = {zero4, zero4};
-        // two k-steps at a time, the next two fragments in flight
-        auto product = [&](const double* t, int par, int ks, v4d* acc) {
-            double a0 = t[0], a1 = t[64];
-            for (int s = 0; s < ks; s += 2) {
-                const long nx = 64L * min(s + 2, ks - 2);
-                const double n0 = t[nx], n1 = t[nx + 64];
-                const double* b = lds + (par * rows + 4 * s + kq) * kS2pLd + lc;
-                const double b00 = b[0], b01 = b[kPencils], b10 = b[4 * kS2pLd], b11 = b[4 * kS2pLd + kPencils];
-                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b00, acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a0, b01, acc[1], 0, 0, 0);
-                acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b10, acc[0], 0, 0, 0);
-                acc[1] = __builtin_amdgcn_mfma_f64_16x16x4f64(a1, b11, acc[1], 0, 0, 0);
-                a0 = n0, a1 = n1;
+    v4d e0[CT], e2[CT], o1[CT], om[CT];
+#pragma unroll
+    for (int ct = 0; ct < CT; ct++) e0[ct] = e2[ct] = o1[ct] = om[ct] = zero4;
+    if (cg < CW) {
+        const double* t = tab + (long)rt * (sh.K0 + sh.K2 + 2 * sh.K1) * 64 + lane;
+        const double* tm = t + (sh.K0 + sh.K2 + sh.K1) * 64;
+        const double* bl = lds + kq * ld + cg * 16 * CT + lc;
+        double c0 = t[0], c1 = t[64], n0 = t[128 * min(1, P1 - 1)], n1 = t[128 * min(1, P1 - 1) + 64];
+        double m0 = tm[0], m1 = tm[64];
+        auto pairs = [&](int p, int end, v4d* acc, bool mirror) {
+            for (; p < end; p++) {
+                const int nx = 128 * min(p + 2, P1 - 1), mx = 128 * min(max(p + 1 - P2, 0), P1 - P2 - 1);
+                const double f0 = t[nx], f1 = t[nx + 64];
+                const double* b = bl + 8 * p * ld;
+                double b0[CT], b1[CT];
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) b0[ct] = b[16 * ct], b1[ct] = b[4 * ld + 16 * ct];
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(c0, b0[ct], acc[ct], 0, 0, 0);
+                if (mirror) {
+                    const double g0 = tm[mx], g1 = tm[mx + 64];
+#pragma unroll
+                    for (int ct = 0; ct < CT; ct++) om[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(m0, b0[ct], om[ct], 0, 0, 0);
+#pragma unroll
+                    for (int ct = 0; ct < CT; ct++) om[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(m1, b1[ct], om[ct], 0, 0, 0);
+                    m0 = g0, m1 = g1;
+                }
+#pragma unroll
+                for (int ct = 0; ct < CT; ct++) acc[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(c1, b1[ct], acc[ct], 0, 0, 0);
+                c0 = n0, c1 = n1, n0 = f0, n1 = f1;
             }
         };
-        product(te, 0, KE, e);
-        product(to, 1, KO, o);
-        if (lc < nb) {
+        pairs(0, P0, e0, false);
+        pairs(P0, P2, e2, false);
+        pairs(P2, P1, o1, true);
+    }
+    const int bp = cg * G + (CT == 2 ? lc : lc & 7);  // this lane's pencil
+    if (cg < CW && bp < nb) {
+        // CT = 2: (re, im) of a row; CT = 1: the part of this lane
+        double* o = (double*)(out + bp) + (CT == 2 ? 0 : lc >> 3);
+        const long ny = 2 * d.ny;
+        auto put = [&](long q, double x, double y) {
+            if constexpr (CT == 2) *(double2*)(o + q * ny) = make_double2(x, y);
+            else o[q * ny] = x;
+        };
 #pragma unroll
-            for (int r = 0; r < 4; r++) {
-                const int q = 16 * rt + kq + 4 * r;
-                if (q > N) continue;
-                out[(long)q * d.ny + lc] = make_double2(e[0][r] + o[0][r], e[1][r] + o[1][r]);
-                if (q < N) out[(long)(2 * N - q) * d.ny + lc] = make_double2(e[0][r] - o[0][r], e[1][r] - o[1][r]);
-            }
+        for (int r = 0; r < 4; r++) {
+            const int q = 1 + 16 * rt + kq + 4 * r;
+            if (2 * q >= N) continue;
+            constexpr int I = CT - 1;
+            const double s0 = e0[0][r] + e2[0][r], s1 = e0[I][r] + e2[I][r];
+            const double t0 = e0[0][r] - e2[0][r], t1 = e0[I][r] - e2[I][r];
+            put(q, s0 + o1[0][r], s1 + o1[I][r]);
+            put(N - q, t0 + om[0][r], t1 + om[I][r]);
+            put(N + q, t0 - om[0][r], t1 - om[I][r]);
+            put(2 * N - q, s0 - o1[0][r], s1 - o1[I][r]);
+        }
+    }
+    // rows 0, N, 2N: sums of the three sets; rows N/2, 3N/2: k = 4j with signs (-1)^j, odd k with
+    // cos(pi k/4).  A wave takes 16 columns, a quarter of the coefficients a lane.
+    const int extra = s2p_extra(sh.RH * CW), waves = nthr >> 6, first = extra ? sh.RH * CW : 0;
+    for (int task = wave - first; task < CT * CW; task += waves - first) {
+        if (task < 0) break;
+        const int c = 16 * task + lc, b = c / (2 * G) * G + c % G, im = c / G & 1;
+        const double* col = lds + c;
+        double s0 = 0.0, s2 = 0.0, s1 = 0.0, z0 = 0.0, z1 = 0.0;
+#pragma unroll 4
+        for (int r = kq; r < rows0; r += 4) {
+            const double v = col[r * ld];
+            s0 += v;
+            z0 += kq & 1 ? -v : v;
+        }
+#pragma unroll 4
+        for (int r = kq; r < rows2; r += 4) s2 += col[(rows0 + r) * ld];
+#pragma unroll 4
+        for (int r = kq; r < rows - rows0 - rows2; r += 4) {
+            const double v = col[(rows0 + rows2 + r) * ld];
+            s1 += v;
+            z1 += (kq + 1) & 2 ? -v : v;
+        }
+#pragma unroll
+        for (int m = 16; m <= 32; m *= 2) {
+            s0 += __shfl_xor(s0, m), s2 += __shfl_xor(s2, m), s1 += __shfl_xor(s1, m);
+            z0 += __shfl_xor(z0, m), z1 += __shfl_xor(z1, m);
+        }
+        if (b >= nb) continue;
+        double* o = (double*)(out + b) + im;
+        const long ny = 2 * d.ny;
+        z1 *= 0.70710678118654752440;
+        if (kq == 0) o[0] = s0 + s2 + s1;
+        else if (kq == 1) o[N * ny] = s0 - s2;
+        else if (kq == 2) o[2 * N * ny] = s0 + s2 - s1;
+        else if (!(N & 1)) {
+            o[N / 2 * ny] = z0 + z1;
+            o[(N + N / 2) * ny] = z0 - z1;
         }
     }
 }

@@ -102,10 +102,14 @@ struct rpcf_ctx {
     int mt_s0 = 0, mt_s1 = 0;
     // FP64 form: the padded p2s with the nonlinear combination as FP64 products (k_cheb_dmfma.hpp)
     int use_dmfma = 0;
-    // lengths without a compiled plan: s2p and p2s as FP64 products of run-time size
+    // lengths without a compiled plan: p2s as FP64 products of run-time size
     int use_dmfma_n = 0;
     cheb_dmfma::NShape dn{};
     double* DT = nullptr;  // fragments of the tables of either
+    // FP64 form: the padded s2p as products on the matrix cores, its tables
+    int use_s2p = 0;
+    cheb_dmfma::SShape sn{};
+    double* ST = nullptr;
     // per-slot arrays ([capacity][...]) and their slot strides in elements
     double2* F = nullptr;     // [6][P][nz] u, v, w, ox, oy, oz
     double2* SV = nullptr;    // [P][nz] v-hat (u0 in pencil 0)
@@ -578,6 +582,21 @@ int enq_velocity(rpcf_ctx* c, const int* ids, int n, bool cap = false) {
 // twiddles of a plan of length n in the LDS of the kernels that copy them there
 size_t tw_lds(int n) { return compiled_len(n) ? ct_tw_lds_len(n) : n; }
 
+// the padded s2p of nf fields (6 a member, or one) by k_s2p_dmfma: enough groups of 16 pencils for
+// four waves a block, fewer where that leaves compute units short of blocks, then groups of 8
+void s2p_product(rpcf_ctx* c, int nf, const double2* F, long fS, long sF, double2* Y, long yS, long sY, const int* ids) {
+    const Dims d = c->d;
+    auto blocks = [&](int cw, int ct) { return (d.ny + 8 * ct * cw - 1) / (8 * ct * cw); };
+    int cw = c->sn.RH == 1 ? 4 : c->sn.RH == 2 ? 2 : 1;
+    while (cw > 1 && (long)blocks(cw, 2) * d.hnx * nf < 4L * c->ncu) cw /= 2;
+    const int ct = (long)blocks(cw, 2) * d.hnx * nf < 4L * c->ncu ? 1 : 2;
+    const dim3 g(blocks(cw, ct), d.hnx, nf);
+    const int thr = cheb_dmfma::s2p_threads(c->sn, cw);
+    const size_t lds = cheb_dmfma::s2p_lds(c->sn, cw, ct);
+    if (ct == 1) k_s2p_dmfma<1><<<g, thr, lds, c->stream>>>(F, fS, sF, Y, yS, sY, d, c->ST, c->sn, cw, ids);
+    else k_s2p_dmfma<2><<<g, thr, lds, c->stream>>>(F, fS, sF, Y, yS, sY, d, c->ST, c->sn, cw, ids);
+}
+
 // span transforms of nf fields (6 or 3 a member, or one): the compiled plan of my where there
 // is one; the mixed form has no other
 template <typename R>
@@ -673,6 +692,9 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                         return;
                     }
                 }
+                if constexpr (f64) {
+                    if (c->use_s2p) return s2p_product(c, 6 * n, c->F, fS, c->sF, Y, yS, c->sY, ids);
+                }
                 switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                             \
     case L:                                                                                                      \
@@ -686,15 +708,9 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
                     default:
-                        if constexpr (f64) {
-                            if (c->use_dmfma_n)
-                                k_s2p_dmfma_n<<<dim3((d.ny + cheb_dmfma::kPencils - 1) / cheb_dmfma::kPencils, d.hnx, 6 * n),
-                                                256, cheb_dmfma::s2p_n_lds(c->dn), c->stream>>>(
-                                    c->F, fS, c->sF, Y, yS, c->sY, d, c->DT, c->dn, ids);
-                            else
-                                k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(c->F, fS, c->sF, Y, yS, c->sY, d,
-                                                                                  c->pl_zn, tw4, TB, ld, ids);
-                        }
+                        if constexpr (f64)
+                            k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(c->F, fS, c->sF, Y, yS, c->sY, d,
+                                                                              c->pl_zn, tw4, TB, ld, ids);
                 }
             },
             cap);
@@ -953,7 +969,7 @@ int autotune_tiles(rpcf_ctx* c) {
 #undef RPCF_CASE
     // k_velocity_tile and k_p2s_nl2 run for compiled Chebyshev lengths only
     const bool span = c->mixed || !two_pass<double>(d.my), lamb = c->mixed || !two_pass<double>(d.mx);
-    const bool tunable[6] = {!c->use_mfma && !c->use_dmfma_n, span, span, lamb, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
+    const bool tunable[6] = {!c->use_mfma && !c->use_s2p, span, span, lamb, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
     if (mode == "half") {
         for (int i = 0; i < 6; i++)
             if (tunable[i] && *tile_ref(c, i) >= 2) *tile_ref(c, i) /= 2;
@@ -1035,7 +1051,7 @@ void free_ctx(rpcf_ctx* c) {
     if (c->gexec) (void)hipGraphExecDestroy(c->gexec);
     void* ptrs[] = {c->F,   c->SV, c->SE, c->NL,  c->Y,     c->W,  c->Z2, c->WL, c->MINV, c->TF,
                     c->U,  c->DU, c->DDU, c->MEANU, c->MP, c->PH, c->T0, c->T2,   c->T4,  c->T0t,
-                    c->qw, c->tw, c->ids_dev, c->ids_zero, c->twf, c->MINVH, c->MINVE, c->MINVF, c->PAIRS, c->MT, c->DT};
+                    c->qw, c->tw, c->ids_dev, c->ids_zero, c->twf, c->MINVH, c->MINVE, c->MINVF, c->PAIRS, c->MT, c->DT, c->ST};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     for (auto& p : c->pending) { (void)hipEventDestroy(p.a); (void)hipEventDestroy(p.b); }
@@ -1088,9 +1104,21 @@ const std::vector<double>& dmfma_tables(int N) {
         rpcf_host::p2s_tables_f64(N, t);
     } else {
         const cheb_dmfma::NShape s = cheb_dmfma::nshape(N);
-        rpcf_host::cheb_tables_n(N, s.RT, s.KP, s.RQ, s.KE, s.KO, t);
+        rpcf_host::p2s_tables_n(N, s.RT, s.KP, t);
     }
     return g_dt.emplace(N, std::move(t)).first->second;
+}
+
+std::map<int, std::vector<double>> g_st;  // and of the s2p product
+
+const std::vector<double>& s2p_tables(int N) {
+    std::lock_guard<std::mutex> lk(g_mt_mu);
+    auto it = g_st.find(N);
+    if (it != g_st.end()) return it->second;
+    const cheb_dmfma::SShape s = cheb_dmfma::sshape(N);
+    std::vector<double> t;
+    rpcf_host::s2p_tables_f64(N, s.RH, s.K0, s.K2, s.K1, t);
+    return g_st.emplace(N, std::move(t)).first->second;
 }
 
 // allocation and shape set-up of a context of `capacity` slots; on failure the caller frees it
@@ -1214,9 +1242,8 @@ int init_ctx(rpcf_ctx* c) {
             c->use_mfma = 1;
         }
     }
-    // FP64 form: the padded p2s + nonlinear combination as FP64 matrix-core products for the
-    // compiled lengths up to 2N = 384, and both padded Chebyshev transforms for the lengths
-    // without a compiled plan; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
+    // FP64 form: the padded s2p and the padded p2s + nonlinear combination as FP64 matrix-core
+    // products, but for 2N = 512; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
     if (!c->mixed && (2 * d.N <= 384 || !compiled_len(2 * d.N))) {
         const char* e = getenv("RPCF_P2S_MFMA");
         if (!(e && e[0] == '0')) {
@@ -1229,6 +1256,11 @@ int init_ctx(rpcf_ctx* c) {
                 c->use_dmfma_n = 1;
                 c->dn = cheb_dmfma::nshape(d.N);
             }
+            const std::vector<double>& st = s2p_tables(d.N);
+            if ((rc = dalloc(c, &c->ST, st.size()))) return rc;
+            RCCHK(copy_sync(c, c->ST, st.data(), sizeof(double) * st.size(), hipMemcpyHostToDevice));
+            c->use_s2p = 1;
+            c->sn = cheb_dmfma::sshape(d.N);
         }
     }
 
@@ -1328,7 +1360,8 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_lin_tv_stream<S, 8>, lim);
     RPCF_TV_STEPS(RPCF_CASE)
 #undef RPCF_CASE
-    allow_lds(k_s2p_dmfma_n<0>, lim);
+    allow_lds(k_s2p_dmfma<1>, lim);
+    allow_lds(k_s2p_dmfma<2>, lim);
 #define RPCF_CASE(RT) allow_lds(k_p2s_dmfma_n<RT>, lim);
     RPCF_P2S_TILES(RPCF_CASE)
 #undef RPCF_CASE
@@ -1780,7 +1813,8 @@ int enq_spec_to_phys(rpcf_ctx* c, const double2* f, double2* y, double2* w, doub
     const int TB = c->TB_s2p, ld = c->ld_zn;
     dim3 g((d.ny + TB - 1) / TB, d.hnx, 1);
     const size_t lds = sizeof(double2) * TB * ld;
-    switch (2 * d.N) {
+    if (padded && c->use_s2p) s2p_product(c, 1, f, 0, 0, y, 0, 0, c->ids_zero);
+    else switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                                \
     case L:                                                                                                         \
         if (!padded)                                                                                                \
@@ -1794,10 +1828,7 @@ int enq_spec_to_phys(rpcf_ctx* c, const double2* f, double2* y, double2* w, doub
         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
         default:
-            if (padded && c->use_dmfma_n)
-                k_s2p_dmfma_n<<<dim3((d.ny + cheb_dmfma::kPencils - 1) / cheb_dmfma::kPencils, d.hnx, 1), 256,
-                                cheb_dmfma::s2p_n_lds(c->dn), c->stream>>>(f, 0, 0, y, 0, 0, d, c->DT, c->dn, c->ids_zero);
-            else if (padded)
+            if (padded)
                 k_cheb_s2p<1><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
             else
                 k_cheb_s2p<0><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);

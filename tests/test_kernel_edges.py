@@ -111,6 +111,27 @@ def test_lamb_vector(mx):
     g.close(), o.close()
 
 
+# padded values by products: blocks of one, two and four groups of 16 pencils, of groups of 8, whole
+# and ragged groups; N odd and even, rows below N/2 that fill tiles, leave one over or are few
+@pytest.mark.parametrize("N,mx,my", [(4, 24, 24), (5, 30, 24), (16, 128, 384), (32, 24, 36), (36, 30, 24), (45, 128, 192),
+                                     (45, 60, 90), (64, 128, 192), (75, 24, 54), (100, 12, 30), (128, 128, 96),
+                                     (192, 24, 36)])
+def test_padded_values(N, mx, my):
+    g, o = pair(rpcf.make_params(mx, my, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=900.0, Ro=0.1, dt=0.002))
+    rng = np.random.default_rng(N + mx)
+    shape = g.s["P"], g.s["nz"]
+    f = [(rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / (1.0 + np.arange(g.s["nz"])) ** 2
+         for _ in range(6)]
+    for s in (g, o):
+        for i in range(6):
+            s.set_field(i, f[i])
+        s.nonlinear()
+    for a, b in zip(g.get_nonlinear(), o.get_nonlinear()):
+        assert rel(a, b) < 1e-12
+    assert rel(g.spec_to_phys(f[0]), o.spec_to_phys(f[0])) < 1e-13
+    g.close(), o.close()
+
+
 # solves of an odd base profile by conjugate parity blocks, at N odd and even, the smallest pair
 # counts, row pairs that fill whole and partial batches of every column group, the largest N: the
 # full inverses' results after one step.  2e-13 is the bound of the even profiles' blocks with
