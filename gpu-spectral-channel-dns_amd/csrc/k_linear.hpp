@@ -254,81 +254,104 @@ __global__ __launch_bounds__(256) void k_transpose_square(double2* __restrict__ 
     if (i2 < n && j2 < n) m[(long)i2 * n + j2] = a[x][y];
 }
 
-// Chebyshev derivative of one complex coefficient: ddz (source/RPCFKernels.cu:476-520)
-__device__ __forceinline__ double2 zddz(const double2* a, int k, int n) {
-    double re = 0.0, im = 0.0;
-    for (int j = k + 1; j < n; j += 2) {
-        const double dm = 2 * (double)j;
-        re = re + a[j].x * dm;
-        im = im + a[j].y * dm;
+template <int W> __device__ __forceinline__ double2 wave_get(double2 a, int lane) {
+    return make_double2(__shfl(a.x, lane, W), __shfl(a.y, lane, W));
+}
+// Chebyshev derivative (ddz, source/RPCFKernels.cu:476-520) of a pencil held by W lanes of a wave, lane
+// l the coefficients k = l + W r, and (X) every lane the coefficient W R: with
+// t_k = 2k a_k + t_{k+2}, (Da)_k = t_{k+1}, halved at k = 0.  A suffix sum over the lanes of each
+// parity per W coefficients, carried down from the next W.
+template <int W, int R, bool X>
+__device__ __forceinline__ void wave_ddz(const double2 (&a)[R], double2 ax, int lane, double2 (&da)[R]) {
+    double2 t[R + 1];
+    t[R] = X ? zmulr(ax, 2.0 * W * R) : make_double2(0.0, 0.0);
+#pragma unroll
+    for (int r = R - 1; r >= 0; r--) {
+        double2 v = zmulr(a[r], 2.0 * (lane + W * r));
+#pragma unroll
+        for (int s = 2; s < W; s *= 2) {
+            const double2 w = make_double2(__shfl_down(v.x, s, W), __shfl_down(v.y, s, W));
+            if (lane + s < W) v = zadd(v, w);
+        }
+        if (r + 1 < R) v = zadd(v, wave_get<W>(t[r + 1], lane & 1));
+        else if (X && !(lane & 1)) v = zadd(v, t[R]);
+        t[r] = v;
     }
-    return k == 0 ? make_double2(re * 0.5, im * 0.5) : make_double2(re, im);
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        double2 v = make_double2(__shfl_down(t[r].x, 1, W), __shfl_down(t[r].y, 1, W));
+        const double2 up = r + 1 < R ? wave_get<W>(t[r + 1], 0) : t[R];
+        if (lane == W - 1) v = up;
+        da[r] = r == 0 && lane == 0 ? zmulr(v, 0.5) : v;
+    }
 }
 
 // -------------------------------------------------------------------------------------
 // Velocity recovery: getVelocityKernel_sm (source/velocity.cu:90-170) after the state
-// copy of source/solver.cpp:95-96.  One block per pencil (x) and member (y), thread k =
-// coefficient k.  F[6][P][nz] <- (u, v, w, ox, oy, oz) from (v-hat, eta-hat).
+// copy of source/solver.cpp:95-96.  F[6][P][nz] <- (u, v, w, ox, oy, oz) from (v-hat, eta-hat):
+// pencil != (0,0):  u = (i a/k2) Dv - (i b/k2) eta,  w = (i b/k2) Dv + (i a/k2) eta,
+//                   ox = D w - i b v,  oy = -D u + i a v,  oz = eta;
+// pencil (0,0):     u = u0, w = w0, v = 0, ox = D w0, oy = -D u0, oz = 0.
+// One wave, or for nz <= 33 half a wave, per pencil (W lanes), R coefficients a lane (X: nz = W R + 1,
+// the last one held by all), the derivatives by wave_ddz: no LDS memory, no barrier, every access a
+// contiguous run of the pencil.  Bound by memory on large grids, by the chain of lane exchanges on
+// small ones: 69 us at 256x97x256 and 32 at 128x129x128 (the bytes take 83 and 28 at the copy rate),
+// 9.3 at 64x65x64, 6.6 at 32x33x32; the tiled scan (k_velocity_tile) takes 76, 38, 12.4 and 8.3.
+// Lengths without a compiled plan summed each derivative directly, O(nz) a coefficient: 167 us at
+// 256x101x256 and 68 at 128x126x128, now 72 and 28.
 // -------------------------------------------------------------------------------------
-__global__ void k_velocity(const double2* __restrict__ sv, const double2* __restrict__ se, long sS,
-                           double2* __restrict__ F, long fstride, long sF, Dims d, Members mb) {
-    __shared__ double2 sw[256], soz[256], su[256], sv2[256];
-    const int slot = mb.ids[blockIdx.y];
+template <int W, int R, bool X>
+__global__ __launch_bounds__(256) void k_velocity(const double2* __restrict__ sv, const double2* __restrict__ se, long sS,
+                                                  double2* __restrict__ F, long fstride, long sF, Dims d, Members mb) {
+    const int slot = mb.ids[blockIdx.y], lane = threadIdx.x % W;
     const MemberParams& mp = mb.mp[slot];
+    const int p = blockIdx.x * (256 / W) + threadIdx.x / W;
+    if (p >= d.P) return;
+    const int kx = p % d.hnx, ky = p / d.hnx, nz = d.nz;
+    const long o = (long)p * nz;
+    sv += slot * sS + o;
+    se += slot * sS + o;
+    F += slot * sF + o;
+    const double2 zero = make_double2(0.0, 0.0);
+    double2 v[R], e[R], u[R], w[R], du[R], dw[R], vx = zero, ex = zero;
+#pragma unroll
+    for (int r = 0; r < R; r++) {
+        const int k = lane + W * r;
+        v[r] = e[r] = zero;
+        if (k < nz) v[r] = sv[k], e[r] = se[k];
+    }
+    if (X) vx = sv[W * R], ex = se[W * R];
+    const bool mean = p == 0;
     LinParams lp;
     lp.aphi = mp.aphi;
     lp.beta = mp.beta;
-    lp.Re = mp.Re;
-    lp.dt = mp.dt;
-    sv += slot * sS;
-    se += slot * sS;
-    F += slot * sF;
-    const int p = blockIdx.x, kx = p % d.hnx, ky = p / d.hnx, k = threadIdx.x, nz = d.nz;
-    const long o = (long)p * nz + k;
-    if (k < nz) {
-        sw[k] = sv[o];
-        soz[k] = se[o];
-    }
-    __syncthreads();
-    if (kx == 0 && ky == 0) {
-        if (k < nz) {
-            su[k] = sw[k];
-            sv2[k] = soz[k];
-        }
-        __syncthreads();
-        if (k < nz) {
-            const double2 du = zddz(su, k, nz), dv = zddz(sv2, k, nz);
-            F[0 * fstride + o] = su[k];
-            F[1 * fstride + o] = sv2[k];
-            F[2 * fstride + o] = make_double2(0.0, 0.0);
-            F[3 * fstride + o] = dv;
-            F[4 * fstride + o] = zmulr(du, -1.0);
-            F[5 * fstride + o] = make_double2(0.0, 0.0);
-        }
-        return;
-    }
     double ia, ib;
     ab_of(d, lp, kx, ky, &ia, &ib);
-    const double kmn = ia * ia + ib * ib;
-    const double kmn1 = 1.0 / kmn;
-    if (k < nz) {
-        const double2 t = zddz(sw, k, nz);
-        su[k] = zsub(zmul(make_double2(0.0, ia * kmn1), t), zmul(make_double2(0.0, ib * kmn1), soz[k]));
-        sv2[k] = zadd(zmul(make_double2(0.0, ib * kmn1), t), zmul(make_double2(0.0, ia * kmn1), soz[k]));
-    }
-    __syncthreads();
-    if (k < nz) {
-        const double2 dv = zddz(sv2, k, nz);
-        const double2 ox = zadd(dv, zmul(make_double2(0.0, -1.0 * ib), sw[k]));
-        const double2 du = zddz(su, k, nz);
-        const double2 oy = zadd(zmulr(du, -1.0), zmul(make_double2(0.0, ia), sw[k]));
-        F[0 * fstride + o] = su[k];
-        F[1 * fstride + o] = sv2[k];
-        F[2 * fstride + o] = sw[k];
-        F[3 * fstride + o] = ox;
-        F[4 * fstride + o] = oy;
-        F[5 * fstride + o] = soz[k];
-    }
+    const double kmn1 = 1.0 / (ia * ia + ib * ib), ca = ia * kmn1, cb = ib * kmn1;
+    auto uw = [&](double2 v, double2 e, double2 dv, double2* u, double2* w) {
+        *u = make_double2(mean ? v.x : cb * e.y - ca * dv.y, mean ? v.y : ca * dv.x - cb * e.x);
+        *w = make_double2(mean ? e.x : -(cb * dv.y + ca * e.y), mean ? e.y : cb * dv.x + ca * e.x);
+    };
+    wave_ddz<W, R, X>(v, vx, lane, du);
+#pragma unroll
+    for (int r = 0; r < R; r++) uw(v[r], e[r], du[r], u + r, w + r);
+    double2 ux, wx;
+    uw(vx, ex, zero, &ux, &wx);
+    wave_ddz<W, R, X>(u, ux, lane, du);
+    wave_ddz<W, R, X>(w, wx, lane, dw);
+    auto put = [&](int k, double2 v, double2 e, double2 u, double2 w, double2 du, double2 dw) {
+        F[0 * fstride + k] = u;
+        F[1 * fstride + k] = w;
+        // (pencil (0,0) has alpha = beta = 0)
+        F[2 * fstride + k] = make_double2(mean ? 0.0 : v.x, mean ? 0.0 : v.y);
+        F[3 * fstride + k] = make_double2(dw.x + ib * v.y, dw.y - ib * v.x);
+        F[4 * fstride + k] = make_double2(-du.x - ia * v.y, -du.y + ia * v.x);
+        F[5 * fstride + k] = make_double2(mean ? 0.0 : e.x, mean ? 0.0 : e.y);
+    };
+#pragma unroll
+    for (int r = 0; r < R; r++)
+        if (lane + W * r < nz) put(lane + W * r, v[r], e[r], u[r], w[r], du[r], dw[r]);
+    if (X && lane == 0) put(W * R, vx, ex, ux, wx, zero, zero);
 }
 
 // r-th entry of (minv of slot) * x, j ascending (m_multi_v, source/matrix_op.cpp:68-78)

@@ -554,6 +554,21 @@ int enq_velocity(rpcf_ctx* c, const int* ids, int n, bool cap = false) {
     return launch(
         c, KID_VELOCITY,
         [&] {
+            if (!c->mixed) {
+                // the coefficients in whole waves (or half waves) and one over, or rounded up
+                auto run = [&](auto kernel, int per) {
+                    kernel<<<dim3((d.P + per - 1) / per, n), 256, 0, c->stream>>>(c->SV, c->SE, c->sS, c->F, fS, c->sF, d,
+                                                                                members(c, ids));
+                };
+                const int over = d.nz % 64 == 1, r = (d.nz + 63 - over) / 64;
+                if (d.nz <= 32) run(k_velocity<32, 1, false>, 8);
+                else if (d.nz == 33) run(k_velocity<32, 1, true>, 8);
+                else if (r == 1) run(over ? k_velocity<64, 1, true> : k_velocity<64, 1, false>, 4);
+                else if (r == 2) run(over ? k_velocity<64, 2, true> : k_velocity<64, 2, false>, 4);
+                else if (r == 3) run(over ? k_velocity<64, 3, true> : k_velocity<64, 3, false>, 4);
+                else run(k_velocity<64, 4, false>, 4);  // nz <= 256
+                return;
+            }
             const int TB = c->TB_vel, ld = c->ld_zn;
             dim3 g((d.ny + TB - 1) / TB, d.hnx, n);
             const size_t lds = sizeof(double2) * ((size_t)TB * ld + 256);
@@ -569,11 +584,6 @@ int enq_velocity(rpcf_ctx* c, const int* ids, int n, bool cap = false) {
         break;
                 RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-                default: {
-                    const int thr = 64 * ((d.nz + 63) / 64);
-                    k_velocity<<<dim3(d.P, n), thr, 0, c->stream>>>(c->SV, c->SE, c->sS, c->F, fS, c->sF, d,
-                                                                    members(c, ids));
-                }
             }
         },
         cap);
@@ -967,9 +977,10 @@ int autotune_tiles(rpcf_ctx* c) {
 #define RPCF_CASE(L) compiled |= 2 * d.N == L;
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-    // k_velocity_tile and k_p2s_nl2 run for compiled Chebyshev lengths only
+    // k_velocity_tile (mixed form) and k_p2s_nl2 run for compiled Chebyshev lengths only
     const bool span = c->mixed || !two_pass<double>(d.my), lamb = c->mixed || !two_pass<double>(d.mx);
-    const bool tunable[6] = {!c->use_mfma && !c->use_s2p, span, span, lamb, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma, compiled};
+    const bool tunable[6] = {!c->use_mfma && !c->use_s2p, span, span, lamb, c->TB_nl2 > 0 && !c->use_mfma && !c->use_dmfma,
+                             compiled && c->mixed};
     if (mode == "half") {
         for (int i = 0; i < 6; i++)
             if (tunable[i] && *tile_ref(c, i) >= 2) *tile_ref(c, i) /= 2;

@@ -132,6 +132,23 @@ def test_padded_values(N, mx, my):
     g.close(), o.close()
 
 
+# velocity recovery: half a wave, one to four coefficients a lane, whole, one over and partial;
+# pencils that fill blocks of 4 and 8 and not.  Sums of at most N/2 terms without cancellation:
+# N/2 2^-53 = 1.4e-14 relative at most.
+@pytest.mark.parametrize("N", [4, 5, 30, 32, 36, 60, 64, 72, 120, 128, 135, 160, 192, 200, 225, 250])
+def test_velocity(N):
+    g, o = pair(rpcf.make_params(12 if N % 2 else 18, 18, 4 * N, n_pi_x=2.0, n_pi_y=1.0))
+    rng = np.random.default_rng(N)
+    shape = g.s["P"], g.s["nz"]
+    state = [rng.standard_normal(shape) + 1j * rng.standard_normal(shape) for _ in range(2)]
+    for s in (g, o):
+        s.set_state(*state)
+        s.velocity()
+    for i in range(6):
+        assert rel(g.get_field(i), o.get_field(i)) < 1e-13, i
+    g.close(), o.close()
+
+
 # solves of an odd base profile by conjugate parity blocks, at N odd and even, the smallest pair
 # counts, row pairs that fill whole and partial batches of every column group, the largest N: the
 # full inverses' results after one step.  2e-13 is the bound of the even profiles' blocks with
