@@ -40,5 +40,7 @@
                                                                   const h8_t*, const int*, int);                       \
     EXT template __global__ void k_p2s_mfma<(L <= 384 ? L : 384)>(const float2*, long, long, double2*, long, Dims,     \
                                                                   const h8_t*, int, int, Members);                     \
-    EXT template __global__ void k_p2s_dmfma<(L <= 384 ? L : 384)>(const double2*, long, long, double2*, long, Dims,   \
-                                                                   const double*, Members, int, int);
+    EXT template __global__ void k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunk>(const double2*, long, long, double2*, long, Dims, \
+                                                                          const double*, Members, int, int); \
+    EXT template __global__ void k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunkMany>(const double2*, long, long, double2*, long, Dims, \
+                                                                          const double*, Members, int, int);

@@ -31,11 +31,16 @@ typedef double v4d __attribute__((ext_vector_type(4)));
 
 constexpr int kPencils = 16;  // pencils per item: columns 0..15 real parts, 16..31 imaginary parts
 constexpr int kCols = 2 * kPencils;
-constexpr int kChunk = 32;    // samples q per chunk of the product's inner dimension, at most
+// samples q per chunk of the product's inner dimension, at most: 16 leave room for a fourth and
+// fifth block per CU, 32 halve a block's serial chunks.  k_p2s_dmfma with 32 / 16 (us): 256x97x256
+// (2064 blocks) 185 / 156, 128x129x128 (1040) 73 / 65, 128x65x128 (520) 29.2 / 27.8, 64x193x64 (264)
+// 71 / 57; 64x65x64 (132) 15.1 / 16.1, 32x129x32 (68) 21.2 / 23.3, 32x33x32 (34) 11.9 / 12.3: 16
+// where the blocks outnumber the compute units.
+constexpr int kChunk = 32, kChunkMany = 16;
 
 constexpr int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-template <int FN>
+template <int FN, int CH = kChunk>
 struct DShape {
     static constexpr int N = FN / 2, nz = N + 1, pz = FN + 1;
     static constexpr int RS = N / 2 + 1, RA = N / 2;  // sym rows p <= N/2, anti rows p < N/2
@@ -53,9 +58,9 @@ struct DShape {
     static constexpr int KP = ceil_div(N + 1, 4), KM = ceil_div(N, 4);  // k-steps of the tables over G+, G-
     // The chunks cover the samples q < N (N/4 k-steps of both G+ and G-); the centre sample
     // q = N (G+ only) is a rank-one update on the vector units.  Samples per chunk: the largest
-    // multiple of 4 dividing N, at most 32.
+    // multiple of 4 dividing N, at most CH.
     static constexpr int chunk_of(int n) {
-        for (int c = kChunk; c >= 4; c -= 4)
+        for (int c = CH; c >= 4; c -= 4)
             if (n % c == 0) return c;
         return 0;
     }
@@ -101,18 +106,18 @@ struct DShape {
 // wave runs the chunk's k-steps for its tile over both column tiles -- Q0 fragments serve h3
 // and h1, Q1 fragments h2 -- while the next chunk's samples are in flight.  The centre
 // sample q = N enters afterwards as a rank-one update of the accumulators on the vector
-// units.  Three blocks share a compute unit, so one block's products overlap another's
+// units.  Several blocks share a compute unit, so one block's products overlap another's
 // loads.  At the end the
 // sym waves write S to rows p and N - p of an LDS stage, the anti waves add A to row p and
 // subtract it from row N - p, and the rows leave as contiguous runs of the pencils.  A
 // centre row N/2 of its own runs on the vector units from the same LDS operands.
 // -------------------------------------------------------------------------------------
-template <int FN>
-__global__ __launch_bounds__(cheb_dmfma::DShape<FN>::NT, 3) void k_p2s_dmfma(
+template <int FN, int CH>
+__global__ __launch_bounds__((cheb_dmfma::DShape<FN, CH>::NT), 3) void k_p2s_dmfma(
     const double2* __restrict__ Z1, long zstride, long sY, double2* __restrict__ NL, long sNL, Dims d,
     const double* __restrict__ tab, Members mb, int nitems, int nyb) {
     using namespace cheb_dmfma;
-    using Sh = DShape<FN>;
+    using Sh = DShape<FN, CH>;
     constexpr int N = Sh::N, nz = Sh::nz, NT = Sh::NT, UPT = Sh::UPT, CHK = Sh::CHK, TPB = Sh::TPB, SR = Sh::SR;
     RPCF_LDS(double);
     __shared__ double cpart[2 * TPB][2][32];  // centre row: per wave, [N_eta, N_v][column]

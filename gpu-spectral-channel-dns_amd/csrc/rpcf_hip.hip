@@ -788,11 +788,17 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                     switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                              \
     case L:                                                                                                       \
-        if constexpr (L <= 384)                                                                                   \
-            k_p2s_dmfma<(L <= 384 ? L : 384)><<<cheb_dmfma::DShape<(L <= 384 ? L : 384)>::blocks(nitems),        \
-                                              cheb_dmfma::DShape<(L <= 384 ? L : 384)>::NT,                       \
-                                              cheb_dmfma::DShape<(L <= 384 ? L : 384)>::lds_bytes(), c->stream>>>( \
-                Y, yS, c->sY, c->NL, c->sNL, d, c->DT, mb, nitems, nyb);                                          \
+        if constexpr (L <= 384) {                                                                                 \
+            constexpr int LC = L <= 384 ? L : 384;                                                                \
+            auto run = [&](auto kernel, auto shape) {                                                             \
+                using Sh = decltype(shape);                                                                       \
+                kernel<<<Sh::blocks(nitems), Sh::NT, Sh::lds_bytes(), c->stream>>>(Y, yS, c->sY, c->NL, c->sNL, d, \
+                                                                                   c->DT, mb, nitems, nyb);       \
+            };                                                                                                    \
+            using namespace cheb_dmfma;                                                                           \
+            if (DShape<LC>::blocks(nitems) > c->ncu) run(k_p2s_dmfma<LC, kChunkMany>, DShape<LC, kChunkMany>{});  \
+            else run(k_p2s_dmfma<LC, kChunk>, DShape<LC>{});                                                      \
+        }                                                                                                         \
         break;
                         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
@@ -1354,7 +1360,8 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_velocity_tile<L, float2>, lim);           \
     allow_lds(k_p2s_mfma<(L <= 384 ? L : 384)>, lim);    \
     allow_lds(k_s2p_mfma<(L <= 384 ? L : 384)>, lim);    \
-    allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384)>, lim);
+    allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunk>, lim);   \
+    allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunkMany>, lim);
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
 #define RPCF_CASE(L)               \
