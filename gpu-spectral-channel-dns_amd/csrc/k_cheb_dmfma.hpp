@@ -361,7 +361,9 @@ __global__ __launch_bounds__((cheb_dmfma::DShape<FN, CH>::NT), 3) void k_p2s_dmf
 // matrix products with N a run-time number.  The runtime-plan FFT kernel it replaces (k_p2s_nl<0>;
 // RPCF_P2S_MFMA=0 keeps it) runs 3 to 5 passes over LDS with index arithmetic by run-time strides:
 // 62 us at 40x46x60 (N = 45) against 10.3 here, 281 at 100x151x100 (N = 150, where the product's N^2
-// meets the FFT's N log N) against 70.  Bound by the latency of a block's phases on small grids, by
+// meets the FFT's N log N) against 70.  A chunk's fragments are requested before its samples are
+// staged (3834 against 3880 us for 50 steps at 40x46x60; k_p2s_dmfma, with more registers held
+// meanwhile, gains nothing by it).  Bound by the latency of a block's phases on small grids, by
 // the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.3 of 72
 // TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
 // -------------------------------------------------------------------------------------
@@ -435,7 +437,6 @@ __global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restr
     const int slot = mb.ids[blockIdx.z], kx = blockIdx.y, ky0 = blockIdx.x * kPencils;
     const int nb = min(kPencils, d.ny - ky0);
     const double2* in = Z1 + slot * sY + (long)kx * pz * d.ny + ky0;
-    const double aphi = mb.mp[slot].aphi, beta = mb.mp[slot].beta;
     double2 sa[UPT][3], sb[UPT][3];
     auto load = [&](int c) {
 #pragma unroll
@@ -450,6 +451,8 @@ __global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restr
             }
         }
     };
+    load(0);  // before anything waits on memory
+    const double aphi = mb.mp[slot].aphi, beta = mb.mp[slot].beta;
     auto stage = [&](int c) {
 #pragma unroll
         for (int u = 0; u < UPT; u++) {
@@ -496,15 +499,15 @@ __global__ __launch_bounds__(128 * RT) void k_p2s_dmfma_n(const double2* __restr
     };
     const v4d zero4 = {0.0, 0.0, 0.0, 0.0};
     v4d accE[2] = {zero4, zero4}, accV[2] = {zero4, zero4};
-    load(0);
     for (int c = 0; c < sh.NCH; c++) {
-        stage(c);
+        // the chunk's fragments, in flight while its samples are staged
         double f0[kNChunk / 4], f1[kNChunk / 4];
 #pragma unroll
         for (int sl = 0; sl < kNChunk / 4; sl++) {
             f0[sl] = tq0[(long)(c * (kNChunk / 4) + sl) * 64];
             f1[sl] = tq1[(long)(c * (kNChunk / 4) + sl) * 64];
         }
+        stage(c);
         __syncthreads();
         if (c + 1 < sh.NCH) load(c + 1);
 #pragma unroll
