@@ -362,8 +362,8 @@ __global__ __launch_bounds__((cheb_dmfma::DShape<FN, CH>::NT), 3) void k_p2s_dmf
 // RPCF_P2S_MFMA=0 keeps it) runs 3 to 5 passes over LDS with index arithmetic by run-time strides:
 // 62 us at 40x46x60 (N = 45) against 10.3 here, 281 at 100x151x100 (N = 150, where the product's N^2
 // meets the FFT's N log N) against 70.  A chunk's fragments are requested before its samples are
-// staged (3834 against 3880 us for 50 steps at 40x46x60; k_p2s_dmfma, with more registers held
-// meanwhile, gains nothing by it).  Bound by the latency of a block's phases on small grids, by
+// staged (11.6 against 12.3 us at 40x46x60, 13.9 against 14.5 at 64x61x64; k_p2s_dmfma, with more
+// registers held meanwhile, gains nothing by it).  Bound by the latency of a block's phases on small grids, by
 // the matrix cores' FP64 rate, operand reads and fragment reads from L2 on long lengths (0.3 of 72
 // TFLOP/s, what a large FP64 matrix product reaches, at N = 150).
 // -------------------------------------------------------------------------------------

@@ -7,11 +7,11 @@
 // Element (r, j) of slot s of equation e sits at minv[(e*nslot + s)*nz*nz + j*nz + r],
 // so thread r of a solve reads consecutive addresses for every j.
 //
-// The matrix build, the inverse, the mean-flow update and the velocity recovery follow
-// the reference expressions in the same order as the oracle (no FP contraction), so they
-// reproduce it bit for bit from identical inputs.  The per-mode update regroups the
-// right-hand-side sums (three dot products per row, fused multiply-adds) and splits the
-// solves over four waves; it matches the oracle to rounding (about 1e-16 relative).
+// The matrix build, the inverse and the mean-flow update follow the reference expressions in the
+// same order as the oracle (no FP contraction), so they reproduce it bit for bit from identical
+// inputs.  The per-mode update regroups the right-hand-side sums (three dot products per row, fused
+// multiply-adds) and splits the solves over column groups, and velocity recovery sums its derivatives
+// over lanes; they match the oracle to rounding (about 1e-16 relative).
 #pragma once
 #include "rpcf_common.hpp"
 
