@@ -355,7 +355,7 @@ __global__ __launch_bounds__(256) void k_cheb_s2p_h(const double2* __restrict__ 
 // field.  Tile: TK kx columns of one
 // plane.  Y[f][kx][q][ky] -> W[f][q][s][kx] for kx < nxh (the x-Nyquist column is zero).
 // -------------------------------------------------------------------------------------
-template <int FN = 0, typename R = double>  // R: precision of Y, W and the FFT
+template <int FN = 0, typename R = double, bool TWL = true>  // R: precision of Y, W and the FFT; TWL: twiddles from LDS
 __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_inv(const cplx<R>* __restrict__ Y, long ystride, long sY, cplx<R>* __restrict__ W,
                                                   long wstride, long sW, Dims d, int planes, FftPlan pl, int TK, int ld,
                                                   const int* __restrict__ ids) {
@@ -405,7 +405,7 @@ __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_inv(const cplx<R>*
                 lds[kxi * ldl + s] = v;
             });
         FftPlan pll = pl;  // twiddles from an LDS copy behind the tile
-        copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
+        if constexpr (TWL) copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, +1, span_tile_max(FN), 1, true>(lds, ldl, nk, pll, tid, nthr);
         C2* out = W + f * wstride;
@@ -547,7 +547,7 @@ __device__ __forceinline__ void lamb_two_pass(double2* lds, const double2* W, lo
 // pairs of span rows.  W[6][pz][my][nxh] -> Z2[3][pz][my][hnx].  LDS: [6 RP][ld] sequences,
 // then (compiled lengths) the FN twiddles.
 // -------------------------------------------------------------------------------------
-template <int FN = 0, typename R = double>  // R: precision of W, Z2, the FFTs and the products
+template <int FN = 0, typename R = double, bool TWL = true>  // R: precision of W, Z2, the FFTs and the products
 __global__ __launch_bounds__(lamb_threads<R>(FN)) void k_lamb_phys(const cplx<R>* __restrict__ W, long wstride, long sW,
                                                    cplx<R>* __restrict__ Z2, long zstride, long sZ, int zld,
                                                    const double* __restrict__ meanU, long sPz, double fac, Dims d,
@@ -624,7 +624,7 @@ __global__ __launch_bounds__(lamb_threads<R>(FN)) void k_lamb_phys(const cplx<R>
         // the FFT twiddles from an LDS copy behind the sequences, so that no butterfly waits on
         // a global load
         FftPlan pll = pl;
-        copy_tw<FN>(lds + 6 * RP * lds_ld, pll, tid, nthr);
+        if constexpr (TWL) copy_tw<FN>(lds + 6 * RP * lds_ld, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, +1, 6 * lamb_pairs_max(FN), 1, true>(lds, lds_ld, 6 * nrp, pll, tid, nthr);
         // Ro U(y) is uniform in x and span, so it reaches only the (0,0) pencil of L_z, which
@@ -723,7 +723,7 @@ __global__ __launch_bounds__(256) void k_x_r2c(const double* __restrict__ phys, 
 // (source/transpose.cu:223-257).  Z2[g][q][s][kx] -> Z1[g][kx][q][ky]; blockIdx.z =
 // member * 3 + component.
 // -------------------------------------------------------------------------------------
-template <int FN = 0, typename R = double>  // R: precision of Z2, Z1 and the FFT
+template <int FN = 0, typename R = double, bool TWL = true>  // R: precision of Z2, Z1 and the FFT
 __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_fwd(const cplx<R>* __restrict__ Z2, long zstride, long sZ, int zld,
                                                   cplx<R>* __restrict__ Z1, long ostride, long sY, Dims d, int planes,
                                                   FftPlan pl, int TK, int ld, const int* __restrict__ ids,
@@ -777,7 +777,7 @@ __global__ __launch_bounds__(span_threads<R>(FN)) void k_span_fwd(const cplx<R>*
                 lds[kxi * ldl + s] = v;
             });
         FftPlan pll = pl;  // twiddles from an LDS copy behind the tile
-        copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
+        if constexpr (TWL) copy_tw<FN>(lds + TK * ldl, pll, tid, nthr);
         __syncthreads();
         fft_any<FN, -1, span_tile_max(FN), 1, true>(lds, ldl, nk, pll, tid, nthr);
         C2* out = Z1 + g * ostride;

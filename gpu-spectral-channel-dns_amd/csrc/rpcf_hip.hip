@@ -91,6 +91,7 @@ struct rpcf_ctx {
     int ld_zn = 0, ld_my = 0, ld_mx = 0, zld = 0;
     int mixed = 0;                   // 1: transform intermediates and x/span FFTs in FP32
     FftPlan pl_x{}, pl_y{}, pl_zp{}, pl_zn{};
+    int twl_x = 0, twl_y = 0;        // twiddles that the x and span transforms keep in LDS (0: read from the table)
     FftPlan pl_xf{}, pl_yf{};        // FP32 twiddles of the x and span plans (mixed form)
     float* twf = nullptr;
     int cap_x = 0, cap_y = 0, cap_zp = 0, cap_zn = 0;  // fft_capacity of each plan
@@ -589,9 +590,6 @@ int enq_velocity(rpcf_ctx* c, const int* ids, int n, bool cap = false) {
         cap);
 }
 
-// twiddles of a plan of length n in the LDS of the kernels that copy them there
-size_t tw_lds(int n) { return compiled_len(n) ? ct_tw_lds_len(n) : n; }
-
 // the padded s2p of nf fields (6 a member, or one) by k_s2p_dmfma: enough groups of 16 pencils for
 // four waves a block, fewer where that leaves compute units short of blocks, then groups of 8
 void s2p_product(rpcf_ctx* c, int nf, const double2* F, long fS, long sF, double2* Y, long yS, long sY, const int* ids) {
@@ -616,7 +614,7 @@ void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* 
     const bool two = two_pass<R>(d.my);  // a tile of its own
     const int TK = two ? span2_tile(d.my) : c->TK_inv, ld = c->ld_my;
     dim3 g((d.nxh + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + tw_lds(d.my));
+    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + c->twl_y);
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
@@ -625,7 +623,12 @@ void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* 
                 switch (d.my) {
                     RPCF_XY_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-                    default: k_span_inv<<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids);
+                    default: {
+                        auto run = [&](auto kernel) {
+                            kernel<<<g, kFftThreads, lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids);
+                        };
+                        c->twl_y ? run(k_span_inv<0, double, true>) : run(k_span_inv<0, double, false>);
+                    }
                 }
     }
 }
@@ -637,7 +640,7 @@ void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld,
     const bool two = two_pass<R>(d.my);
     const int TK = two ? span2_tile(d.my) : c->TK_fwd, ld = c->ld_my;
     dim3 g((d.hnx + TK - 1) / TK, planes, nf);
-    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + tw_lds(d.my));
+    const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + c->twl_y);
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)
@@ -646,7 +649,12 @@ void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld,
                 switch (d.my) {
                     RPCF_XY_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-                    default: k_span_fwd<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase);
+                    default: {
+                        auto run = [&](auto kernel) {
+                            kernel<<<g, kFftThreads, lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase);
+                        };
+                        c->twl_y ? run(k_span_fwd<0, double, true>) : run(k_span_fwd<0, double, false>);
+                    }
                 }
     }
 }
@@ -732,7 +740,7 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
         const bool two = two_pass<R>(d.mx);
         const int RP = two ? lamb2_pairs(d.mx) : c->RP, ld = c->ld_mx;
         dim3 g((d.my / 2 + RP - 1) / RP, d.pz, n);
-        const size_t lds = sizeof(C2) * (two ? 6 * RP * tp_ld(d.mx) : 6 * RP * ld + tw_lds(d.mx));
+        const size_t lds = sizeof(C2) * (two ? 6 * RP * tp_ld(d.mx) : 6 * RP * ld + c->twl_x);
         rc = launch(
             c, KID_LAMB,
             [&] {
@@ -744,10 +752,13 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                             switch (d.mx) {
                                 RPCF_XY_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
-                                default:
-                                    k_lamb_phys<<<g, kFftThreads, lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld,
-                                                                                    c->MEANU, c->sPz, c->fac, d, plx,
-                                                                                    RP, ld, mb);
+                                default: {
+                                    auto run = [&](auto kernel) {
+                                        kernel<<<g, kFftThreads, lds, c->stream>>>(W, wS, c->sW, Z2, zS, sZ, zld, c->MEANU,
+                                                                                   c->sPz, c->fac, d, plx, RP, ld, mb);
+                                    };
+                                    c->twl_x ? run(k_lamb_phys<0, double, true>) : run(k_lamb_phys<0, double, false>);
+                                }
                             }
                 }
             },
@@ -1318,6 +1329,8 @@ int init_ctx(rpcf_ctx* c) {
         });
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
+    c->twl_x = compiled_len(d.mx) ? ct_tw_lds_len(d.mx) : 0;
+    c->twl_y = compiled_len(d.my) ? ct_tw_lds_len(d.my) : 0;
     int tk_max = kSpanTile, rp_max = kLambPairs;  // the runtime-plan kernels size registers for these
 #define RPCF_CASE(L)                          \
     if (d.my == L) tk_max = span_tile_max(L); \
@@ -1325,19 +1338,28 @@ int init_ctx(rpcf_ctx* c) {
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     c->TK_inv = pick_tile(tk_max, d.my, c->cap_y, lim3, [&](int t) {
-        return sizeof(double2) * ((size_t)t * c->ld_my + tw_lds(d.my));
+        return sizeof(double2) * ((size_t)t * c->ld_my + c->twl_y);
     });
     c->TK_fwd = c->TK_inv;
     c->RP = pick_tile(rp_max, 6 * d.mx, c->cap_x, lim3, [&](int t) {
-        return sizeof(double2) * (6 * (size_t)t * c->ld_mx + tw_lds(d.mx));
+        return sizeof(double2) * (6 * (size_t)t * c->ld_mx + c->twl_x);
     });
+    // a runtime plan's twiddles, where they cost no tile: mx = 500 and 540 would be left without a row
+    // pair, my from 1728 on without a column, and a narrower tile is the slower way (k_span_inv,
+    // 8 columns without the copy against 7 with it at my = 400, 6 against 5 at 500 and 2 against 1
+    // at 1620, 32 modes: 21, 41 and 49 us against 28, 52 and 70)
+    if (!c->twl_y && sizeof(double2) * ((size_t)c->TK_inv * c->ld_my + d.my) <= (size_t)lim3) c->twl_y = d.my;
+    if (!c->twl_x && sizeof(double2) * (6 * (size_t)c->RP * c->ld_mx + d.mx) <= (size_t)lim3) c->twl_x = d.mx;
     if (!c->TB_s2p || !c->TB_nl || !c->TK_inv || !c->RP)
         return fail(c, RPCF_EINVAL, "grid too large for the LDS tiles (limit %d bytes)", lim);
     allow_lds(k_cheb_s2p<1>, lim);
     allow_lds(k_cheb_s2p<0>, lim);
     allow_lds(k_span_inv<0>, lim);
+    allow_lds(k_span_inv<0, double, false>, lim);
     allow_lds(k_span_fwd<0>, lim);
+    allow_lds(k_span_fwd<0, double, false>, lim);
     allow_lds(k_lamb_phys<0>, lim);
+    allow_lds(k_lamb_phys<0, double, false>, lim);
     allow_lds(k_p2s_nl<0>, lim);
 #define RPCF_CASE(L)                  \
     allow_lds(k_cheb_s2p<1, L>, lim); \
@@ -1852,11 +1874,12 @@ int enq_spec_to_phys(rpcf_ctx* c, const double2* f, double2* y, double2* w, doub
                 k_cheb_s2p<0><<<g, kFftThreads, lds, c->stream>>>(f, 0, 0, y, 0, 0, d, plz, tw4, TB, ld, c->ids_zero);
     }
     span_inv<double>(c, 1, y, 0, 0, w, 0, 0, planes, c->pl_y, c->ids_zero);
+    const int twl = c->twl_x ? c->twl_x : d.mx;  // (one sequence a row pair: the twiddles always fit)
     const int RP1 = pick_tile(kC2rRows, d.mx, c->cap_x, c->lds_limit / 3, [&](int t) {
-        return sizeof(double2) * ((size_t)t * c->ld_mx + tw_lds(d.mx));
+        return sizeof(double2) * ((size_t)t * c->ld_mx + twl);
     });
     dim3 g3((d.my / 2 + RP1 - 1) / RP1, planes);
-    const size_t lds3 = sizeof(double2) * (RP1 * c->ld_mx + tw_lds(d.mx));
+    const size_t lds3 = sizeof(double2) * (RP1 * c->ld_mx + twl);
     switch (d.mx) {
 #define RPCF_CASE(L) case L: k_x_c2r<L><<<g3, kFftThreads, lds3, c->stream>>>(w, ph, d, c->pl_x, RP1, c->ld_mx); break;
         RPCF_FFT_LENGTHS(RPCF_CASE)

@@ -177,3 +177,26 @@ def test_odd_profile_solves(N, precision, monkeypatch):
     if precision == 2:
         b = step(0, False)
         assert all(np.array_equal(x, y) for x, y in zip(a, b))
+
+
+# x and span lengths whose run-time plan has no room in LDS for its twiddles beside the tile, and
+# the longest that have: one row pair or column, and a few.  The library's bars, as above.
+@pytest.mark.parametrize("mx,my", [(486, 10), (500, 18), (540, 12), (12, 400), (24, 1000), (18, 1620), (12, 1728), (6, 3240)])
+def test_long_lengths(mx, my):
+    prm = rpcf.make_params(mx, my, 24, n_pi_x=2.0, n_pi_y=1.0, Re=900.0, Ro=0.1, dt=0.002)
+    g, o = pair(prm)
+    rng = np.random.default_rng(mx + my)
+    shape = g.s["P"], g.s["nz"]
+    f = [(rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / (1.0 + np.arange(g.s["nz"])) ** 2
+         for _ in range(6)]
+    for s in (g, o):
+        for i in range(6):
+            s.set_field(i, f[i])
+        s.nonlinear()
+    for a, b in zip(g.get_nonlinear(), o.get_nonlinear()):
+        assert rel(a, b) < 1e-12
+    p, q = g.spec_to_phys(f[0]), o.spec_to_phys(f[0])
+    assert rel(p, q) < 1e-13
+    f = rng.standard_normal(q.shape)
+    assert rel(g.phys_to_spec(f), o.phys_to_spec(f)) < 1e-13
+    g.close(), o.close()
