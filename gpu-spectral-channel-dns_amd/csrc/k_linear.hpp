@@ -390,7 +390,7 @@ struct LinState {
     const float2* minvf;   // [nslot][np][nz] mixed form: the high parts of the eta blocks (FP32)
     double qw_target_re, qw_target_im;  // flow-rate target (flow_control)
     int flow_control;
-    int parity;           // MemberParams::parity
+    int parity;           // 1: solve with the parity blocks, 2: with the blocks and remainders
 };
 
 // -------------------------------------------------------------------------------------
@@ -694,36 +694,16 @@ __device__ __forceinline__ double2 bf16x2_to_double2(unsigned w) {
     return make_double2((double)__uint_as_float(w << 16), (double)__uint_as_float(w & 0xffff0000u));
 }
 
-// the real part of m times the u's, plus i times its imaginary part times the w's
-__device__ __forceinline__ void gemv_acc_split(double2 m, double2 u0, double2 u1, double2 w0, double2 w1, double* a) {
-    a[0] = fma(m.x, u0.x, fma(-m.y, w0.y, a[0]));
-    a[1] = fma(m.x, u0.y, fma(m.y, w0.x, a[1]));
-    a[2] = fma(m.x, u1.x, fma(-m.y, w1.y, a[2]));
-    a[3] = fma(m.x, u1.y, fma(m.y, w1.x, a[3]));
-}
-
-// A parity block with its remainders as k_parity_blocks stores them ([cols][rows], column-major)
-struct BlockColumns {
-    static constexpr int batch = kGemvBatch;
-    const double2* __restrict__ M;
-    const unsigned* __restrict__ E;
-    int rows;
-    template <bool CORR>
-    __device__ __forceinline__ void load(int c, int r, double2* m, unsigned* e) const {
-        *m = M[(long)c * rows + r];
-        if (CORR) *e = E[(long)c * rows + r];
-    }
-};
-
-// The same with a rows x cols matrix whose rows r < split take the vectors xa and the others
-// xb; columns from j0.  With ODD only the real part of an entry multiplies that vector and the
-// imaginary part the other one.  With CORR the remainders E multiply the vectors the other way
-// round, and each column adds M x + E x' in that order.
-template <bool CORR, bool ODD, typename Columns>
-__device__ __forceinline__ void gemv_sel(const Columns M, const double2* xa0, const double2* xa1, const double2* xb0,
+// The same with a rows x cols matrix (column-major, M[c*rows + r]) whose rows r < split
+// take the vectors xa and the others xb; columns from j0.  With CORR the remainders E (same
+// layout, BF16 pairs) multiply the other vectors (rows r < split xb, the others xa), and
+// each column adds M x + E x' in that order.
+template <bool CORR>
+__device__ __forceinline__ void gemv_sel(const double2* __restrict__ M, const unsigned* __restrict__ E,
+                                         const double2* xa0, const double2* xa1, const double2* xb0,
                                          const double2* xb1, int rows, int cols, int split, double2* part, int tid,
                                          int nthr, double2* y0, double2* y1, int j0) {
-    constexpr int B = Columns::batch;
+    constexpr int B = kGemvBatch;
     const int G = nthr / rows;
     const int g = tid / rows, r = tid - g * rows;
     const double2* x0 = r < split ? xa0 : xb0;
@@ -731,38 +711,41 @@ __device__ __forceinline__ void gemv_sel(const Columns M, const double2* xa0, co
     const double2* o0 = r < split ? xb0 : xa0;
     const double2* o1 = r < split ? xb1 : xa1;
     double a[4] = {0.0, 0.0, 0.0, 0.0};
-    auto add = [&](double2 m, unsigned e, double2 u0, double2 u1, double2 w0, double2 w1) {
-        if (ODD) {
-            gemv_acc_split(m, u0, u1, w0, w1, a);
-            if (CORR) gemv_acc_split(bf16x2_to_double2(e), w0, w1, u0, u1, a);
-        } else {
-            gemv_acc(m, u0, u1, a);
-            if (CORR) gemv_acc(bf16x2_to_double2(e), w0, w1, a);
-        }
-    };
     if (g < G) {
         int j = j0 + g;
         for (; j + G * (B - 1) < cols; j += G * B) {
             double2 m[B];
             unsigned e[B];
 #pragma unroll
-            for (int u = 0; u < B; u++) M.template load<CORR>(j + G * u, r, m + u, e + u);
+            for (int u = 0; u < B; u++) {
+                m[u] = M[(long)(j + G * u) * rows + r];
+                if (CORR) e[u] = E[(long)(j + G * u) * rows + r];
+            }
 #pragma unroll
             for (int u = 0; u < B; u++) {
-                const int jj = j + G * u;
-                add(m[u], e[u], x0[jj], x1[jj], o0[jj], o1[jj]);
+                gemv_acc(m[u], x0[j + G * u], x1[j + G * u], a);
+                if (CORR) gemv_acc(bf16x2_to_double2(e[u]), o0[j + G * u], o1[j + G * u], a);
             }
         }
         if (j < cols) {
             double2 m[B];
             unsigned e[B];
 #pragma unroll
-            for (int u = 0; u < B; u++) M.template load<CORR>(min(j + G * u, cols - 1), r, m + u, e + u);
+            for (int u = 0; u < B; u++) {
+                m[u] = M[(long)min(j + G * u, cols - 1) * rows + r];
+                if (CORR) e[u] = E[(long)min(j + G * u, cols - 1) * rows + r];
+            }
 #pragma unroll
             for (int u = 0; u < B; u++) {
                 const int jj = min(j + G * u, cols - 1);
                 const double k = j + G * u < cols ? 1.0 : 0.0;
-                add(m[u], e[u], zmulr(x0[jj], k), zmulr(x1[jj], k), zmulr(o0[jj], k), zmulr(o1[jj], k));
+                const double2 u0 = x0[jj], u1 = x1[jj];
+                gemv_acc(m[u], make_double2(u0.x * k, u0.y * k), make_double2(u1.x * k, u1.y * k), a);
+                if (CORR) {
+                    const double2 w0 = o0[jj], w1 = o1[jj];
+                    gemv_acc(bf16x2_to_double2(e[u]), make_double2(w0.x * k, w0.y * k),
+                             make_double2(w1.x * k, w1.y * k), a);
+                }
             }
         }
         part[tid] = make_double2(a[0], a[1]);
@@ -865,20 +848,10 @@ __device__ __forceinline__ void gemv_sel_hilo(const float2* __restrict__ Mf, con
 // eta system is well conditioned), so only the v blocks keep remainders (same layout as H):
 // the solves read (2 x 16 + 4)/64 of the full inverses' bytes and keep their results.
 //
-// With an odd base profile (U = c1 y) the imaginary parts of A change sign under the
-// reflection, A R = Q conj(A), so M[j][i'] = (-1)^j s conj(M[j][i]) and
-//   x_j = sum_p Re H (b_i + (-1)^j s b_i') + i Im H (b_i - (-1)^j s b_i')
-//             + Re E (b_i - (-1)^j s b_i') + i Im E (b_i + (-1)^j s b_i')
-// with H, E = (M[j][i] +- (-1)^j s conj(M[j][i']))/2: the same two combined sides, the same
-// bytes and the same remainders (v only).  At 256x97x256 (Couette) k_lin_solve went from 1033 us
-// with the full inverses to 679, at 64x65x64 in a group with two channel members from 134 to 114.
-//
 // The mixed form (bar 1e-6) solves with the blocks alone, the eta blocks split into an FP32
 // high part and a BF16 low part (hi + lo = H to ~2^-33 relative, 12 of 16 bytes): the eta
 // system is well conditioned, so its solve stays within ~1e-10 of the FP64 blocks'; the v
-// system (condition ~5e7 at 128x129x128) keeps FP64 blocks.  An odd profile's mixed
-// solves read the full inverses: its slot has no room for eta's FP64 blocks, and a last-bit
-// change of the state moves the FP32 transforms' rounding by 4e-9.
+// system (condition ~5e7 at 128x129x128) keeps FP64 blocks.
 // minve: the v remainders (FP64 form, minvf null) or the eta low parts (mixed form, with
 // minvf the eta high parts); both may be null.
 // -------------------------------------------------------------------------------------
@@ -887,36 +860,9 @@ __device__ __forceinline__ unsigned bf16_bits(double x) {
     u += 0x7fffu + ((u >> 16) & 1u);  // round to nearest even
     return u >> 16;
 }
-__device__ __forceinline__ unsigned bf16x2_bits(double2 w) { return bf16_bits(w.x) | (bf16_bits(w.y) << 16); }
-
-// H and E of an odd profile from a = M[j][i], b = M[j][i'], sg = (-1)^j s (a centre row: b = a)
-__device__ __forceinline__ void parity_split_odd(double2 a, double2 b, double sg, double2* h, double2* e) {
-    *h = make_double2(0.5 * (a.x + sg * b.x), 0.5 * (a.y - sg * b.y));
-    *e = make_double2(0.5 * (a.x - sg * b.x), 0.5 * (a.y + sg * b.y));
-}
-
-// The v block and its remainders of an odd profile formed on the way from the full inverse, bit
-// for bit as k_parity_blocks stores them: the FP64 form without remainders in its slots
-// (precision 2), whose odd-profile members solve as precision 0 does.  Columns p >= j0/2 only:
-// rows i = p + j0/2 and i' = N + j0/2 - p, sign +1.  It reads all of the v
-// inverse: 256x97x256 takes 2.82 ms a step, 2.98 with
-// the full inverses, 2.62 from stored blocks.
-struct OddColumns {
-    static constexpr int batch = 2;  // two entries per column
-    const double2* __restrict__ M;
-    int n, ne, half;  // half = j0/2
-    template <bool CORR>
-    __device__ __forceinline__ void load(int p, int r, double2* m, unsigned* e) const {
-        const int j = r < ne ? 2 * r : 2 * (r - ne) + 1;
-        double2 w;
-        parity_split_odd(M[(long)(p + half) * n + j], M[(long)(n - 1 + half - p) * n + j], r < ne ? 1.0 : -1.0, m, &w);
-        if (CORR) *e = bf16x2_bits(w);
-    }
-};
-
 __global__ void k_parity_blocks(const double2* __restrict__ minv, double2* __restrict__ minvh,
                                 unsigned* __restrict__ minve, float2* __restrict__ minvf,
-                                const int4* __restrict__ pairs, int np, int odd, Dims d) {
+                                const int4* __restrict__ pairs, int np, Dims d) {
     const int slot = blockIdx.x, eq = blockIdx.y, n = d.nz, ne = d.N / 2 + 1;
     const double2* M = minv + ((long)eq * d.nslot + slot) * n * n;  // M[j][i] at i*n + j
     // the mixed form keeps no FP64 eta blocks (its solves read the split parts)
@@ -931,9 +877,7 @@ __global__ void k_parity_blocks(const double2* __restrict__ minv, double2* __res
         const bool even = r < ne;
         const int j = even ? 2 * r : 2 * (r - ne) + 1;
         double2 v, w;
-        if (odd) {
-            parity_split_odd(M[(long)q.x * n + j], M[(long)q.y * n + j], even ? (double)q.z : -(double)q.z, &v, &w);
-        } else if (q.x == q.y) {
+        if (q.x == q.y) {
             const double2 a = M[(long)q.x * n + j];
             v = even ? a : make_double2(0.0, 0.0);
             w = even ? make_double2(0.0, 0.0) : a;
@@ -944,11 +888,11 @@ __global__ void k_parity_blocks(const double2* __restrict__ minv, double2* __res
             w = make_double2(0.5 * (a.x - sg * b.x), 0.5 * (a.y - sg * b.y));
         }
         if (Hm) Hm[e] = v;
-        if (Em) Em[e] = bf16x2_bits(w);
+        if (Em) Em[e] = bf16_bits(w.x) | (bf16_bits(w.y) << 16);
         if (Fm) {
             const float2 hi = make_float2((float)v.x, (float)v.y);
             Fm[e] = hi;
-            Lm[e] = bf16x2_bits(make_double2(v.x - (double)hi.x, v.y - (double)hi.y));
+            Lm[e] = bf16_bits(v.x - (double)hi.x) | (bf16_bits(v.y - (double)hi.y) << 16);
         }
     }
 }
@@ -999,14 +943,14 @@ __device__ __forceinline__ void gemv_t0_reflect(const double* __restrict__ T0t, 
 }
 
 // x = M b for the two right-hand sides rhs[0..1][nz] of a slot: with the full inverse M, or,
-// for a member with an even or odd base profile, with its parity blocks H (k_parity_blocks): the
+// for a member with an even base profile, with its parity blocks H (k_parity_blocks): the
 // combined sides b_i + s b_i' and b_i - s b_i' per row pair, then one nz x np GEMV whose even
-// rows take the first and odd rows the second.  Em: with the remainders; Hf: the blocks as FP32
-// high parts Hf and BF16 low parts Em; odd profile without Hm: the block and its remainders formed from M.  b vanishes
+// rows take the first and odd rows the second (parity 2 and Em given: and the remainders E
+// the other; Hf given: the blocks as FP32 high parts Hf and BF16 low parts Em).  b vanishes
 // on the rows below j0 (an even count: whole row pairs), whose columns are skipped.  Thread
 // r < nz returns x at coefficient *jrow.  Every thread of the block calls it (it synchronises).
 __device__ __forceinline__ void solve_slot(const double2* M, const double2* Hm, const unsigned* Em, const float2* Hf,
-                                           const int4* pairs, int np, int parity, bool corr, double2 (*rhs)[256],
+                                           const int4* pairs, int np, int parity, double2 (*rhs)[256],
                                            double2 (*bc)[2][128], double2* part, int n, int N, int tid, int nthr,
                                            double2* y0, double2* y1, int* jrow, int j0) {
     if (!parity) {
@@ -1030,26 +974,12 @@ __device__ __forceinline__ void solve_slot(const double2* M, const double2* Hm, 
     }
     __syncthreads();
     const int ne = N / 2 + 1;
-    auto gemv = [&](auto corr_, auto odd_, auto columns) {
-        gemv_sel<corr_, odd_>(columns, bc[0][0], bc[1][0], bc[0][1], bc[1][1], n, np, ne, part, tid, nthr, y0, y1,
-                              j0 / 2);
-    };
-    const BlockColumns H{Hm, Em, n};
-    const std::true_type yes;
-    const std::false_type no;
     if (Hf)
         gemv_sel_hilo(Hf, Em, bc[0][0], bc[1][0], bc[0][1], bc[1][1], n, np, ne, part, tid, nthr, y0, y1, j0 / 2);
-    else if (parity == kParityOdd && !Hm)
-        gemv(yes, yes, OddColumns{M, n, ne, j0 / 2});
-    else if (parity == kParityOdd) {
-        if (corr)
-            gemv(yes, yes, H);
-        else
-            gemv(no, yes, H);
-    } else if (corr)
-        gemv(yes, no, H);
+    else if (parity == 2 && Em)
+        gemv_sel<true>(Hm, Em, bc[0][0], bc[1][0], bc[0][1], bc[1][1], n, np, ne, part, tid, nthr, y0, y1, j0 / 2);
     else
-        gemv(no, no, H);
+        gemv_sel<false>(Hm, Em, bc[0][0], bc[1][0], bc[0][1], bc[1][1], n, np, ne, part, tid, nthr, y0, y1, j0 / 2);
     *jrow = tid < ne ? 2 * tid : 2 * (tid - ne) + 1;
 }
 
@@ -1192,14 +1122,12 @@ __global__ __launch_bounds__(kSolveThreads, 6) void k_lin_solve(double2* __restr
     }
     __syncthreads();
     const long nh = (long)n * np;
-    const bool odd = st.parity == kParityOdd;
     {
         double2 y0, y1;
         int j;
         const unsigned* Ev = st.minve && !st.minvf ? st.minve + (long)slot * nh : nullptr;
-        solve_slot(Mv, odd && !Ev ? nullptr : st.minvh + (long)slot * nh, Ev, nullptr, pairs, np, st.parity,
-                   odd || (st.parity == kParityEvenRem && Ev), rhs, bc, &part[0][0], n, d.N, r, blockDim.x, &y0, &y1,
-                   &j, 4);
+        solve_slot(Mv, st.minvh + (long)slot * nh, Ev, nullptr, pairs, np, st.parity, rhs, bc, &part[0][0], n, d.N,
+                   r, blockDim.x, &y0, &y1, &j, 4);
         if (r < n) vnew[0][j] = y0, vnew[1][j] = y1;
     }
     __syncthreads();
@@ -1229,9 +1157,9 @@ __global__ __launch_bounds__(kSolveThreads, 6) void k_lin_solve(double2* __restr
     double2 e0, e1;
     int je;
     // eta: the FP64 blocks without remainders, or (mixed form) their FP32 + BF16 split
-    const bool split = st.minvf && st.parity == kParityEven;
+    const bool split = st.minvf && st.parity == 1;
     solve_slot(Mo, split ? nullptr : st.minvh + ((long)d.nslot + slot) * nh, split ? st.minve + (long)slot * nh : nullptr,
-               split ? st.minvf + (long)slot * nh : nullptr, pairs + np, np, st.parity, false, rhs, bc, &part[0][0], n, d.N,
+               split ? st.minvf + (long)slot * nh : nullptr, pairs + np, np, st.parity, rhs, bc, &part[0][0], n, d.N,
                r, blockDim.x, &e0, &e1, &je, 2);
     if (r < n) {
         st.se[po0 + je] = e0;

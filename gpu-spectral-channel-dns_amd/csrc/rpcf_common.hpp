@@ -2,8 +2,6 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
-#include <type_traits>
-
 // Grid sizes in the reference's naming (include/data.h:189-334, source/data.cpp:3-14):
 // mx, my padded x / span lengths; nx = mx/3*2, ny = my/3*2 kept modes; nz = mz/4+1
 // Chebyshev coefficients, N = nz-1; pz = mz/2+1 = 2N+1 padded wall-normal points;
@@ -29,15 +27,12 @@ __host__ __device__ __forceinline__ int ky_of_span(const Dims& d, int s) {
 // Scalars of one simulation (slot) of a group: wavenumber scales aphi = Lx/2, beta = Lz/2
 // (include/data.h:321-322), Re, dt, rotation number, the flow-rate target (bulk of u0 at
 // set_state) and the flow-control switch.
-constexpr int kParityNone = 0;     // the full inverses
-constexpr int kParityEven = 1;     // even base profile: their parity blocks
-constexpr int kParityEvenRem = 2;  // and the blocks' BF16 remainders (the full inverse's values)
-constexpr int kParityOdd = 3;      // odd base profile: parity blocks with the v remainders
 struct MemberParams {
     double aphi, beta, Re, dt, Ro;
     double q_re, q_im;
     int flow_control;
-    int parity;  // how the solves read the inverses: kParity..
+    int parity;  // even base profile: 1, the solves read the parity blocks of the inverses;
+                 // 2, the parity blocks and their BF16 remainders (the full inverse's values)
 };
 
 // Member addressing of one grouped launch: launch member j runs slot ids[j]; a per-slot

@@ -121,8 +121,8 @@ struct rpcf_ctx {
     double2* Z2 = nullptr;    // [3][pz][my][zld], zld = hnx rounded up to 8 (128-byte rows; FP32: 16)
     double2* WL = nullptr;    // [5][P][nz] operator products of the linear right-hand sides
     double2* MINV = nullptr;  // [2][nslot][nz*nz] inverses, column-major
-    double2* MINVH = nullptr; // [2][nslot][np][nz] parity blocks of the inverses (even and odd base
-                              // profiles; the mixed form keeps the v blocks only, [1][nslot][np][nz])
+    double2* MINVH = nullptr; // [2][nslot][np][nz] parity blocks of the inverses (even base profiles;
+                              // the mixed form keeps the v blocks only, [1][nslot][np][nz])
     unsigned* MINVE = nullptr; // [nslot][np][nz] BF16 (re, im): the v blocks' remainders (FP64 form)
                                // or the eta blocks' low parts (mixed form)
     float2* MINVF = nullptr;   // [nslot][np][nz] the eta blocks' FP32 high parts (mixed form)
@@ -205,8 +205,8 @@ struct SlotSizes {
     }
 };
 
-// Inverses: the full ones (the mean flow's slot, base profiles neither even nor odd, and the
-// source of the rest), their parity blocks (even and odd base profiles), and in the FP64 form the BF16 remainders
+// Inverses: the full ones (the mean flow's slot, odd base profiles, and the source of the
+// rest), their parity blocks (even base profiles), and in the FP64 form the BF16 remainders
 // of the v blocks, which restore the full inverses' results (the blocks alone agree with them
 // to ~1e-11 after a step, enough for the mixed form only; the eta blocks need none); in the
 // mixed form the eta blocks also as FP32 high and BF16 low parts, which its solves read.
@@ -1418,19 +1418,19 @@ int init_ctx(rpcf_ctx* c) {
 // state, fields and history are cleared.
 // Whether solves that give the full inverses' results are faster from the parity blocks: these
 // read 9/16 of the bytes, but combine the row pairs first (a barrier and 1.5 us).  k_lin_solve,
-// full inverses against blocks (us, either profile): 32x33x32 8.2 / 9.7, 64x49x64 22 / 24.4,
+// full inverses against blocks (us): 32x33x32 8.2 / 9.7, 64x49x64 22 / 24.4,
 // 128x33x128 57.7 / 61.8 (0.15 GB of full inverses); 128x41x128 76.3 / 74.5 (0.23 GB, more than
 // the last-level cache keeps), 128x49x128 97 / 83, 32x65x32 12.5 / 12.9, 48x65x48 17.9 / 16.1,
 // 16x101x16 13.2 / 12.9, 128x65x128 154 / 112.
 bool blocks_pay(const Dims& d) { return d.N >= 64 || 32.0 * d.nslot * d.nz * d.nz > 0.2e9; }
 
 // parity blocks of a slot's inverses (k_parity_blocks), on the context stream
-int build_parity_blocks(rpcf_ctx* c, int slot, int parity) {
+int build_parity_blocks(rpcf_ctx* c, int slot) {
     const Dims d = c->d;
     k_parity_blocks<<<dim3(d.nslot, 2), 256, 0, c->stream>>>(c->MINV + slot * c->sM, c->MINVH + slot * c->sMH,
                                                              c->MINVE ? c->MINVE + slot * c->sME : nullptr,
                                                              c->MINVF ? c->MINVF + slot * c->sME : nullptr,
-                                                             c->PAIRS, c->npair, parity == kParityOdd, d);
+                                                             c->PAIRS, c->npair, d);
     const hipError_t e = hipGetLastError();
     return e == hipSuccess ? RPCF_OK : fail(c, RPCF_EDEVICE, "k_parity_blocks: %s", hipGetErrorString(e));
 }
@@ -1456,20 +1456,13 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     sh.mp.q_re = sh.mp.q_im = 0.0;
     sh.mp.flow_control = prm->flow_control;
     // an even base profile U(y) (no linear part) keeps the collocation systems symmetric under
-    // y -> -y, an odd one (linear part only) up to conjugation, so the solves can use the parity
-    // blocks of the inverses: in the FP64 form where they pay, with the remainders that give the
-    // full inverses' values; in the others, for even profiles, alone.  An odd profile's blocks
-    // stop at N = 160: the BF16 rounding of its remainders leaves 1.3e-13 of a step there and
-    // 2e-12 at N = 250.  RPCF_FULL_INVERSE=1 keeps the full inverses.
+    // y -> -y, so the solves can use the parity blocks of the inverses: in the FP64 form where they
+    // pay, with the remainders that give the full inverses' values; in the others alone.
+    // RPCF_FULL_INVERSE=1 keeps the full inverses.
     const char* fe = getenv("RPCF_FULL_INVERSE");
     const bool full = fe && atoi(fe) != 0;
-    const double* up = prm->u_profile;
-    const int prec = c->shape.precision;
-    sh.mp.parity = kParityNone;
-    if (!full && up[1] == 0.0)
-        sh.mp.parity = prec != 0 ? kParityEven : blocks_pay(d) ? kParityEvenRem : kParityNone;
-    else if (!full && up[0] == 0.0 && up[2] == 0.0 && prec != 1 && blocks_pay(d) && d.N <= 160)
-        sh.mp.parity = kParityOdd;
+    sh.mp.parity = 0;
+    if (!full && prm->u_profile[1] == 0.0) sh.mp.parity = c->shape.precision != 0 ? 1 : blocks_pay(d) ? 2 : 0;
 
     std::vector<double> U(nz), dU(nz), ddU(nz), mU(d.pz);
     rpcf_host::base_profile(d.nz, prm->u_profile, U.data(), dU.data(), ddU.data());
@@ -1529,7 +1522,7 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
             a.u_profile[2] == prm->u_profile[2]) {
             HIPCHK(c, hipMemcpyAsync(minv, c->MINV + s2 * c->sM, sizeof(double2) * 2 * (size_t)d.nslot * per,
                                      hipMemcpyDeviceToDevice, c->stream));
-            if (sh.mp.parity) RCCHK(build_parity_blocks(c, slot, sh.mp.parity));
+            if (sh.mp.parity) RCCHK(build_parity_blocks(c, slot));
             HIPCHK(c, hipStreamSynchronize(c->stream));
             c->matrix_cache_hits++;
             sh.configured = 1;
@@ -1566,7 +1559,7 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     (void)hipFree(work);
     (void)hipFree(status);
     if (!rc && hstatus) rc = fail(c, RPCF_EINVAL, "%d singular collocation matrices", hstatus);
-    if (!rc && sh.mp.parity) rc = build_parity_blocks(c, slot, sh.mp.parity);
+    if (!rc && sh.mp.parity) rc = build_parity_blocks(c, slot);
     if (!rc && hipStreamSynchronize(c->stream) != hipSuccess) rc = fail(c, RPCF_EDEVICE, "parity blocks failed");
     if (!rc) sh.configured = 1;
     return rc;

@@ -200,3 +200,22 @@ def test_long_lengths(mx, my):
     f = rng.standard_normal(q.shape)
     assert rel(g.phys_to_spec(f), o.phys_to_spec(f)) < 1e-13
     g.close(), o.close()
+
+
+# profiles that are not even keep both FP64 inverses whole at every size: the state after a step is,
+# bit for bit, that of RPCF_FULL_INVERSE=1
+@pytest.mark.parametrize("N,mx", [(32, 24), (64, 24), (75, 24), (96, 24), (128, 24), (160, 24), (40, 192)])
+@pytest.mark.parametrize("profile", [(0.0, 1.0, 0.0), (0.5, 0.5, 0.0)])
+@pytest.mark.parametrize("precision", [0, 2])
+def test_other_profiles_solve_with_the_full_inverses(N, mx, profile, precision, monkeypatch):
+    def step(full):
+        monkeypatch.setenv("RPCF_FULL_INVERSE", str(full))
+        prm = rpcf.make_params(mx, mx, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=1300.0, Ro=0.1, dt=0.002,
+                               u_profile=profile, precision=precision)
+        with rpcf.Simulation(rpcf.HIP_LIB, prm) as s:
+            s.set_state(*rpcf.seed_state(s.dll, prm, 0, 0.1, 4, 24, 5.0 / 6.0, True))
+            s.bootstrap()
+            return s.get_state()
+
+    for a, b in zip(step(0), step(1)):
+        assert np.array_equal(a, b)
