@@ -257,9 +257,12 @@ __global__ __launch_bounds__((cheb_dmfma::DShape<FN, CH>::NT), 3) void k_p2s_dmf
                 accV[ct] = __builtin_amdgcn_mfma_f64_16x16x4f64(f1[sl], bop(1, 1 - pm0, sl, ct), accV[ct], 0, 0, 0);
         }
         if (centre) {
-            // column tid % 32, samples qq = tid / 32 + (NT / 32) j of the chunk
+            // column tid % 32; of each BASE samples, those of index tid / 32 + HW j, whatever the
+            // chunk: the order of this sum is the same in the forms of both chunk lengths
+            constexpr int HW = NT / 32, BASE = DShape<FN>::CHK;
+            static_assert(!Sh::CENTRE || BASE % CHK == 0, "chunks of one form tile those of the other");
             const int col = tid & 31;
-            for (int qq = tid >> 5; qq < CHK; qq += NT / 32) {
+            for (int qq = ((tid >> 5) + HW - c * CHK % BASE % HW) % HW; qq < CHK; qq += HW) {
                 const int q = c * CHK + qq;
                 const double w0 = ctr[q];
                 cE = fma(w0, lds[(0 * CHK + qq) * kCols + col], cE);

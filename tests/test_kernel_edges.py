@@ -219,3 +219,51 @@ def test_other_profiles_solve_with_the_full_inverses(N, mx, profile, precision, 
 
     for a, b in zip(step(0), step(1)):
         assert np.array_equal(a, b)
+
+
+# a member alone and beside others whose blocks together outnumber the compute units (16-sample
+# chunks in the padded p2s, wider blocks in the padded s2p): the same bits.  N with and without a
+# compiled plan, with the centre row N/2 in a tile of its own (32, 96, 128, 192) and not.
+@pytest.mark.parametrize("N,mx,my,members", [(24, 96, 96, 2), (32, 96, 96, 2), (45, 60, 90, 4), (48, 96, 96, 2),
+                                             (96, 96, 96, 2), (128, 48, 96, 2), (192, 48, 96, 2)])
+def test_member_alone_and_in_a_full_group(N, mx, my, members):
+    def prm(i):
+        return rpcf.make_params(mx, my, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=900.0 + 100 * i, Ro=0.1, dt=0.002,
+                                u_profile=(1.0, 0.0, -1.0), flow_control=1)
+
+    def initial(i):
+        return rpcf.seed_state(rpcf.load(rpcf.HIP_LIB), prm(i), i, 0.1, 4, 12, 5.0 / 6.0, True)
+
+    ids = list(range(members))
+    with rpcf.Group(rpcf.HIP_LIB, prm(0), members) as g:
+        for i in ids:
+            g.init(i, prm(i))
+            g.set_state(i, *initial(i))
+        g.bootstrap(ids)
+        g.step(ids, 2)
+        got = [g.get_state(i) for i in ids]
+    for i in (0, members - 1):
+        with rpcf.Simulation(rpcf.HIP_LIB, prm(i)) as s:
+            s.set_state(*initial(i))
+            s.bootstrap()
+            s.step(2)
+            for a, b in zip(s.get_state(), got[i]):
+                assert np.array_equal(a, b), i
+
+
+# the padded p2s in chunks of 16 samples (more blocks than compute units) at the lengths the grids
+# above leave out: chunks of 12 and 16 samples, row tiles in one block and in two
+@pytest.mark.parametrize("N,mx,my", [(24, 128, 192), (48, 128, 192), (96, 128, 192), (192, 96, 96)])
+def test_padded_p2s_with_many_blocks(N, mx, my):
+    g, o = pair(rpcf.make_params(mx, my, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=900.0, Ro=0.1, dt=0.002))
+    rng = np.random.default_rng(N)
+    shape = g.s["P"], g.s["nz"]
+    f = [(rng.standard_normal(shape) + 1j * rng.standard_normal(shape)) / (1.0 + np.arange(g.s["nz"])) ** 2
+         for _ in range(6)]
+    for s in (g, o):
+        for i in range(6):
+            s.set_field(i, f[i])
+        s.nonlinear()
+    for a, b in zip(g.get_nonlinear(), o.get_nonlinear()):
+        assert rel(a, b) < 1e-12
+    g.close(), o.close()
