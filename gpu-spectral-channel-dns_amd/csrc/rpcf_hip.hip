@@ -1413,17 +1413,6 @@ int init_ctx(rpcf_ctx* c) {
     return RPCF_OK;
 }
 
-// Physics of one slot: base profile, per-slot operator tables and the inverses of its
-// Crank-Nicolson collocation matrices (initAuxMatrix, source/solver.cpp:260-320); the slot's
-// state, fields and history are cleared.
-// Whether solves that give the full inverses' results are faster from the parity blocks: these
-// read 9/16 of the bytes, but combine the row pairs first (a barrier and 1.5 us).  k_lin_solve,
-// full inverses against blocks (us): 32x33x32 8.2 / 9.7, 64x49x64 22 / 24.4,
-// 128x33x128 57.7 / 61.8 (0.15 GB of full inverses); 128x41x128 76.3 / 74.5 (0.23 GB, more than
-// the last-level cache keeps), 128x49x128 97 / 83, 32x65x32 12.5 / 12.9, 48x65x48 17.9 / 16.1,
-// 16x101x16 13.2 / 12.9, 128x65x128 154 / 112.
-bool blocks_pay(const Dims& d) { return d.N >= 64 || 32.0 * d.nslot * d.nz * d.nz > 0.2e9; }
-
 // parity blocks of a slot's inverses (k_parity_blocks), on the context stream
 int build_parity_blocks(rpcf_ctx* c, int slot) {
     const Dims d = c->d;
@@ -1435,6 +1424,9 @@ int build_parity_blocks(rpcf_ctx* c, int slot) {
     return e == hipSuccess ? RPCF_OK : fail(c, RPCF_EDEVICE, "k_parity_blocks: %s", hipGetErrorString(e));
 }
 
+// Physics of one slot: base profile, per-slot operator tables and the inverses of its
+// Crank-Nicolson collocation matrices (initAuxMatrix, source/solver.cpp:260-320); the slot's
+// state, fields and history are cleared.
 int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     const Dims d = c->d;
     const size_t nz = d.nz;
@@ -1456,13 +1448,15 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     sh.mp.q_re = sh.mp.q_im = 0.0;
     sh.mp.flow_control = prm->flow_control;
     // an even base profile U(y) (no linear part) keeps the collocation systems symmetric under
-    // y -> -y, so the solves can use the parity blocks of the inverses: in the FP64 form where they
-    // pay, with the remainders that give the full inverses' values; in the others alone.
-    // RPCF_FULL_INVERSE=1 keeps the full inverses.
+    // y -> -y, so the solves use the parity blocks of the inverses: with their remainders in
+    // the FP64 form (the full inverses' values), alone in the others.  RPCF_FULL_INVERSE=1
+    // keeps the full inverses: slower from 41 points on, the more members a launch has the more
+    // (64x49x64: 103 us a step alone and 984 for 16 members, 101 and 927 with the blocks), within 1 %
+    // of a step below, and with more rounding in eta (2-norm of the state's error against 64 bits
+    // after ten to fifty steps, N = 32 .. 60: 1.7e-14 .. 1.1e-13, with the blocks 1.4e-14 .. 1.0e-13).
     const char* fe = getenv("RPCF_FULL_INVERSE");
     const bool full = fe && atoi(fe) != 0;
-    sh.mp.parity = 0;
-    if (!full && prm->u_profile[1] == 0.0) sh.mp.parity = c->shape.precision != 0 ? 1 : blocks_pay(d) ? 2 : 0;
+    sh.mp.parity = full || prm->u_profile[1] != 0.0 ? 0 : c->shape.precision == 0 ? 2 : 1;
 
     std::vector<double> U(nz), dU(nz), ddU(nz), mU(d.pz);
     rpcf_host::base_profile(d.nz, prm->u_profile, U.data(), dU.data(), ddU.data());

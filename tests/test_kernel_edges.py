@@ -267,3 +267,32 @@ def test_padded_p2s_with_many_blocks(N, mx, my):
     for a, b in zip(g.get_nonlinear(), o.get_nonlinear()):
         assert rel(a, b) < 1e-12
     g.close(), o.close()
+
+
+# even profiles solve with the parity blocks and their v remainders at every size up to the longest
+# compiled one: N odd (no centre row) and even, the smallest pair counts, row pairs that fill whole
+# and partial batches of every column group; inverses of a few kB and (N = 40) of more than 0.2 GB.  The full
+# inverses' results after one step, to the library's bar -- and not their bits, which would mean
+# that the full inverses were read.
+@pytest.mark.parametrize("N,mx", [(4, 24), (5, 24), (6, 24), (12, 24), (15, 24), (27, 24), (32, 24), (36, 24), (45, 24),
+                                  (48, 24), (60, 24), (64, 24), (75, 24), (81, 24), (96, 24), (125, 24), (128, 24),
+                                  (160, 24), (192, 24), (40, 192)])
+def test_even_profile_solves(N, mx, monkeypatch):
+    def step(full):
+        monkeypatch.setenv("RPCF_FULL_INVERSE", str(full))
+        prm = rpcf.make_params(mx, mx, 4 * N, n_pi_x=2.0, n_pi_y=1.0, Re=1300.0, Ro=0.1, dt=0.002,
+                               u_profile=(1.0, 0.0, -1.0), flow_control=1)
+        with rpcf.Simulation(rpcf.HIP_LIB, prm) as s:
+            if N < 12:  # no room for a seed that satisfies the wall conditions
+                rng = np.random.default_rng(N)
+                shape = s.s["P"], s.s["nz"]
+                s.set_state(*(rng.standard_normal(shape) + 1j * rng.standard_normal(shape) for _ in range(2)))
+            else:
+                s.set_state(*rpcf.seed_state(s.dll, prm, 0, 0.1, 4, min(24, N - 5), 5.0 / 6.0, True))
+            s.bootstrap()
+            return s.get_state()
+
+    for a, f in zip(step(0), step(1)):
+        print("N=%d: blocks vs full inverses %.2e" % (N, rel(a, f)))
+        assert rel(a, f) < 1e-12
+        assert not np.array_equal(a, f)
