@@ -48,7 +48,7 @@ def device_sync():
 
 def kernel_bytes(s, prm):
     """algorithmic HBM bytes per launch of each kernel: the arrays it must read and write
-    once.  FP64 form: complex FP64 (16 B) throughout; with an even base profile (the channel)
+    once.  FP64 form: complex FP64 (16 B) throughout; with an even base profile (the channel) and N <= 192
     the solves read the two parity blocks of each inverse (nz x (N/2 + 1) complex FP64
     entries) and the remainders of the v blocks (the same count of complex BF16 pairs, 4 B),
     otherwise the full inverses (nz x nz).  Mixed form (precision 1; channel profile, matrix-core
@@ -59,7 +59,8 @@ def kernel_bytes(s, prm):
     more at 128x129x128, not counted.)"""
     P, nz, hnx, ny, pz = s["P"], s["nz"], s["hnx"], s["ny"], s["pz"]
     my, nxh = prm.my, s["nx"] // 2
-    parity = prm.u_profile[1] == 0.0 and os.environ.get("RPCF_FULL_INVERSE", "0") == "0"
+    parity = (prm.u_profile[1] == 0.0 and (prm.precision != 0 or nz <= 193)
+              and os.environ.get("RPCF_FULL_INVERSE", "0") == "0")
     mixed = prm.precision == 1 and 2 * (nz - 1) <= 384 and os.environ.get("RPCF_MIXED_MFMA", "1") != "0"
     h = 0.5 if prm.precision == 1 else 1.0  # FP32 intermediates of the mixed form
     S = P * nz * 16                    # one spectral field

@@ -1454,9 +1454,12 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     // (64x49x64: 103 us a step alone and 984 for 16 members, 101 and 927 with the blocks), within 1 %
     // of a step below, and with more rounding in eta (2-norm of the state's error against 64 bits
     // after ten to fifty steps, N = 32 .. 60: 1.7e-14 .. 1.1e-13, with the blocks 1.4e-14 .. 1.0e-13).
+    // Past N = 192 the FP64 form keeps them too: the BF16 rounding of the remainders grows with the
+    // condition of the v system, and a step then ends up to 1.5e-13 of v from the oracle's at N = 160
+    // and 192, 8e-13 at 216, 1e-12 at 225 and 2.2e-12 at 250 -- 3e-14 with the full inverses.
     const char* fe = getenv("RPCF_FULL_INVERSE");
     const bool full = fe && atoi(fe) != 0;
-    sh.mp.parity = full || prm->u_profile[1] != 0.0 ? 0 : c->shape.precision == 0 ? 2 : 1;
+    sh.mp.parity = full || prm->u_profile[1] != 0.0 ? 0 : c->shape.precision != 0 ? 1 : d.N <= 192 ? 2 : 0;
 
     std::vector<double> U(nz), dU(nz), ddU(nz), mU(d.pz);
     rpcf_host::base_profile(d.nz, prm->u_profile, U.data(), dU.data(), ddU.data());

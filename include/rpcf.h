@@ -47,8 +47,8 @@ typedef struct rpcf_ctx rpcf_ctx;
  *   flow_control  0: none (reference); 1: constant flow rate -- a uniform mean
  *                 pressure-gradient correction keeps the bulk of u0 at its value at set_state.
  *   precision     0: FP64 everywhere (reference REAL_DOUBLE, include/data.h:11); the HIP
- *                 library solves an even base profile (u_profile[1] == 0) with the
- *                 reflection-parity blocks of the inverses (half their bytes) plus the v
+ *                 library solves an even base profile (u_profile[1] == 0) up to mz = 768 with
+ *                 the reflection-parity blocks of the inverses (half their bytes) plus the v
  *                 blocks' remainders in BF16 (a sixteenth), which restore the full
  *                 inverses' results: the state agrees with the full-inverse solve to ~1e-13
  *                 after one step (environment RPCF_FULL_INVERSE=1 keeps the full inverses).
