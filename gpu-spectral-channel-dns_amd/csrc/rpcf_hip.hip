@@ -18,13 +18,13 @@
 #include <map>
 #include <mutex>
 #include <string>
-#include <thread>
 #include <vector>
 
 #include "../../include/rpcf.h"
 #include "../../include/rpcf_group.h"
 #include "../../include/rpcf_static.h"
 #include "host_prep.hpp"
+#include "host_stage.hpp"
 #include "instances.hpp"
 #include "k_linear.hpp"
 
@@ -355,122 +355,27 @@ int pick_tile(int tmax, int seq_len, int cap, int limit, L lds_bytes) {
 
 size_t spec_elems(const rpcf_ctx* c) { return (size_t)c->d.P * c->d.nz; }
 
-// ---- host arrays across the boundary ---------------------------------------------------
-// `rows` rows of row_bytes each, contiguous on the device, `pitch` bytes apart on the host.
-// An array of at least kStageMin bytes goes through pinned buffers, kStageThreads threads each
-// taking pieces of whole rows in turn: while one piece is on the link the others are copied
-// between the caller's pageable memory and their buffers (which also faults fresh pages in
-// parallel).  Smaller ones, and calls that find the buffers taken by another context's, go
-// straight from or to the caller's memory.  Both ways replace a zeroed std::vector filled by
-// the runtime's pageable copy and then copied once more number by number.  Two 17.2 MB arrays
-// (rpcf_get_state at 128x129x128): 6.5-8.5 ms -> 1.7 ms; a padded
-// field to physical planes (75.8 MB, rpcf_spec_to_phys, which also made four device
-// allocations per call): 10.0 -> 3.1 ms.
-constexpr size_t kStageMin = 8u << 20, kStagePiece = 2u << 20;
-constexpr int kStageThreads = 6;
-std::mutex g_stage_mu;    // held while the buffers are in use
-char* g_stage = nullptr;  // kStageThreads pieces, pinned; freed with the last context
-std::mutex g_ctx_mu;
-int g_ctx_count = 0;
-
-void stage_ref(int by) {
-    std::lock_guard<std::mutex> lk(g_ctx_mu);
-    g_ctx_count += by;
-    if (g_ctx_count) return;
-    std::lock_guard<std::mutex> ls(g_stage_mu);
-    if (g_stage) (void)hipHostFree(g_stage);
-    g_stage = nullptr;
-}
-
-void copy_rows(char* dst, size_t dst_pitch, const char* src, size_t src_pitch, size_t rows, size_t row_bytes) {
-    if (dst_pitch == row_bytes && src_pitch == row_bytes) memcpy(dst, src, rows * row_bytes);
-    else
-        for (size_t r = 0; r < rows; r++) memcpy(dst + r * dst_pitch, src + r * src_pitch, row_bytes);
-}
-
-// the pieces t, t + kStageThreads, .. through buffer t
-hipError_t stage_pieces(rpcf_ctx* c, int t, char* dev, char* host, size_t rows, size_t row_bytes, size_t pitch, bool out) {
-    hipError_t e = hipSetDevice(c->device);
-    hipEvent_t ev = nullptr;
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess) return e;
-    char* buf = g_stage + t * kStagePiece;
-    const size_t per = kStagePiece / row_bytes;
-    bool pending = false;
-    for (size_t r = t * per; r < rows && e == hipSuccess; r += kStageThreads * per) {
-        const size_t n = std::min(per, rows - r);
-        if (!out) {
-            if (pending) e = hipEventSynchronize(ev);  // the buffer's last piece has left
-            if (e == hipSuccess) copy_rows(buf, row_bytes, host + r * pitch, pitch, n, row_bytes);
-        }
-        if (e == hipSuccess)
-            e = hipMemcpyAsync(out ? buf : dev + r * row_bytes, out ? dev + r * row_bytes : buf, n * row_bytes,
-                               out ? hipMemcpyDeviceToHost : hipMemcpyHostToDevice, c->stream);
-        if (e == hipSuccess) e = hipEventRecord(ev, c->stream);
-        pending = e == hipSuccess;
-        if (out && pending) {
-            e = hipEventSynchronize(ev);
-            if (e == hipSuccess) copy_rows(host + r * pitch, pitch, buf, row_bytes, n, row_bytes);
-        }
-    }
-    if (!out && pending) {
-        const hipError_t w = hipEventSynchronize(ev);
-        if (e == hipSuccess) e = w;
-    }
-    (void)hipEventDestroy(ev);
-    return e;
-}
-
-// *done = false: the caller takes the direct way
-hipError_t staged_copy(rpcf_ctx* c, char* dev, char* host, size_t rows, size_t row_bytes, size_t pitch, bool out,
-                       bool* done) {
-    *done = false;
-    if (rows * row_bytes < kStageMin || row_bytes > kStagePiece) return hipSuccess;
-    std::unique_lock<std::mutex> lk(g_stage_mu, std::try_to_lock);
-    if (!lk.owns_lock()) return hipSuccess;
-    if (!g_stage && hipHostMalloc((void**)&g_stage, kStageThreads * kStagePiece, hipHostMallocPortable) != hipSuccess) {
-        g_stage = nullptr;
-        (void)hipGetLastError();
-        return hipSuccess;
-    }
-    hipError_t err[kStageThreads];
-    std::thread th[kStageThreads];
-    for (int t = 1; t < kStageThreads; t++) {
-        err[t] = hipSuccess;
-        try {
-            th[t] = std::thread([&, t] { err[t] = stage_pieces(c, t, dev, host, rows, row_bytes, pitch, out); });
-        } catch (const std::exception&) {  // no thread: its pieces are taken below
-        }
-    }
-    err[0] = stage_pieces(c, 0, dev, host, rows, row_bytes, pitch, out);
-    for (int t = 1; t < kStageThreads; t++) {
-        if (th[t].joinable()) th[t].join();
-        else err[t] = stage_pieces(c, t, dev, host, rows, row_bytes, pitch, out);
-    }
-    *done = true;
-    for (hipError_t e : err)
-        if (e != hipSuccess) return e;
-    return hipSuccess;
-}
-
+// ---- host arrays across the boundary (host_stage.hpp) -----------------------------------
 int to_device(rpcf_ctx* c, void* dev, const void* host, size_t rows, size_t row_bytes, size_t pitch) {
     bool done;
-    HIPCHK(c, staged_copy(c, (char*)dev, (char*)const_cast<void*>(host), rows, row_bytes, pitch, false, &done));
+    HIPCHK(c, rpcf_host::staged_copy(c->device, c->stream, (char*)dev, (char*)const_cast<void*>(host), rows, row_bytes, pitch,
+                                     false, &done));
     if (done) return RPCF_OK;
     if (pitch == row_bytes) return copy_sync(c, dev, host, rows * row_bytes, hipMemcpyHostToDevice);
     std::vector<char> h(rows * row_bytes);
-    copy_rows(h.data(), row_bytes, (const char*)host, pitch, rows, row_bytes);
+    rpcf_host::copy_rows(h.data(), row_bytes, (const char*)host, pitch, rows, row_bytes);
     return copy_sync(c, dev, h.data(), h.size(), hipMemcpyHostToDevice);
 }
 
 int to_host(rpcf_ctx* c, void* host, const void* dev, size_t rows, size_t row_bytes, size_t pitch) {
     bool done;
-    HIPCHK(c, staged_copy(c, (char*)const_cast<void*>(dev), (char*)host, rows, row_bytes, pitch, true, &done));
+    HIPCHK(c, rpcf_host::staged_copy(c->device, c->stream, (char*)const_cast<void*>(dev), (char*)host, rows, row_bytes, pitch,
+                                     true, &done));
     if (done) return RPCF_OK;
     if (pitch == row_bytes) return copy_sync(c, host, dev, rows * row_bytes, hipMemcpyDeviceToHost);
     std::vector<char> h(rows * row_bytes);
     RCCHK(copy_sync(c, h.data(), dev, h.size(), hipMemcpyDeviceToHost));
-    copy_rows((char*)host, pitch, h.data(), row_bytes, rows, row_bytes);
+    rpcf_host::copy_rows((char*)host, pitch, h.data(), row_bytes, rows, row_bytes);
     return RPCF_OK;
 }
 
@@ -1089,7 +994,7 @@ void free_ctx(rpcf_ctx* c) {
     if (c->side) (void)hipStreamDestroy(c->side);
     if (c->stream) (void)hipStreamDestroy(c->stream);
     delete c;
-    stage_ref(-1);
+    rpcf_host::stage_ref(-1);
 }
 
 // Raise a kernel's dynamic-LDS cap to `bytes`; a refusal leaves the default cap, and the
@@ -1657,7 +1562,7 @@ int create_ctx(const rpcf_params* shape, int capacity, rpcf_ctx** out) {
         if (!(ok_x && ok_y && ok_z)) return RPCF_EINVAL;
     }
     rpcf_ctx* c = new rpcf_ctx();
-    stage_ref(1);
+    rpcf_host::stage_ref(1);
     c->shape = *shape;
     c->d = d;
     c->capacity = capacity;
