@@ -582,10 +582,13 @@ __device__ __forceinline__ void fft_any(C* buf, int ld, int B, const FftPlan& pl
     else fft_run<DIR>(buf, ld, B, pl, tid, nthr);
 }
 
-// lengths with compiled plans (every grid of the benchmark, ensemble and serving sets)
-#define RPCF_FFT_LENGTHS(X) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384) X(512)
+// lengths with compiled plans (every grid of the benchmark, ensemble and serving sets), and the one
+// that only the span has (the others are refused there: 2N above 510, rows of 512 beyond LDS)
+#define RPCF_FFT_LENGTHS(X) X(24) X(32) X(48) X(64) X(96) X(128) X(192) X(256) X(384)
+#define RPCF_SPAN_ONLY_LENGTH 512
+#define RPCF_SPAN_LENGTHS(X) RPCF_FFT_LENGTHS(X) X(512)
 // the further lengths whose x and span transforms are compiled, in FP64 (two passes): with the
-// ones above (but 512) every even 2^a 3^b 5^c of 24 .. 384
+// ones above every even 2^a 3^b 5^c of 24 .. 384
 #define RPCF_XY_LENGTHS(X) \
     X(30) X(36) X(40) X(50) X(54) X(60) X(72) X(80) X(90) X(100) X(108) X(120) X(144) X(150) X(160) X(162) X(180) \
     X(200) X(216) X(240) X(250) X(270) X(288) X(300) X(320) X(324) X(360)

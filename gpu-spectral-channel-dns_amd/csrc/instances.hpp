@@ -6,12 +6,15 @@
 #include "k_cheb_mfma.hpp"
 #include "k_transform.hpp"
 
-// x and span transforms, precision R (all that an RPCF_XY_LENGTHS length has, in FP64)
-#define RPCF_INSTANCES_XY(EXT, L, R)                                                                                  \
+// span transforms, precision R (all that RPCF_SPAN_ONLY_LENGTH has)
+#define RPCF_INSTANCES_SPAN(EXT, L, R)                                                                                \
     EXT template __global__ void k_span_inv<L, R>(const cplx<R>*, long, long, cplx<R>*, long, long, Dims, int, FftPlan, \
                                                   int, int, const int*);                                               \
     EXT template __global__ void k_span_fwd<L, R>(const cplx<R>*, long, long, int, cplx<R>*, long, long, Dims, int,     \
-                                                  FftPlan, int, int, const int*, int*);                                \
+                                                  FftPlan, int, int, const int*, int*);
+// x and span transforms (all that an RPCF_XY_LENGTHS length has, in FP64)
+#define RPCF_INSTANCES_XY(EXT, L, R)                                                                                  \
+    RPCF_INSTANCES_SPAN(EXT, L, R)                                                                                     \
     EXT template __global__ void k_lamb_phys<L, R>(const cplx<R>*, long, long, cplx<R>*, long, long, int, const double*, \
                                                    long, double, Dims, FftPlan, int, int, Members);
 // Chebyshev transforms of length 2N = L with the padded side in precision R
@@ -36,11 +39,11 @@
                                                              long, Dims, Members, int, int);                           \
     EXT template __global__ void k_velocity_tile<L, float2>(const double2*, const double2*, long, float2*, long, long, \
                                                             Dims, Members, int, int);                                  \
-    EXT template __global__ void k_s2p_mfma<(L <= 384 ? L : 384)>(const float2*, long, long, float2*, long, long, Dims, \
+    EXT template __global__ void k_s2p_mfma<L>(const float2*, long, long, float2*, long, long, Dims, \
                                                                   const h8_t*, const int*, int);                       \
-    EXT template __global__ void k_p2s_mfma<(L <= 384 ? L : 384)>(const float2*, long, long, double2*, long, Dims,     \
+    EXT template __global__ void k_p2s_mfma<L>(const float2*, long, long, double2*, long, Dims,     \
                                                                   const h8_t*, int, int, Members);                     \
-    EXT template __global__ void k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunk>(const double2*, long, long, double2*, long, Dims, \
+    EXT template __global__ void k_p2s_dmfma<L, cheb_dmfma::kChunk>(const double2*, long, long, double2*, long, Dims, \
                                                                           const double*, Members, int, int); \
-    EXT template __global__ void k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunkMany>(const double2*, long, long, double2*, long, Dims, \
+    EXT template __global__ void k_p2s_dmfma<L, cheb_dmfma::kChunkMany>(const double2*, long, long, double2*, long, Dims, \
                                                                           const double*, Members, int, int);

@@ -418,11 +418,10 @@ typedef double rpcf_v4d __attribute__((ext_vector_type(4)));
 constexpr int kTvChunk = 3;
 constexpr int kTvBlockPencils = 32;
 
-// three waves per SIMD (168 registers, no accumulation registers) up to S = 17: the
-// B-fragment loads of more waves in flight; two waves (136 + 48) took 76 us against 68 at
-// 128x129x128.  Longer Chebyshev lengths (S = 25, 33) hold 4 S B-fragment registers and
-// would spill at three waves, so they run two.
-constexpr int tv_waves(int s) { return s <= 17 ? 3 : 2; }
+// k-steps per parity up to which an operator's whole table (2 RT S tiles of 512 bytes, 87 KB at
+// 2N = 256) stays in LDS: k_lin_tv_stream.  Past it this kernel, two waves per SIMD: its 4 S
+// B-fragment registers would spill at three.
+constexpr bool tv_streams(int s) { return s <= 17; }
 // Instantiated k-step counts: those of the compiled Chebyshev lengths; another length takes the
 // next one up (its table is zero-padded): 7.7 us at 40x46x60 (S = 7 for the 6 it needs)
 // and 104 at 100x151x100 (25 for 19) against 33 and 489 for a kernel on the vector units.
@@ -434,7 +433,7 @@ inline int tv_steps(int need) {
     return 0;
 }
 template <int S>  // k-steps per parity: S >= ceil((N/2 + 1)/4)
-__global__ __launch_bounds__(256, tv_waves(S)) void k_lin_tv_mfma(const double2* __restrict__ sv, const double2* __restrict__ se,
+__global__ __launch_bounds__(256, 2) void k_lin_tv_mfma(const double2* __restrict__ sv, const double2* __restrict__ se,
                                                      long sS, double2* __restrict__ W, long sWl, Dims d,
                                                      const double* __restrict__ Tf, long sTf, int RT,
                                                      const int* __restrict__ ids) {

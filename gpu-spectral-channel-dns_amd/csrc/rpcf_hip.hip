@@ -31,6 +31,8 @@
 #define RPCF_CASE(L) RPCF_INSTANCES(extern, L)
 RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
+RPCF_INSTANCES_SPAN(extern, RPCF_SPAN_ONLY_LENGTH, double)
+RPCF_INSTANCES_SPAN(extern, RPCF_SPAN_ONLY_LENGTH, float)
 #define RPCF_CASE(L) RPCF_INSTANCES_XY(extern, L, double)
 RPCF_XY_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
@@ -235,7 +237,7 @@ SlotSizes slot_sizes(const Dims& d, int precision) {
 bool compiled_len(int n) {
     bool ok = false;
 #define RPCF_CASE(L) ok |= n == L;
-    RPCF_FFT_LENGTHS(RPCF_CASE)
+    RPCF_SPAN_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     return ok;
 }
@@ -522,7 +524,7 @@ void span_inv(rpcf_ctx* c, int nf, const cplx<R>* Y, long yS, long sY, cplx<R>* 
     const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + c->twl_y);
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_inv<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Y, yS, sY, W, wS, sW, d, planes, pl, TK, ld, ids); break;
-        RPCF_FFT_LENGTHS(RPCF_CASE)
+        RPCF_SPAN_LENGTHS(RPCF_CASE)
         default:
             if constexpr (sizeof(R) == 8)
                 switch (d.my) {
@@ -548,7 +550,7 @@ void span_fwd(rpcf_ctx* c, int nf, const cplx<R>* Z2, long zS, long sZ, int zld,
     const size_t lds = sizeof(cplx<R>) * (two ? TK * tp_ld(d.my) : TK * ld + c->twl_y);
     switch (d.my) {
 #define RPCF_CASE(L) case L: k_span_fwd<L, R><<<g, span_threads<R>(L), lds, c->stream>>>(Z2, zS, sZ, zld, Y, yS, sY, d, planes, pl, TK, ld, ids, phase); break;
-        RPCF_FFT_LENGTHS(RPCF_CASE)
+        RPCF_SPAN_LENGTHS(RPCF_CASE)
         default:
             if constexpr (sizeof(R) == 8)
                 switch (d.my) {
@@ -604,10 +606,8 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                         switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                               \
     case L:                                                                                                        \
-        if constexpr (L <= 384)                                                                                    \
-            k_s2p_mfma<(L <= 384 ? L : 384)><<<grid, S2pMfma<(L <= 384 ? L : 384)>::threads,                     \
-                                               S2pMfma<(L <= 384 ? L : 384)>::lds, c->stream>>>(                  \
-                (const float2*)c->F, fS, c->sF, Y, yS, c->sY, d, (const h8_t*)c->MT, ids, n);                     \
+        k_s2p_mfma<L><<<grid, S2pMfma<L>::threads, S2pMfma<L>::lds, c->stream>>>(                                  \
+            (const float2*)c->F, fS, c->sF, Y, yS, c->sY, d, (const h8_t*)c->MT, ids, n);                          \
         break;
                             RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
@@ -682,10 +682,8 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                     switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                                 \
     case L:                                                                                                          \
-        if constexpr (L <= 384)                                                                                      \
-            k_p2s_mfma<(L <= 384 ? L : 384)><<<g, 128 * cheb_mfma::Shape<(L <= 384 ? L : 384)>::RTS,               \
-                                             p2s_mfma_lds<(L <= 384 ? L : 384)>(), c->stream>>>(                    \
-                Y, yS, c->sY, c->NL, c->sNL, d, (const h8_t*)(c->MT + c->mt_p2s), c->mt_s0, c->mt_s1, mb);          \
+        k_p2s_mfma<L><<<g, 128 * cheb_mfma::Shape<L>::RTS, p2s_mfma_lds<L>(), c->stream>>>(                          \
+            Y, yS, c->sY, c->NL, c->sNL, d, (const h8_t*)(c->MT + c->mt_p2s), c->mt_s0, c->mt_s1, mb);               \
         break;
                         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
@@ -703,19 +701,17 @@ int enq_transforms(rpcf_ctx* c, const int* ids, int n, bool cap) {
                 [&] {
                     switch (2 * d.N) {
 #define RPCF_CASE(L)                                                                                              \
-    case L:                                                                                                       \
-        if constexpr (L <= 384) {                                                                                 \
-            constexpr int LC = L <= 384 ? L : 384;                                                                \
-            auto run = [&](auto kernel, auto shape) {                                                             \
-                using Sh = decltype(shape);                                                                       \
-                kernel<<<Sh::blocks(nitems), Sh::NT, Sh::lds_bytes(), c->stream>>>(Y, yS, c->sY, c->NL, c->sNL, d, \
-                                                                                   c->DT, mb, nitems, nyb);       \
-            };                                                                                                    \
-            using namespace cheb_dmfma;                                                                           \
-            if (DShape<LC>::blocks(nitems) > c->ncu) run(k_p2s_dmfma<LC, kChunkMany>, DShape<LC, kChunkMany>{});  \
-            else run(k_p2s_dmfma<LC, kChunk>, DShape<LC>{});                                                      \
-        }                                                                                                         \
-        break;
+    case L: {                                                                                                     \
+        auto run = [&](auto kernel, auto shape) {                                                                 \
+            using Sh = decltype(shape);                                                                           \
+            kernel<<<Sh::blocks(nitems), Sh::NT, Sh::lds_bytes(), c->stream>>>(Y, yS, c->sY, c->NL, c->sNL, d,     \
+                                                                               c->DT, mb, nitems, nyb);           \
+        };                                                                                                        \
+        using namespace cheb_dmfma;                                                                               \
+        if (DShape<L>::blocks(nitems) > c->ncu) run(k_p2s_dmfma<L, kChunkMany>, DShape<L, kChunkMany>{});         \
+        else run(k_p2s_dmfma<L, kChunk>, DShape<L>{});                                                            \
+        break;                                                                                                    \
+    }
                         RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
                     }
@@ -791,21 +787,20 @@ int enq_nonlinear(rpcf_ctx* c, const int* ids, int n, bool with_velocity, bool c
 int enq_lin_tv(rpcf_ctx* c, const int* ids, int n, bool cap, hipStream_t s) {
     const Dims d = c->d;
     auto body = [&] {
-            const size_t lds = sizeof(double) * 2 * kTvChunk * c->tv_s * 64;
-            dim3 g((d.P + kTvBlockPencils - 1) / kTvBlockPencils, 5 * n);
-            // persistent blocks with an operator's whole table in LDS when it fits (2N <= 256):
-            // about one block per compute unit (two when the table is small)
+            // persistent blocks with an operator's whole table in LDS: about one block per compute unit
+            // (two when the table is small); longer lengths in chunks of row tiles
             const size_t lds_stream = sizeof(double) * 2 * c->tv_rt * c->tv_s * 64;
-            const bool tv_stream = c->tv_s <= 17 && lds_stream <= (size_t)c->lds_limit;
             const int per_cu = lds_stream * 2 <= (size_t)c->lds_limit ? 2 : 1;
             int gs = std::max(1, std::min((d.P + 31) / 32, per_cu * c->ncu / (5 * n)));
             // a multiple of 8: the five operator blocks of one pencil range (linear ids x + gs y)
             // land on the same XCD (id mod 8), so v-hat and eta-hat come from its L2 after the first read
             if (gs >= 16) gs &= ~7;
+            const size_t lds = sizeof(double) * 2 * kTvChunk * c->tv_s * 64;
+            const dim3 g((d.P + kTvBlockPencils - 1) / kTvBlockPencils, 5 * n);
             switch (c->tv_s) {
 #define RPCF_CASE(S)                                                                                             \
     case S:                                                                                                      \
-        if (tv_stream)                                                                                           \
+        if constexpr (tv_streams(S))                                                                             \
             k_lin_tv_stream<S, 8><<<dim3(gs, 5 * n), 512, lds_stream, s>>>(c->SV, c->SE, c->sS, c->WL, c->sWl,    \
                                                                           d, c->TF, c->sTf, c->tv_rt, ids);      \
         else                                                                                                     \
@@ -1163,7 +1158,7 @@ int init_ctx(rpcf_ctx* c) {
     if ((rc = make_plan(c, 2 * d.N, tw, &c->pl_zn, &c->cap_zn))) return rc;
     // mixed form: fragments of the split-FP16 Chebyshev products (k_cheb_mfma.hpp) for the
     // compiled lengths up to 2N = 384; RPCF_MIXED_MFMA=0 keeps the FFT-based kernels
-    if (c->mixed && 2 * d.N <= 384) {
+    if (c->mixed) {
         const char* e = getenv("RPCF_MIXED_MFMA");
         if (!(e && e[0] == '0')) {
             const MfmaTables& t = mfma_tables(d.N);
@@ -1176,8 +1171,8 @@ int init_ctx(rpcf_ctx* c) {
         }
     }
     // FP64 form: the padded s2p and the padded p2s + nonlinear combination as FP64 matrix-core
-    // products, but for 2N = 512; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
-    if (!c->mixed && (2 * d.N <= 384 || !compiled_len(2 * d.N))) {
+    // products; RPCF_P2S_MFMA=0 keeps the FFT-based kernels
+    if (!c->mixed) {
         const char* e = getenv("RPCF_P2S_MFMA");
         if (!(e && e[0] == '0')) {
             const std::vector<double>& t = dmfma_tables(d.N);
@@ -1240,7 +1235,7 @@ int init_ctx(rpcf_ctx* c) {
 #define RPCF_CASE(L)                          \
     if (d.my == L) tk_max = span_tile_max(L); \
     if (d.mx == L) rp_max = lamb_pairs_max(L);
-    RPCF_FFT_LENGTHS(RPCF_CASE)
+    RPCF_SPAN_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
     c->TK_inv = pick_tile(tk_max, d.my, c->cap_y, lim3, [&](int t) {
         return sizeof(double2) * ((size_t)t * c->ld_my + c->twl_y);
@@ -1285,12 +1280,16 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_velocity_tile<L>, lim);                   \
     allow_lds(k_x_c2r<L>, lim);                           \
     allow_lds(k_velocity_tile<L, float2>, lim);           \
-    allow_lds(k_p2s_mfma<(L <= 384 ? L : 384)>, lim);    \
-    allow_lds(k_s2p_mfma<(L <= 384 ? L : 384)>, lim);    \
-    allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunk>, lim);   \
-    allow_lds(k_p2s_dmfma<(L <= 384 ? L : 384), cheb_dmfma::kChunkMany>, lim);
+    allow_lds(k_p2s_mfma<L>, lim);                        \
+    allow_lds(k_s2p_mfma<L>, lim);                        \
+    allow_lds(k_p2s_dmfma<L, cheb_dmfma::kChunk>, lim);   \
+    allow_lds(k_p2s_dmfma<L, cheb_dmfma::kChunkMany>, lim);
     RPCF_FFT_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
+    allow_lds(k_span_inv<RPCF_SPAN_ONLY_LENGTH>, lim);
+    allow_lds(k_span_fwd<RPCF_SPAN_ONLY_LENGTH>, lim);
+    allow_lds(k_span_inv<RPCF_SPAN_ONLY_LENGTH, float>, lim);
+    allow_lds(k_span_fwd<RPCF_SPAN_ONLY_LENGTH, float>, lim);
 #define RPCF_CASE(L)               \
     allow_lds(k_span_inv<L>, lim); \
     allow_lds(k_span_fwd<L>, lim); \
@@ -1300,9 +1299,9 @@ int init_ctx(rpcf_ctx* c) {
     allow_lds(k_cheb_p2s<0>, lim);
     allow_lds(k_x_c2r<0>, lim);
     allow_lds(k_x_r2c<0>, lim);
-#define RPCF_CASE(S)                 \
-    allow_lds(k_lin_tv_mfma<S>, lim); \
-    allow_lds(k_lin_tv_stream<S, 8>, lim);
+#define RPCF_CASE(S)                                                    \
+    if constexpr (tv_streams(S)) allow_lds(k_lin_tv_stream<S, 8>, lim); \
+    else allow_lds(k_lin_tv_mfma<S>, lim);
     RPCF_TV_STEPS(RPCF_CASE)
 #undef RPCF_CASE
     allow_lds(k_s2p_dmfma<1>, lim);
@@ -1557,7 +1556,7 @@ int create_ctx(const rpcf_params* shape, int capacity, rpcf_ctx** out) {
         // the mixed form runs compiled FFT lengths only
         bool ok_x = false, ok_y = false, ok_z = false;
 #define RPCF_CASE(L) ok_x |= d.mx == L; ok_y |= d.my == L; ok_z |= 2 * d.N == L;
-        RPCF_FFT_LENGTHS(RPCF_CASE)
+        RPCF_SPAN_LENGTHS(RPCF_CASE)
 #undef RPCF_CASE
         if (!(ok_x && ok_y && ok_z)) return RPCF_EINVAL;
     }
