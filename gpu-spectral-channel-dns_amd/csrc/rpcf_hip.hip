@@ -212,6 +212,7 @@ struct SlotSizes {
 // of the v blocks, which restore the full inverses' results (the blocks alone agree with them
 // to ~1e-11 after a step, enough for the mixed form only; the eta blocks need none); in the
 // mixed form the eta blocks also as FP32 high and BF16 low parts, which its solves read.
+constexpr int kRemainderMax = 192;  // largest N of the FP64 form's blocks with remainders (init_slot)
 SlotSizes slot_sizes(const Dims& d, int precision) {
     SlotSizes s;
     const long P = d.P, nz = d.nz, zld = (d.hnx + 7) & ~7;
@@ -224,8 +225,9 @@ SlotSizes slot_sizes(const Dims& d, int precision) {
     s.Z = 3L * d.pz * d.my * zld;
     s.Wl = 5 * P * nz;
     s.M = 2L * d.nslot * nz * nz;
-    s.MH = (precision == 1 ? 1L : 2L) * d.nslot * nz * (d.N / 2 + 1);  // nz rows x (N/2 + 1) pair columns; mixed: v
-    s.ME = precision <= 1 ? (long)d.nslot * nz * (d.N / 2 + 1) : 0;  // v remainders / eta low parts
+    const long block = precision == 0 && d.N > kRemainderMax ? 0 : d.nslot * nz * (d.N / 2 + 1);
+    s.MH = (precision == 1 ? 1 : 2) * block;  // nz rows x (N/2 + 1) pair columns; mixed: v
+    s.ME = precision <= 1 ? block : 0;        // v remainders / eta low parts
     s.MF = precision == 1 ? s.ME : 0;                                  // eta high parts
     s.Tf = 5 * 2 * RT * S * 64;
     s.U = nz;
@@ -1077,7 +1079,7 @@ int init_ctx(rpcf_ctx* c) {
     if ((rc = dalloc(c, &c->F, C * ss.F)) || (rc = dalloc(c, &c->SV, C * ss.S)) || (rc = dalloc(c, &c->SE, C * ss.S)) ||
         (rc = dalloc(c, &c->NL, C * ss.NL)) || (rc = dalloc(c, &c->Y, C * ss.Y)) || (rc = dalloc(c, &c->W, C * ss.W)) ||
         (rc = dalloc(c, &c->Z2, C * ss.Z)) || (rc = dalloc(c, &c->WL, C * ss.Wl)) ||
-        (rc = dalloc(c, &c->MINV, C * ss.M)) || (rc = dalloc(c, &c->MINVH, C * ss.MH)) ||
+        (rc = dalloc(c, &c->MINV, C * ss.M)) || (ss.MH && (rc = dalloc(c, &c->MINVH, C * ss.MH))) ||
         (ss.ME && (rc = dalloc(c, &c->MINVE, C * ss.ME))) || (ss.MF && (rc = dalloc(c, &c->MINVF, C * ss.MF))) ||
         (rc = dalloc(c, &c->TF, C * ss.Tf)) ||
         (rc = dalloc(c, &c->U, C * ss.U)) || (rc = dalloc(c, &c->DU, C * ss.U)) || (rc = dalloc(c, &c->DDU, C * ss.U)) ||
@@ -1363,7 +1365,7 @@ int init_slot(rpcf_ctx* c, int slot, const rpcf_params* prm) {
     // and 192, 8e-13 at 216, 1e-12 at 225 and 2.2e-12 at 250 -- 3e-14 with the full inverses.
     const char* fe = getenv("RPCF_FULL_INVERSE");
     const bool full = fe && atoi(fe) != 0;
-    sh.mp.parity = full || prm->u_profile[1] != 0.0 ? 0 : c->shape.precision != 0 ? 1 : d.N <= 192 ? 2 : 0;
+    sh.mp.parity = full || prm->u_profile[1] != 0.0 ? 0 : c->shape.precision != 0 ? 1 : d.N <= kRemainderMax ? 2 : 0;
 
     std::vector<double> U(nz), dU(nz), ddU(nz), mU(d.pz);
     rpcf_host::base_profile(d.nz, prm->u_profile, U.data(), dU.data(), ddU.data());
