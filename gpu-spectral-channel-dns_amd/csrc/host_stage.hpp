@@ -5,7 +5,11 @@
 // taking pieces of whole rows in turn: while one piece is on the link the others are copied
 // between the caller's pageable memory and their buffers (which also faults fresh pages in
 // parallel).  Smaller ones, and calls that find the buffers taken by another context's, go
-// straight from or to the caller's memory.  Both ways replace a zeroed std::vector filled by
+// straight from or to the caller's memory.  The line lies where both directions together gain
+// (two fields, us, straight / by pieces): out 115 / 255 at 0.9 MB a field, 330-1050 / 1220 at 2.2,
+// 1800 / 1080-1390 at 5.7, 1900-2200 / 1280-1570 at 7.3, 3130 / 1750 at 12.9, 7030 / 2420 at 34
+// (what varies is the first touch of the caller's pages); in 95 / 230 at 0.9, 330 / 445 at 4.9,
+// 440 / 580 at 7.3, 750 / 865 at 12.9, 1000 / 1090 at 17.2, 2370 / 1960 at 34.  Both ways replace a zeroed std::vector filled by
 // the runtime's pageable copy and then copied once more number by number.  Two 17.2 MB arrays
 // (rpcf_get_state at 128x129x128): 6.5-8.5 ms -> 1.7 ms; a padded
 // field to physical planes (75.8 MB, rpcf_spec_to_phys, which also made four device
